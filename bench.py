@@ -48,10 +48,16 @@ def log(*a):
 
 def kernel_name(info):
     """The kernel a plan launches, spelled as rocprof shows its template
-    (ttc::<family kernel><Op, VA, VB, BETA, NT[, FAST]>)."""
+    (ttc::<family kernel><Op, VA, VB, BETA, NT[, FAST or DIV]>)."""
     ops = {(0, 0): "ttc::OpF32<float, float>", (1, 1): "ttc::OpDD"}
     tf = lambda x: "true" if x else "false"
     op = ops.get((info["type_a"], info["type_b"]), "?")
+    if info["family"] == 2 and info["lane_fixed"]:  # one work-group per tile; DIV 2 where half the slots do
+        va, vb, r, c = info["vec_a"], info["vec_b"], info["rows"], info["cols"]
+        ea, eb = info["slots_a"] * va, info["slots_b"] * vb
+        half = 256 // (r // va) * (ea // va // 2) >= c and 256 // (c // vb) * (eb // vb // 2) >= r
+        return "ttc::transpose_lane_kernel<%s, %d, %d, %s, %s, %d>" % (
+            op, va, vb, tf(not info["beta_is_zero"]), tf(info["nt_store"]), 2 if half else 1)
     if info["family"] == 2:
         return "ttc::transpose_rc_kernel<%s, %d, %d, %s, %s, %s>" % (
             op, info["vec_a"], info["vec_b"], tf(not info["beta_is_zero"]), tf(info["nt_store"]),

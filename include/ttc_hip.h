@@ -73,7 +73,8 @@ typedef struct {
   int tile[TTC_MAX_DIM]; /* tile extent per fused A dimension (all 0 = heuristic) */
   int vec_a;             /* elements per lane vector on the A (read) side; 0 = widest legal */
   int vec_b;             /* elements per lane vector on the B (write) side; 0 = widest legal */
-  int wg_per_cu;         /* resident persistent work-groups per CU; 0 = occupancy limit */
+  int wg_per_cu;         /* resident persistent work-groups per CU; 0 = occupancy limit, or, for row x column
+                            tiles, one work-group per tile */
   int nt_store;          /* non-temporal B stores (beta_is_zero only): 0 = auto (off), 1 = on, 2 = off */
   int grid_order;        /* 0 = auto (4), 1 = strided tile walk, 2 = contiguous tile ranges,
                             3 = strided walk with the work-groups of one XCD on consecutive tiles,
@@ -83,9 +84,12 @@ typedef struct {
   int family;            /* kernel family: 0 = auto, 1 = box tile, 2 = row x column tile,
                             3 = row copy (perm[0] == 0 after fusion only) */
   int tile_order;        /* tile numbering (row x column tiles): 0 = auto (B order), 1 = A order, 2 = B order,
-                            3 / 4 = B order in groups of 8 / 16 tiles along A's leading tiled dimension */
-  int lds_buffers;       /* LDS tile buffers (row x column tiles): 0 = auto (2), 1 = one (two barriers per
-                            tile, more resident work-groups), 2 = two (one barrier per tile) */
+                            3 / 4 = B order in groups of 8 / 16 tiles along A's leading tiled dimension (launches
+                            of one work-group per tile walk order 2 in groups of 8 too) */
+  int lds_buffers;       /* LDS tile buffers of work-groups that walk several row x column tiles: 0 = auto (2), 1 = one
+                            (two barriers per tile, more resident work-groups), 2 = two (one barrier per tile).
+                            A single-op launch has such work-groups where an explicit `tile` comes with 1 or 2 here,
+                            with wg_per_cu, or where a tile does not fit a launch of one work-group per tile */
 } ttc_config_t;
 
 /* What a plan resolved to (fused geometry, tile, launch shape). */
@@ -115,7 +119,7 @@ typedef struct {
   int rows, cols;                /* row x column tile: row and column counts (0 for box tiles) */
   int tile_order;                /* 1 = A order, 2 = B order, 3 / 4 grouped B order */
   int lds_buffers;               /* LDS tile buffers of the row x column kernel (1 for other families) */
-  int lane_fixed;                /* row x column kernel: full tiles take the lane-fixed walk (1) or the general one */
+  int lane_fixed;                /* row x column kernel: tiles take a lane-fixed walk (1) or the general one */
 } ttc_plan_info_t;
 
 /* Library version string. */

@@ -36,7 +36,7 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-I" + INCLUDE, "-I" + CSRC]
 
-HEADERS = ["ttc_kernels.hpp", "ttc_rc.hpp", "ttc_row.hpp", "ttc_launch.hpp", "ttc_batch_kernels.hpp", "ttc_params.h",
+HEADERS = ["ttc_kernels.hpp", "ttc_rc.hpp", "ttc_lane.hpp", "ttc_row.hpp", "ttc_launch.hpp", "ttc_batch_kernels.hpp", "ttc_params.h",
            "ttc_plan.h", "ttc_runtime.h", "gen/inst_all.h"]
 VERSION = "0.2.0"
 

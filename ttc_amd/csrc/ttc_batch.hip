@@ -273,9 +273,9 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
     };
     for (int pass = 0; pass < 2; ++pass) {
       ttc_plan_t pl = nullptr;
-      ttc_status_t st = ttc_plan_create(&pl, op.type_a, op.type_b, op.dim, op.perm, op.size,
-                                        any_lda ? op.lda : nullptr, any_ldb ? op.ldb : nullptr,
-                                        op.beta_is_zero, &cfg);
+      ttc_status_t st = plan_create(&pl, op.type_a, op.type_b, op.dim, op.perm, op.size,
+                                    any_lda ? op.lda : nullptr, any_ldb ? op.ldb : nullptr, op.beta_is_zero, &cfg,
+                                    true);
       if (st != TTC_SUCCESS) return st;
       const bool ok_a = width_ok(pl, pl->va), ok_b = width_ok(pl, pl->vb);
       if ((ok_a && ok_b) || pass == 1) {

@@ -39,8 +39,6 @@ struct f16s { uint16_t u; };
 struct e4m3s { uint8_t u; };
 struct e5m2s { uint8_t u; };
 
-__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) { return (__umulhi(n, f.m) + n) >> f.s; }
-
 // ------------------------------------------------------------ conversions
 __device__ __forceinline__ float to_f32(float a) { return a; }
 __device__ __forceinline__ float to_f32(bf16s a) { return __uint_as_float((uint32_t)a.u << 16); }
@@ -488,8 +486,6 @@ struct TileRange {
 // strided walk: neighbouring tiles share the cache lines at their edges, and
 // those then meet in one L2 instead of being fetched (and partially written
 // back) by two.
-constexpr uint32_t kXcds = 8;
-
 __device__ __forceinline__ TileRange tile_range(uint32_t ntiles, uint32_t wg, uint32_t nwg, int order) {
   TileRange r;
   if (order == 3 && nwg % kXcds == 0) {

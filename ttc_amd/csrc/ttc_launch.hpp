@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include "ttc_kernels.hpp"
+#include "ttc_lane.hpp"
 #include "ttc_rc.hpp"
 #include "ttc_row.hpp"
 
@@ -23,6 +24,11 @@ using LaunchRCFn = hipError_t (*)(const RCParams&, const void*, void*, double, d
 using LaunchFp8RCFn = hipError_t (*)(const RCParams&, const void*, void*, float, const float*, const float*, float,
                                      float, float*, float*, unsigned, size_t, hipStream_t);
 
+using LaunchLaneFn = hipError_t (*)(const RCLaneParams&, const void*, void*, double, double, size_t, hipStream_t);
+
+using LaunchFp8LaneFn = hipError_t (*)(const RCLaneParams&, const void*, void*, float, const float*, const float*,
+                                       float, float, float*, float*, size_t, hipStream_t);
+
 using LaunchRowFn = hipError_t (*)(const RowParams&, const void*, void*, double, double, const float*, const float*,
                                    float, float, float*, float*, unsigned, hipStream_t);
 
@@ -38,6 +44,9 @@ struct KernelEntry {
   LaunchRCFn launch_rc_fast;
   LaunchFp8RCFn launch_fp8_rc_fast;
   const void* func_fast;
+  // row x column family, one tile per work-group: instance of DIV 1, 2
+  LaunchLaneFn launch_lane[2];
+  LaunchFp8LaneFn launch_fp8_lane[2];
 };
 
 template <class OP, int VA, int VB, bool BETA, bool NT>
@@ -86,21 +95,52 @@ hipError_t launch_fp8_rc(const RCParams& p, const void* A, void* B, float alpha,
                          dim3(kRcThreads), args, lds, s);
 }
 
+template <class OP, int VA, int VB, bool BETA, bool NT, int DIV>
+hipError_t launch_lane(const RCLaneParams& p, const void* A, void* B, double alpha, double beta, size_t lds,
+                       hipStream_t s) {
+  const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
+  typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  void* args[] = {const_cast<RCLaneParams*>(&p), &a, &b, &alpha, &beta};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&transpose_lane_kernel<OP, VA, VB, BETA, NT, DIV>),
+                         dim3(p.walk.ntiles), dim3(kRcThreads), args, lds, s);
+}
+
+template <class OP, int VA, int VB, int DIV>
+hipError_t launch_fp8_lane(const RCLaneParams& p, const void* A, void* B, float alpha, const float* scale_in,
+                           const float* amax_in, float fp8_max, float scale_host, float* amax_out,
+                           float* scale_inv_out, size_t lds, hipStream_t s) {
+  const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
+  typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  void* args[] = {const_cast<RCLaneParams*>(&p), &a, &b, &alpha, &scale_in, &amax_in, &fp8_max, &scale_host,
+                  &amax_out, &scale_inv_out};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&cast_fp8_lane_kernel<OP, VA, VB, DIV>),
+                         dim3(p.walk.ntiles), dim3(kRcThreads), args, lds, s);
+}
+
 template <class OP, int VA, int VB, int MODE>
 KernelEntry make_rc_entry(int ta, int tb) {
   KernelEntry e{ta, tb, VA, VB, MODE, kFamRC, nullptr, nullptr, nullptr, nullptr};
   if constexpr (MODE == kModeFp8) {
     e.launch_fp8_rc = &launch_fp8_rc<OP, VA, VB, false>;
     e.func = reinterpret_cast<const void*>(&cast_fp8_rc_kernel<OP, VA, VB, false>);
-    e.launch_fp8_rc_fast = &launch_fp8_rc<OP, VA, VB, true>;
-    e.func_fast = reinterpret_cast<const void*>(&cast_fp8_rc_kernel<OP, VA, VB, true>);
+    if constexpr (sizeof(typename OP::TA) == 2) {
+      e.launch_fp8_rc_fast = &launch_fp8_rc<OP, VA, VB, true>;
+      e.func_fast = reinterpret_cast<const void*>(&cast_fp8_rc_kernel<OP, VA, VB, true>);
+    }
+    e.launch_fp8_lane[0] = &launch_fp8_lane<OP, VA, VB, 1>;
+    e.launch_fp8_lane[1] = &launch_fp8_lane<OP, VA, VB, 2>;
   } else {
     constexpr bool beta = MODE == kModeBeta;
     constexpr bool nt = MODE == kModeBzNt;
     e.launch_rc = &launch_rc<OP, VA, VB, beta, nt, false>;
     e.func = reinterpret_cast<const void*>(&transpose_rc_kernel<OP, VA, VB, beta, nt, false>);
-    e.launch_rc_fast = &launch_rc<OP, VA, VB, beta, nt, true>;
-    e.func_fast = reinterpret_cast<const void*>(&transpose_rc_kernel<OP, VA, VB, beta, nt, true>);
+    // (RCParams::fast: pairs with a 2-byte side only)
+    if constexpr (sizeof(typename OP::TA) == 2 || sizeof(typename OP::TB) == 2) {
+      e.launch_rc_fast = &launch_rc<OP, VA, VB, beta, nt, true>;
+      e.func_fast = reinterpret_cast<const void*>(&transpose_rc_kernel<OP, VA, VB, beta, nt, true>);
+    }
+    e.launch_lane[0] = &launch_lane<OP, VA, VB, beta, nt, 1>;
+    e.launch_lane[1] = &launch_lane<OP, VA, VB, beta, nt, 2>;
   }
   return e;
 }

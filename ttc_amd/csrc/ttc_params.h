@@ -10,6 +10,12 @@
 #pragma once
 #include <stdint.h>
 
+#ifdef __HIPCC__
+#define TTC_HD __host__ __device__
+#else
+#define TTC_HD
+#endif
+
 namespace ttc {
 
 constexpr int kMaxDim = 8;     // fused rank limit
@@ -40,6 +46,15 @@ inline FastDiv make_fastdiv(uint32_t d) {
   f.m = (uint32_t)(((1ull << 32) * ((1ull << s) - d)) / d + 1);
   return f;
 }
+
+TTC_HD inline uint32_t fdiv(uint32_t n, uint32_t m, uint32_t s) {
+  return ((uint32_t)(((uint64_t)n * m) >> 32) + n) >> s;
+}
+TTC_HD inline uint32_t fdiv(uint32_t n, const FastDiv& f) { return fdiv(n, f.m, f.s); }
+
+// Work-groups are dispatched round-robin over the 8 XCDs (work-group w runs
+// on XCD w % 8), each XCD with its own L2.
+constexpr uint32_t kXcds = 8;
 
 struct TileParams {
   int32_t rank;
@@ -138,6 +153,85 @@ struct RCParams {
 constexpr uint32_t kRcTabOOB = 0xC0000000u;
 constexpr long long kRcFastSpan = (1ll << 30) - 64;
 
+// Order in which a single-op launch hands out its row x column tiles.
+struct RCWalk {
+  uint32_t ntiles;     // tiles of the launch (no padding ids)
+  int32_t grid_order;  // as RCParams::grid_order
+  // Bands: the walk's dimension of `bandn` tiles with `bandin` tiles before
+  // it runs in bands of `bandw` tiles (the last one narrower), each band's
+  // tiles innermost.  bandw 0: no bands.
+  uint32_t bandw, bandn, bandin;
+  FastDiv dper, dband, dw, dwl;  // divisions by bandn * bandin, bandw * bandin, bandw, the last band's width
+};
+
+// Tile of work-group w: a permutation of [0, ntiles).
+// grid_order 3: XCD x (work-groups w % 8 == x) takes a contiguous share of
+// the tile numbering, so that the tiles in flight on one L2 are neighbours;
+// 2: the same within rounds of 512 tiles; otherwise tile w.  Then the bands:
+// tiles of a band neighbour each other on A's side and, one band's pass after
+// the other, on B's, so both sides' shared cache lines meet in the L2.
+TTC_HD inline uint32_t rc_tile_of(const RCWalk& p, uint32_t w) {
+  uint32_t id = w;
+  if (p.grid_order == 3) {
+    const uint32_t x = w % kXcds, q = p.ntiles / kXcds, rem = p.ntiles % kXcds;
+    id = x * q + (x < rem ? x : rem) + w / kXcds;
+  } else if (p.grid_order == 2) {
+    constexpr uint32_t kRound = 512, kPer = kRound / kXcds;
+    const uint32_t base = w / kRound * kRound, l = w - base;
+    if (base + kRound <= p.ntiles) id = base + l % kXcds * kPer + l / kXcds;
+  }
+  if (p.bandw) {
+    const uint32_t hi = fdiv(id, p.dper);
+    uint32_t r = id - hi * p.dper.d;
+    const uint32_t b = fdiv(r, p.dband);
+    r -= b * p.dband.d;
+    const bool last = (b + 1) * p.bandw > p.bandn;
+    const uint32_t low = last ? fdiv(r, p.dwl) : fdiv(r, p.dw);
+    const uint32_t x = b * p.bandw + (r - low * (last ? p.dwl.d : p.dw.d));
+    id = low + p.bandin * (x + p.bandn * hi);
+  }
+  return id;
+}
+
+// One dimension of a tile's row or column group, and one tiled dimension of
+// the tile grid, in the single-op launches.
+struct RCDim {
+  uint32_t d, m, s;  // division by the tile extent (FastDiv)
+  int32_t sa, sb;    // A and B byte strides
+};
+struct RCGridDim {
+  uint32_t d, m, s;  // division by the tiles along the dimension
+  uint32_t part;     // 1 / 2: its last tile is partial in the row / column group
+  int64_t tsa, tsb;  // element offset of the next tile along it, in A and B
+};
+
+// Single-op row x column launch (ttc_rc.hpp, RCLane): each lane keeps one
+// vector of rows of the read walk (lane tid: column jl + it * kA of slot it,
+// jl = tid / la, rows (tid % la) * VA ...) and one vector of columns of the
+// write walk (row il + it * kB, il = tid / lb, columns (tid % lb) * VB ...).
+// Everything a tile needs besides is two slot-ordered offset tables.  The
+// records in use lie together at the front of dim and grid: the kernel reads
+// them from the kernel arguments with scalar loads.
+struct RCLaneParams {
+  int32_t R, C;        // rows and columns of a full tile
+  int32_t Rl, Cl;      // of the last tile along the split dimensions
+  int32_t RP;          // LDS pitch of a column (R | 1)
+  int32_t kA, kB;      // column step of the read walk, row step of the write walk
+  uint32_t la, lam, las;  // division by R / VA (lanes per column)
+  uint32_t lb, lbm, lbs;  // division by C / VB (lanes per row)
+  int32_t spare;       // LDS element where lanes past the walk stage (VA elements)
+  int32_t tab;         // byte offset of the tables in LDS: colS[kA * NIA] rowS[kB * NIB] rowA[R] colB[C]
+  int32_t na, nb;      // dimensions of the row group, the column group
+  int32_t grank;       // tiled grid dimensions, in walk order
+  RCWalk walk;
+  RCDim dim[kMaxDim];  // row group, then column group
+  RCGridDim grid[kMaxDim];
+};
+
+// Elements per thread per tile side of the row x column kernels: as many as
+// fit 128 bytes, at most 32.
+constexpr int rc_elems(int bytes) { return 128 / bytes > 32 ? 32 : 128 / bytes; }
+
 // Row copy for perm[0] == 0, where A and B share the stride-1 dimension:
 // a row is one position of the other dimensions, the rows are walked in B
 // order, and each lane moves one vector of V elements of dimension 0.
@@ -161,9 +255,5 @@ struct RCTile {
   int64_t a, b;
   uint32_t flags, pad_;
 };
-
-// Elements per thread per tile side of the row x column kernels: as many as
-// fit 128 bytes, at most 32.
-constexpr int rc_elems(int bytes) { return 128 / bytes > 32 ? 32 : 128 / bytes; }
 
 }  // namespace ttc

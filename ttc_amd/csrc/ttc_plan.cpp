@@ -476,6 +476,7 @@ ttc_status_t build_params(const Geometry& g, const int* tile, int ta, int tb, in
 // LDS per work-group (tile data plus offset tables): four 256-thread
 // work-groups per CU (160 KiB of LDS).
 static constexpr int kRcLdsBudget = 40960 * (kRcThreads / 256);
+static constexpr long long kLaneMaxTiles = 1ll << 23;  // work-groups of one launch (HIP counts a grid's threads in 32 bits)
 static constexpr long long kRcFastTiles = 2048;  // fewest tiles of a launch on the lane-fixed walk
 
 int max_rc_volume(int ta, int tb) {
@@ -732,6 +733,133 @@ ttc_status_t build_rc_params(const Geometry& g, const int* tile, int ta, int tb,
   return TTC_SUCCESS;
 }
 
+// Largest byte offsets of a group's dimensions on both sides.
+static void group_span(const Geometry& g, const int* tile, const int* grp, int n, int szA, int szB, long long& oa,
+                       long long& ob) {
+  oa = ob = 0;
+  for (int m = 0; m < n; ++m) {
+    oa += (long long)(tile[grp[m]] - 1) * g.sa[grp[m]] * szA;
+    ob += (long long)(tile[grp[m]] - 1) * g.sb[grp[m]] * szB;
+  }
+}
+
+// Row and column groups of a tile on the one-tile-per-work-group walk.
+struct LaneFit {
+  int na, nb, ga[kMaxDim], gb[kMaxDim];
+  long long R, C, Rl, Cl, ntiles, kA, kB;
+};
+
+// Whether the instance with 1/div of the family's slots covers the tile: all
+// lanes of a column (row) in one work-group and enough slots on both sides.
+static bool lane_fit(const Geometry& g, const int* tile, int szA, int szB, int va, int vb, int div, LaneFit& f) {
+  if (g.elements == 0 || !rc_groups(g, tile, f.na, f.ga, f.nb, f.gb)) return false;
+  const int p0 = g.perm[0];
+  if (tile[0] % va || tile[p0] % vb || g.size[0] % va || g.size[p0] % vb) return false;
+  f.R = f.C = f.ntiles = 1;
+  for (int m = 0; m < f.na; ++m) f.R *= tile[f.ga[m]];
+  for (int m = 0; m < f.nb; ++m) f.C *= tile[f.gb[m]];
+  for (int k = 0; k < g.rank; ++k) {
+    if (tile[k] < 1 || tile[k] > g.size[k]) return false;
+    f.ntiles *= (g.size[k] + tile[k] - 1) / tile[k];
+    if (f.ntiles > kLaneMaxTiles) return false;
+  }
+  const long long la = f.R / va, lb = f.C / vb, nia = rc_elems(szA) / va / div, nib = rc_elems(szB) / vb / div;
+  if (la < 1 || lb < 1 || la > kRcThreads || lb > kRcThreads) return false;
+  f.kA = kRcThreads / la;
+  f.kB = kRcThreads / lb;
+  if (f.kA * nia < f.C || f.kB * nib < f.R) return false;
+  const int ka = f.ga[f.na - 1], kb = f.gb[f.nb - 1];
+  f.Rl = f.R / tile[ka] * (g.size[ka] % tile[ka] ? g.size[ka] % tile[ka] : tile[ka]);
+  f.Cl = f.C / tile[kb] * (g.size[kb] % tile[kb] ? g.size[kb] % tile[kb] : tile[kb]);
+  // Real offsets stay below the buffer range 2^31; where one group's entries
+  // can be kRcTabOOB, the other group's stay below kRcFastSpan, so that the
+  // sums are out of range and do not wrap.
+  long long ra, rb, ca, cb;
+  group_span(g, tile, f.ga, f.na, szA, szB, ra, rb);
+  group_span(g, tile, f.gb, f.nb, szA, szB, ca, cb);
+  if (ra + ca + 64 >= INT_MAX || rb + cb + 64 >= INT_MAX) return false;
+  const bool oobRowA = f.kA * la < kRcThreads || f.Rl < f.R, oobColA = f.kA * nia > f.C || f.Cl < f.C;
+  const bool oobColB = f.kB * lb < kRcThreads || f.Cl < f.C, oobRowB = f.kB * nib > f.R || f.Rl < f.R;
+  return !(oobRowA && ca >= kRcFastSpan) && !(oobColA && ra >= kRcFastSpan) && !(oobColB && rb >= kRcFastSpan) &&
+         !(oobRowB && cb >= kRcFastSpan);
+}
+
+bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int va, int vb, int grid_order,
+                       int tile_order, int div, RCLaneParams& p, int& lds_bytes) {
+  const int szA = dtype_bytes(ta), szB = dtype_bytes(tb);
+  LaneFit f;
+  if (!lane_fit(g, tile, szA, szB, va, vb, div, f)) return false;
+  std::memset(&p, 0, sizeof(p));
+  const int na = f.na, nb = f.nb, *ga = f.ga, *gb = f.gb, ka = ga[na - 1], kb = gb[nb - 1];
+  const long long R = f.R, C = f.C, Rl = f.Rl, Cl = f.Cl, kA = f.kA, kB = f.kB;
+  const long long la = R / va, lb = C / vb, nia = rc_elems(szA) / va / div, nib = rc_elems(szB) / vb / div;
+  long long gk[kMaxDim];
+  for (int k = 0; k < g.rank; ++k) gk[k] = (g.size[k] + tile[k] - 1) / tile[k];
+  p.R = (int32_t)R;
+  p.C = (int32_t)C;
+  p.Rl = (int32_t)Rl;
+  p.Cl = (int32_t)Cl;
+  p.RP = (int32_t)(R | 1);
+  p.kA = (int32_t)kA;
+  p.kB = (int32_t)kB;
+  const FastDiv dla = make_fastdiv((uint32_t)la), dlb = make_fastdiv((uint32_t)lb);
+  p.la = dla.d, p.lam = dla.m, p.las = dla.s;
+  p.lb = dlb.d, p.lbm = dlb.m, p.lbs = dlb.s;
+  // LDS: everything the read walk stages (kA * nia columns), everything the
+  // write walk reads (kB * nib rows of the last column), a spare vector
+  const int le = lds_elem_bytes(ta, tb);
+  const long long reach = std::max(p.RP * kA * nia, kB * nib + (C - 1) * p.RP);
+  const long long data = ((reach + va) * le + 15) / 16 * 16;
+  const long long tab = kA * nia + kB * nib + R + C;
+  if (data + tab * 4 > 65536) return false;
+  p.spare = (int32_t)reach;
+  p.tab = (int32_t)data;
+  lds_bytes = (int)(data + tab * 4);
+  p.na = na;
+  p.nb = nb;
+  auto set_dim = [&](RCDim& d, int k) {
+    const FastDiv q = make_fastdiv((uint32_t)tile[k]);
+    d.d = q.d, d.m = q.m, d.s = q.s;
+    d.sa = (int32_t)(g.sa[k] * szA);
+    d.sb = (int32_t)(g.sb[k] * szB);
+  };
+  for (int m = 0; m < na; ++m) set_dim(p.dim[m], ga[m]);
+  for (int m = 0; m < nb; ++m) set_dim(p.dim[na + m], gb[m]);
+  for (int q = 0; q < g.rank; ++q) {
+    const int k = tile_order >= 2 ? g.perm[q] : q;
+    if (gk[k] <= 1) continue;
+    RCGridDim& d = p.grid[p.grank++];
+    const FastDiv q2 = make_fastdiv((uint32_t)gk[k]);
+    d.d = q2.d, d.m = q2.m, d.s = q2.s;
+    d.part = (k == ka && Rl < R ? 1u : 0u) | (k == kb && Cl < C ? 2u : 0u);
+    d.tsa = (int64_t)tile[k] * g.sa[k];
+    d.tsb = (int64_t)tile[k] * g.sb[k];
+  }
+  p.walk.ntiles = (uint32_t)f.ntiles;
+  p.walk.grid_order = kernel_grid_order(grid_order);
+  if (tile_order >= 2) {
+    // B order in bands along the row group's outermost tiled dimension,
+    // unless that dimension is the innermost already
+    const long long band = tile_order == 4 ? 16 : 8;
+    int kg = -1;
+    for (int m = na - 1; m >= 0 && kg < 0; --m)
+      if (gk[ga[m]] > 1) kg = ga[m];
+    long long before = 1;
+    for (int q = 0; q < g.rank && g.perm[q] != kg; ++q) before *= gk[g.perm[q]];
+    if (kg >= 0 && before > 1) {
+      const long long nk = gk[kg], w = std::min(band, nk);
+      p.walk.bandw = (uint32_t)w;
+      p.walk.bandn = (uint32_t)nk;
+      p.walk.bandin = (uint32_t)before;
+      p.walk.dper = make_fastdiv((uint32_t)(nk * before));
+      p.walk.dband = make_fastdiv((uint32_t)(w * before));
+      p.walk.dw = make_fastdiv((uint32_t)w);
+      p.walk.dwl = make_fastdiv((uint32_t)(nk % w ? nk % w : w));
+    }
+  }
+  return true;
+}
+
 // Offsets of tile row i (A and B) and tile column j: the mixed-radix
 // decomposition the kernel's setup() performs.
 static void rc_row(const RCParams& p, int i, int32_t& oa, int32_t& ob) {
@@ -865,6 +993,111 @@ static int rc_whole_extent_tiles(const Geometry& g, int va, int vb, int vmax, in
   return std::min(n, max_out);
 }
 
+// Cost of a launch of one work-group per tile, in bytes of HBM traffic (a fit
+// of 79 shapes x ~190 tiles, measured: the tile it picks is 2.6% (mean) behind
+// each shape's fastest, the run-length score of choose_rc_tile's 8%): the
+// bytes moved plus what partial cache lines add to each contiguous run, each
+// tile's fixed cost and that of its slots (issued whether or not they hold an
+// element), and the latency of a tile, which the whole launch waits for once.
+static double lane_cost(const Geometry& g, const int* tile, int szA, int szB, int va, int vb, int div, bool beta,
+                        const LaneFit& f) {
+  long long ra, rb;
+  tile_runs(g, tile, ra, rb);
+  const double N = (double)g.elements, m = beta ? 2.0 : 1.0;
+  const double ba = std::min(8192.0, (double)ra * szA), bb = std::min(8192.0, (double)rb * szB);
+  const double slots = rc_elems(szA) / va / div + rc_elems(szB) / vb / div * m;
+  return N * szA * (1.0 + 64.0 / ba) + N * szB * m * (1.0 + 180.0 / bb) + (double)f.ntiles * (600.0 + 1300.0 * slots) +
+         1000.0 * (double)(f.R * f.C) * (szA + szB * m);
+}
+
+// Tile of a launch of one work-group per tile: run-length targets on both
+// sides, tiles covering short leading extents whole, and of each that the
+// walk does not fit, the largest that fits along a group's outermost
+// dimension; the cheapest by lane_cost.
+bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile) {
+  if (g.elements == 0 || g.rank < 2 || g.perm[0] == 0) return false;
+  const int szA = dtype_bytes(ta), szB = dtype_bytes(tb), vmax = max_rc_volume(ta, tb);
+  double best = -1.0;
+  int cand[kMaxDim];
+  uint64_t seen[512] = {0};  // tiles already weighed (many run targets meet in one tile)
+  auto first_time = [&](const int* c) {
+    uint64_t h = 1469598103934665603ull;
+    for (int k = 0; k < g.rank; ++k) h = (h ^ (uint64_t)c[k]) * 1099511628211ull;
+    h |= 1;
+    size_t i = (h >> 20) % 512;
+    for (int tries = 0; tries < 8; ++tries, i = (i + 1) % 512) {
+      if (seen[i] == h) return false;
+      if (seen[i] == 0) {
+        seen[i] = h;
+        return true;
+      }
+    }
+    return true;
+  };
+  auto consider = [&](const int* c) {
+    LaneFit f;
+    for (int div = 2; div >= 1; --div) {
+      if (!lane_fit(g, c, szA, szB, va, vb, div, f)) continue;
+      const double cost = lane_cost(g, c, szA, szB, va, vb, div, beta, f);
+      // (the plan keeps the family's parameters too, within its LDS budget)
+      long long RP, data, tab;
+      rc_layout(f.R, f.C, f.R, f.C, 0, 0, lds_elem_bytes(ta, tb), false, RP, data, tab);
+      if ((best < 0.0 || cost < best) && data + tab * 4 <= kRcLdsBudget) {
+        best = cost;
+        for (int k = 0; k < kMaxDim; ++k) tile[k] = k < g.rank ? c[k] : 1;
+      }
+      return true;
+    }
+    return false;
+  };
+  // a tile, or the largest along a group's outermost dimension that has
+  // enough slots for the other group's extent
+  auto weigh = [&](int* c) {
+    if (consider(c)) return;
+    int na, nb, ga[kMaxDim], gb[kMaxDim];
+    if (!rc_groups(g, c, na, ga, nb, gb)) return;
+    long long R = 1, C = 1;
+    for (int m = 0; m < na; ++m) R *= c[ga[m]];
+    for (int m = 0; m < nb; ++m) C *= c[gb[m]];
+    auto shrink = [&](int k, long long other, long long all, int v_other, int v_own, int slots) {
+      if (other < v_other || other / v_other > kRcThreads) return;
+      const long long most = std::min<long long>(kRcThreads / (other / v_other) * slots, (long long)kRcThreads * v_own);
+      const int keep = c[k], a = align_of(g, k, va, vb);
+      const long long t = most / (all / keep) / a * a;
+      if (t < a || t >= keep) return;
+      c[k] = (int)t;
+      consider(c);
+      c[k] = keep;
+    };
+    shrink(gb[nb - 1], R, C, va, vb, rc_elems(szA) / va);
+    shrink(ga[na - 1], C, R, vb, va, rc_elems(szB) / vb);
+  };
+  for (int ra = 1; ra <= vmax; ra *= 2)
+    for (int rb = 1; rb <= vmax; rb *= 2) {
+      const long long v = (long long)ra * rb;
+      if (v > 2LL * vmax || v * 16 < vmax) continue;
+      tile_for_runs(g, va, vb, vmax, szA, szB, ra, rb, cand);
+      if (!first_time(cand)) continue;
+      int base[kMaxDim];
+      std::memcpy(base, cand, sizeof(base));
+      weigh(cand);
+      long long vol = 1;
+      for (int k = 0; k < g.rank; ++k) vol *= base[k];
+      for (int room = vmax / 2; room <= vmax; room *= 2) {
+        if (2 * vol > room) continue;
+        std::memcpy(cand, base, sizeof(cand));
+        rc_grow(g, cand, room);
+        if (first_time(cand)) weigh(cand);
+      }
+    }
+  for (int vol = vmax / 2; vol <= vmax; vol *= 2) {
+    int whole[2 * kMaxDim][kMaxDim];
+    const int nw = rc_whole_extent_tiles(g, va, vb, vol, whole, 2 * kMaxDim);
+    for (int i = 0; i < nw; ++i) weigh(whole[i]);
+  }
+  return best >= 0.0;
+}
+
 bool choose_rc_tile(const Geometry& g, int ta, int tb, int va, int vb, int run_a, int run_b, int* tile,
                     double* score) {
   if (g.elements == 0 || g.rank < 2 || g.perm[0] == 0) return false;
@@ -979,9 +1212,17 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
   } else {
     int rc_tile[kMaxDim];
     double rc_score = -1.0;
-    const bool rc_ok = fam != kFamilyBox &&
+    const bool lane = fam != kFamilyBox && pl->one_tile && run_a == 0 && run_b == 0 &&
+                      choose_lane_tile(g, pl->type_a, pl->type_b, va, vb, !pl->beta_is_zero, rc_tile);
+    // (a caller that names the family is refused the shapes choose_rc_tile refuses)
+    if (lane && fam == kFamilyRC) {
+      int t[kMaxDim];
+      if (!choose_rc_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, t, nullptr)) return TTC_ERROR_UNSUPPORTED;
+    }
+    if (lane) fam = kFamilyRC;
+    const bool rc_ok = fam != kFamilyBox && !lane &&
                        choose_rc_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, rc_tile, &rc_score);
-    if (fam == kFamilyRC && !rc_ok) return TTC_ERROR_UNSUPPORTED;
+    if (fam == kFamilyRC && !rc_ok && !lane) return TTC_ERROR_UNSUPPORTED;
     if (fam != kFamilyRC) choose_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, tile);
     if (fam == 0) {
       // The row x column kernel issues all of a tile's slots: it wins when
@@ -1009,6 +1250,14 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     pl->p.ntiles = pl->rc.ntiles;
     pl->p.V = pl->rc.R * pl->rc.C;
     pl->p.grid_order = pl->rc.grid_order;
+    // one tile per work-group unless the caller asks for resident
+    // work-groups or LDS buffers, which only the pipelined kernel has
+    pl->lane_div = 0;
+    if (pl->one_tile && st == TTC_SUCCESS)
+      for (int div = 2; div >= 1 && pl->lane_div == 0; --div)
+        if (build_lane_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->tile_order, div, pl->lane,
+                              pl->lane_lds))
+          pl->lane_div = div;
   } else {
     std::memset(&pl->rc, 0, sizeof(pl->rc));
     st = build_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->p, pl->lds_bytes, pl->lds_pad);
@@ -1024,6 +1273,12 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
 extern "C" ttc_status_t ttc_plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim,
                                         const int* perm, const int* size, const int* lda, const int* ldb,
                                         int beta_is_zero, const ttc_config_t* cfg) {
+  return plan_create(plan, type_a, type_b, dim, perm, size, lda, ldb, beta_is_zero, cfg, false);
+}
+
+ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim, const int* perm,
+                              const int* size, const int* lda, const int* ldb, int beta_is_zero,
+                              const ttc_config_t* cfg, bool grouped) {
   if (!plan) return TTC_ERROR_INVALID_VALUE;
   *plan = nullptr;
   if (!pair_supported(type_a, type_b)) return TTC_ERROR_UNSUPPORTED;
@@ -1059,6 +1314,9 @@ extern "C" ttc_status_t ttc_plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, tt
   // of resident work-groups (measured +1.4% over the C2 permutations)
   pl->lds_buffers = c.lds_buffers == 0 ? 2 : c.lds_buffers;
   pl->wg_per_cu = c.wg_per_cu;
+  bool explicit_tile = false;
+  for (int k = 0; k < TTC_MAX_DIM; ++k) explicit_tile |= c.tile[k] != 0;
+  pl->one_tile = !grouped && c.wg_per_cu == 0 && (c.lds_buffers == 0 || !explicit_tile);
   auto in_list = [](int w, int bytes) {
     for (int x : vec_widths(bytes))
       if (x == w) return true;
@@ -1160,7 +1418,7 @@ extern "C" ttc_status_t ttc_plan_get_info(ttc_plan_t pl, ttc_plan_info_t* info) 
     info->cols = pl->rc.C;
   }
   info->lds_buffers = pl->family == kFamilyRC ? pl->rc.nbuf : 1;
-  info->lane_fixed = pl->family == kFamilyRC ? pl->rc.fast : 0;
+  info->lane_fixed = pl->family == kFamilyRC ? (pl->lane_div || pl->rc.fast) : 0;
   if (pl->family == kFamilyRow) {
     info->slots_a = info->slots_b = kRowUnroll;
     info->tiles = g.size[0] > 0 ? g.elements / g.size[0] : 0;  // rows

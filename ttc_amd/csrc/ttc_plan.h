@@ -95,6 +95,14 @@ ttc_status_t build_rc_params(const Geometry& g, const int* tile, int ta, int tb,
                              int tile_order, RCParams& p, int& lds_bytes, int nbuf = 1);
 bool choose_rc_tile(const Geometry& g, int ta, int tb, int va, int vb, int run_a, int run_b, int* tile,
                     double* score);
+// One-tile-per-work-group launch of a row x column tile (ttc_lane.hpp): its
+// parameters for the instance of 1/div of the family's slots, or false where
+// the tile does not fit it (more than 256 lanes across a column or a row, too
+// few slots, offsets that could meet kRcTabOOB); such tiles take the pipelined
+// kernel.  choose_lane_tile: the heuristic tile of such a launch.
+bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int va, int vb, int grid_order,
+                       int tile_order, int div, RCLaneParams& p, int& lds_bytes);
+bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile);
 // The launch's LDS offset tables (p.ntab entries, the layout of RCParams),
 // as the kernel's setup() builds them.
 void rc_fill_tables(const RCParams& p, int32_t* out);
@@ -102,6 +110,12 @@ void rc_fill_tables(const RCParams& p, int32_t* out);
 // Row-copy family (perm[0] == 0): launch parameters for vectors of v
 // elements; TTC_ERROR_UNSUPPORTED when the shape does not fit the kernel.
 ttc_status_t build_row_params(const Geometry& g, int ta, int tb, int v, RowParams& p);
+
+// ttc_plan_create; grouped: for an op of a grouped launch, whose work-groups
+// walk several tiles each.
+ttc_status_t plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim, const int* perm,
+                         const int* size, const int* lda, const int* ldb, int beta_is_zero, const ttc_config_t* cfg,
+                         bool grouped);
 
 }  // namespace ttc
 
@@ -120,6 +134,10 @@ struct ttc_plan_s {
   int tile_order;        // 1 A order, 2 B order, 3 / 4 grouped B order (row x column tiles only)
   int lds_buffers;       // LDS tile buffers of the row x column kernel
   ttc::RCParams rc;
+  int one_tile;          // row x column tiles: one tile per work-group where the tile fits (ttc_lane.hpp)
+  int lane_div;          // one tile per work-group: 1 / 2 = instance, 0 = the pipelined kernel on rc
+  int lane_lds;          // its LDS bytes
+  ttc::RCLaneParams lane;
   ttc::RowParams row;
   ttc_plan_s* fallback;  // scalar-vector plan for misaligned pointers (may be null)
 };

@@ -125,6 +125,10 @@ ttc_status_t launch_plan(const ttc_plan_s* pl, const void* A, void* B, double al
                ? TTC_SUCCESS
                : TTC_ERROR_HIP;
   }
+  if (use->family == kFamRC && use->lane_div)
+    return e->launch_lane[use->lane_div - 1](use->lane, A, B, alpha, beta, (size_t)use->lane_lds, s) == hipSuccess
+               ? TTC_SUCCESS
+               : TTC_ERROR_HIP;
   const bool fast = use->family == kFamRC && use->rc.fast;
   const unsigned grid = grid_size(use->p.ntiles, pl->wg_per_cu, fast ? e->func_fast : e->func, use->lds_bytes,
                                   use->family == kFamRC ? kRcThreads : kThreads);
@@ -232,6 +236,11 @@ extern "C" ttc_status_t ttc_execute_fp8(ttc_plan_t pl, const void* A, void* B, d
                ? TTC_SUCCESS
                : TTC_ERROR_HIP;
   }
+  if (use->family == kFamRC && use->lane_div)
+    return e->launch_fp8_lane[use->lane_div - 1](use->lane, A, B, al, d_scale_in, amax_in, fp8_max, scale, amax_out,
+                                                 d_scale_inv_out, (size_t)use->lane_lds, s) == hipSuccess
+               ? TTC_SUCCESS
+               : TTC_ERROR_HIP;
   if (use->family == kFamRC) {
     const bool fast = use->rc.fast != 0;
     const unsigned grid = grid_size(use->p.ntiles, pl->wg_per_cu, fast ? e->func_fast : e->func, use->lds_bytes,
