@@ -1,0 +1,45 @@
+"""GPU parity of the row copy with one chunk per work-group at the row
+lengths where its unaligned vectors can go wrong: rows shorter than, equal to
+and just past a vector, odd rows, one chunk and several, padded leading
+dimensions and misaligned pointers; bit-exact against the oracle."""
+import numpy as np
+import pytest
+
+from common import BF16, CODE, F16, S, same_bits, to_device
+from oracle import oracle as orc
+from test_gpu_cast_batch import E4M3, E5M2, _heavy_input
+from test_gpu_parity import check
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 33, 127, 129]
+
+
+@pytest.mark.parametrize("code", ["s", "d", "c", "z", "b", "h", "sb", "bs", "sd", "ds", "cz"])
+def test_row_lengths(gpu, code):
+    tA, tB = CODE[code]
+    for n0 in ROWS:
+        for pad in (0, 3):
+            size = [n0, 13, 22]
+            lda = [n0 + pad, 13, 22 + pad] if pad else None
+            ldb = [n0 + pad + 1, 22 + pad, 13] if pad else None
+            for beta in (0.0, 0.75):
+                check(gpu, tA, tB, [0, 2, 1], size, 1.25, beta, lda, ldb, seed=n0)
+        check(gpu, tA, tB, [0, 2, 1], [n0, 13, 22], 1.0, 0.0, seed=n0, offset_a=1, offset_b=1)
+
+
+@pytest.mark.parametrize("tA,tB", [(S, E4M3), (BF16, E4M3), (F16, E5M2)])
+def test_row_lengths_fp8(gpu, tA, tB):
+    import torch
+    from ttc_amd import runtime as rt
+    for n0 in ROWS:
+        size = [n0, 37, 90]
+        n = int(np.prod(size))
+        A = _heavy_input(tA, n, n0)
+        dA, dB = to_device(A, gpu), torch.zeros(n, dtype=torch.uint8, device=gpu)
+        amax = torch.full((1,), -1.0, dtype=torch.float32, device=gpu)
+        want = np.zeros(n, np.uint8)
+        want_amax = orc.cast_fp8(tA, tB, A, want, 0.5, 3.5, [0, 2, 1], size)
+        rt.Plan(tA, tB, [0, 2, 1], size, beta_is_zero=True).execute_fp8(dA, dB, 0.5, scale=3.5, amax_out=amax)
+        torch.cuda.synchronize()
+        assert same_bits(dB.cpu().numpy(), want) and float(amax.item()) == want_amax, (tA, tB, n0)

@@ -12,7 +12,8 @@
 namespace ttc {
 
 // kernel family (matches ttc_config_t.family)
-enum : int { kFamBox = 1, kFamRC = 2, kFamRow = 3 };
+// (kFamRowUnaligned: registry only, never a plan's family)
+enum : int { kFamBox = 1, kFamRC = 2, kFamRow = 3, kFamRowUnaligned = 4 };
 
 using LaunchFn = hipError_t (*)(const TileParams&, const void*, void*, double, double, unsigned, size_t, hipStream_t);
 using LaunchFp8Fn = hipError_t (*)(const TileParams&, const void*, void*, float, const float*, const float*, float,
@@ -39,6 +40,7 @@ struct KernelEntry {
   LaunchRCFn launch_rc;
   const void* func;
   LaunchRowFn launch_row;
+  LaunchRowFn launch_row_once;  // one chunk per work-group
   LaunchFp8RCFn launch_fp8_rc;
   // row x column family: the instance for RCParams::fast launches
   LaunchRCFn launch_rc_fast;
@@ -157,11 +159,32 @@ hipError_t launch_row(const RowParams& p, const void* A, void* B, double alpha, 
                          0, s);
 }
 
+template <class OP, int V, int MODE, bool UNAL>
+hipError_t launch_row_once(const RowParams& p, const void* A, void* B, double alpha, double beta,
+                           const float* scale_in, const float* amax_in, float fp8_max, float scale_host,
+                           float* amax_out, float* scale_inv_out, unsigned grid, hipStream_t s) {
+  const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
+  typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  void* args[] = {const_cast<RowParams*>(&p), &a, &b, &alpha, &beta, &scale_in, &amax_in, &fp8_max, &scale_host,
+                  &amax_out, &scale_inv_out};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&row_once_kernel<OP, V, MODE, UNAL>), dim3(grid),
+                         dim3(kThreads), args, 0, s);
+}
+
 template <class OP, int V, int MODE>
 KernelEntry make_row_entry(int ta, int tb) {
   KernelEntry e{ta, tb, V, V, MODE, kFamRow, nullptr, nullptr, nullptr, nullptr, nullptr};
   e.launch_row = &launch_row<OP, V, MODE>;
+  e.launch_row_once = &launch_row_once<OP, V, MODE, false>;
   e.func = reinterpret_cast<const void*>(&row_kernel<OP, V, MODE>);
+  return e;
+}
+
+// Row copy in unaligned vectors (one chunk per work-group only).
+template <class OP, int V, int MODE>
+KernelEntry make_row_unaligned_entry(int ta, int tb) {
+  KernelEntry e{ta, tb, V, V, MODE, kFamRowUnaligned, nullptr, nullptr, nullptr, nullptr, nullptr};
+  e.launch_row_once = &launch_row_once<OP, V, MODE, true>;
   return e;
 }
 

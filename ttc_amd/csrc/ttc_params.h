@@ -239,9 +239,11 @@ constexpr int kRowUnroll = 4;  // vectors in flight per lane in the row-copy ker
 
 struct RowParams {
   uint32_t total;         // rows * nv (< 2^31)
-  uint32_t nv;            // vectors per row: extent of dimension 0 / V
+  uint32_t nv;            // vectors per row: extent of dimension 0 / V (rounded up on unaligned vectors)
   FastDiv dnv;
   int32_t rank;           // row dimensions, in B order
+  int32_t n0;             // extent of dimension 0
+  int32_t xcd_share;      // one chunk per work-group: XCDs take contiguous shares of the chunks
   int32_t pad_;
   FastDiv dn[kMaxDim];    // their extents
   int64_t sa[kMaxDim];    // A byte strides
@@ -255,5 +257,14 @@ struct RCTile {
   int64_t a, b;
   uint32_t flags, pad_;
 };
+
+// One-chunk-per-work-group row copy (row_once_kernel): vectors in flight per
+// lane.  16-byte vectors: one, so that a launch has the most work-groups (200
+// MiB fp32: 6.0 TB/s with one, 5.7 with two, 5.6 with four); narrower and
+// unaligned ones: two (fp64 rows of 9 with beta: 4.5 with one, 4.9 with two);
+// fp8 casts: four, since each work-group also reduces its amax.
+constexpr int row_once_unroll(int bytes_a, int bytes_b, int v, bool fp8, bool unaligned) {
+  return fp8 ? 4 : ((v * bytes_a == 16 || v * bytes_b == 16) && !unaligned ? 1 : 2);
+}
 
 }  // namespace ttc

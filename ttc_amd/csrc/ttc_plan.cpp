@@ -939,7 +939,36 @@ ttc_status_t build_row_params(const Geometry& g, int ta, int tb, int v, RowParam
   p.total = (uint32_t)total;
   p.nv = (uint32_t)nv;
   p.dnv = make_fastdiv((uint32_t)nv);
+  p.n0 = g.size[0];
   return TTC_SUCCESS;
+}
+
+// The one-chunk-per-work-group launch of row copy p (aligned vectors of v
+// elements): unaligned vectors where they are wider.  Rows shorter than a
+// cache line share lines with their neighbours in A and B, which then meet in
+// one L2: XCD shares (fp32 rows of 5: 2.6 -> 3.3 TB/s, bf16 rows of 3: 1.3 ->
+// 1.6; rows of 512 bytes and more measured 1-3% slower with them).
+static void build_row_once(ttc_plan_s* pl, int v) {
+  const int szA = dtype_bytes(pl->type_a), szB = dtype_bytes(pl->type_b), n0 = pl->row.n0;
+  const bool fp8 = szB == 1;
+  pl->row1 = pl->row;
+  pl->row1_v = v;
+  pl->row1_unaligned = 0;
+  pl->row1_grid = 0;
+  if (pl->row.total == 0 || pl->wg_per_cu > 0) return;
+  const bool may = !pl->vec_given && row_unaligned_mode(szA, szB, !pl->beta_is_zero, pl->nt_store != 0);
+  const int w = may ? row_unaligned_width(szA, szB, n0) : 1;
+  if (w > v) {
+    const uint32_t rows = pl->row.total / pl->row.nv;
+    pl->row1_v = w;
+    pl->row1_unaligned = 1;
+    pl->row1.nv = (uint32_t)((n0 + w - 1) / w);
+    pl->row1.dnv = make_fastdiv(pl->row1.nv);
+    pl->row1.total = rows * pl->row1.nv;
+  }
+  pl->row1.xcd_share = (long long)n0 * std::min(szA, szB) < 128;
+  const long long chunk = (long long)kThreads * row_once_unroll(szA, szB, pl->row1_v, fp8, pl->row1_unaligned != 0);
+  pl->row1_grid = (unsigned)((pl->row1.total + chunk - 1) / chunk);
 }
 
 static int rc_whole_extent_tiles(const Geometry& g, int va, int vb, int vmax, int (*out)[kMaxDim], int max_out) {
@@ -1195,6 +1224,7 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
       std::memset(&pl->p, 0, sizeof(pl->p));
       std::memset(&pl->rc, 0, sizeof(pl->rc));
       pl->row = rp;
+      build_row_once(pl, v);
       const long long chunk = (long long)kThreads * kRowUnroll;
       pl->p.ntiles = (uint32_t)((rp.total + chunk - 1) / chunk);
       pl->p.V = g.size[0];
@@ -1316,6 +1346,7 @@ ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t 
   pl->wg_per_cu = c.wg_per_cu;
   bool explicit_tile = false;
   for (int k = 0; k < TTC_MAX_DIM; ++k) explicit_tile |= c.tile[k] != 0;
+  pl->vec_given = c.vec_a != 0 || c.vec_b != 0;
   pl->one_tile = !grouped && c.wg_per_cu == 0 && (c.lds_buffers == 0 || !explicit_tile);
   auto in_list = [](int w, int bytes) {
     for (int x : vec_widths(bytes))

@@ -31,6 +31,20 @@ inline std::vector<int> row_widths(int bytes_a, int bytes_b) {
   return w;
 }
 
+// Widest vector of the row copy in unaligned vectors for rows of n0 elements
+// (1: none).  The kernel generator instantiates 2, 4, ... up to 16 bytes.
+inline int row_unaligned_width(int bytes_a, int bytes_b, int n0) {
+  int v = 1;
+  while (2 * v * (bytes_a > bytes_b ? bytes_a : bytes_b) <= 16 && 2 * v <= n0) v *= 2;
+  return v;
+}
+// With beta, elements wider than 2 bytes stay on aligned vectors, which
+// measured as fast or faster (fp64 rows of 9: 4.87 against 4.63 TB/s, fp32
+// rows of 127: 4.91 against 4.80).
+inline bool row_unaligned_mode(int bytes_a, int bytes_b, bool beta, bool nt) {
+  return !nt && (!beta || (bytes_a > bytes_b ? bytes_a : bytes_b) <= 2);
+}
+
 int dtype_bytes(int t);
 // Bytes of the LDS staging type (alpha * a in A's arithmetic) for a type pair.
 int lds_elem_bytes(int ta, int tb);
@@ -134,10 +148,14 @@ struct ttc_plan_s {
   int tile_order;        // 1 A order, 2 B order, 3 / 4 grouped B order (row x column tiles only)
   int lds_buffers;       // LDS tile buffers of the row x column kernel
   ttc::RCParams rc;
+  int vec_given;         // the caller chose the vector widths
   int one_tile;          // row x column tiles: one tile per work-group where the tile fits (ttc_lane.hpp)
   int lane_div;          // one tile per work-group: 1 / 2 = instance, 0 = the pipelined kernel on rc
   int lane_lds;          // its LDS bytes
   ttc::RCLaneParams lane;
   ttc::RowParams row;
+  ttc::RowParams row1;   // one chunk per work-group (row_once_kernel)
+  int row1_v, row1_unaligned;
+  unsigned row1_grid;    // 0: row_kernel (wg_per_cu given)
   ttc_plan_s* fallback;  // scalar-vector plan for misaligned pointers (may be null)
 };

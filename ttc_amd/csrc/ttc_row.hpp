@@ -105,4 +105,146 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
+// V elements with the alignment of one element: gfx950 takes vector accesses
+// at any such address.
+template <class T, int V> struct __attribute__((packed, aligned(sizeof(T)))) RowVec {
+  T x[V];
+};
+
+// One chunk of kThreads * U vectors per work-group.  The dispatcher keeps
+// every CU full to the end of the launch, where a work-group striding over
+// the whole tensor (row_kernel) leaves the chip in step with the slowest.
+//   UNAL: dimension 0 (extent n0 >= V) is not a whole number of aligned
+// vectors.  A row takes ceil(n0 / V) vectors at element alignment, the last
+// one shifted back to end at the row's end; its first elements are its
+// neighbour's too.  With beta == 0 both write the same values; with beta the
+// shifted lane stores only its own elements, since its neighbour's may
+// already hold their results.
+// Bound by HBM (16-byte vectors) or by the address arithmetic per vector
+// (narrow ones).  Striding work-groups -> this kernel, GB/s: fp32 200 MiB
+// copy 4740 -> 6010; bf16 128 x 4096 x 32 x 8 perm (0,2,1,3) 4760 -> 5340;
+// fp32 rows of 127 3890 -> 4730, of 5 2210 -> 3040; bf16 rows of 127
+// 2180 -> 4070, of 5 1270 -> 2240.
+template <class OP, int V, int MODE, bool UNAL>
+__global__ void __launch_bounds__(kThreads)
+    row_once_kernel(const RowParams p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
+                    double alpha, double beta, const float* __restrict__ scale_in, const float* __restrict__ amax_in,
+                    float fp8_max, float scale_host, float* __restrict__ amax_out,
+                    float* __restrict__ scale_inv_out) {
+  using TA = typename OP::TA;
+  using TB = typename OP::TB;
+  using L = typename OP::L;
+  constexpr bool FP8 = MODE == kModeFp8;
+  constexpr bool BETA = MODE == kModeBeta;
+  constexpr bool NT = MODE == kModeBzNt;
+  constexpr int U = row_once_unroll((int)sizeof(TA), (int)sizeof(TB), V, FP8, UNAL);
+  float scale = 1.0f;
+  if constexpr (FP8) {
+    scale = scale_host;
+    if (scale_in) {
+      scale = *scale_in;
+    } else if (amax_in) {
+      const float m = *amax_in;
+      scale = (m > 0.0f && m <= 3.402823466e38f) ? fp8_max / m : 1.0f;
+    }
+    if (scale_inv_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_inv_out = 1.0f / scale;
+  }
+  const typename OP::AL al = (typename OP::AL)alpha;
+  const typename OP::BE be = (typename OP::BE)beta;
+  uint32_t w = blockIdx.x;
+  if (p.xcd_share) {
+    const uint32_t x = w % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
+    w = x * q + (x < r ? x : r) + w / kXcds;
+  }
+  const uint32_t g0 = w * (uint32_t)(kThreads * U) + threadIdx.x;
+  const char* a = reinterpret_cast<const char*>(A);
+  char* b = reinterpret_cast<char*>(B);
+  int64_t ob[U];
+  bool ok[U];
+  int skip[U];  // UNAL: leading elements of a shifted vector that are its neighbour's
+  TA va[U][V];
+  TB old[U][V];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t g = g0 + (uint32_t)(u * kThreads);
+    ok[u] = g < p.total;
+    const uint32_t gg = ok[u] ? g : 0u;
+    const uint32_t row = fdiv(gg, p.dnv);
+    int32_t e = (int32_t)(gg - row * p.nv) * V;
+    skip[u] = 0;
+    if constexpr (UNAL) {
+      skip[u] = e + V > p.n0 ? e + V - p.n0 : 0;
+      e -= skip[u];
+    }
+    int64_t xa = (int64_t)e * (int64_t)sizeof(TA), xb = (int64_t)e * (int64_t)sizeof(TB);
+    uint32_t rem = row;
+#pragma unroll
+    for (int k = 0; k < kMaxDim; ++k) {
+      if (k < p.rank) {
+        const uint32_t q = fdiv(rem, p.dn[k]);
+        const uint32_t x = rem - q * p.dn[k].d;
+        rem = q;
+        xa += (int64_t)x * p.sa[k];
+        xb += (int64_t)x * p.sb[k];
+      }
+    }
+    ob[u] = xb;
+    if (!ok[u]) continue;
+    if constexpr (UNAL) {
+      const RowVec<TA, V> t = *reinterpret_cast<const RowVec<TA, V>*>(a + xa);
+      __builtin_memcpy(&va[u][0], &t, sizeof(t));
+      if constexpr (BETA) {
+        const RowVec<TB, V> o = *reinterpret_cast<const RowVec<TB, V>*>(b + xb);
+        __builtin_memcpy(&old[u][0], &o, sizeof(o));
+      }
+    } else {
+      vload<TA, V>(va[u], reinterpret_cast<const TA*>(a + xa));
+      if constexpr (BETA) vload<TB, V>(old[u], reinterpret_cast<const TB*>(b + xb));
+    }
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (!ok[u]) continue;
+    TB o[V];
+    if constexpr (FP8) {
+      L x[V];
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        x[v] = OP::prod(al, va[u][v]);
+        amax = fmaxf(amax, fabsf(x[v]));
+      }
+      if constexpr (V == 1) {
+        o[0] = OP::outs(x[0], scale);
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; v += 2) OP::outs2(x[v], x[v + 1], scale, o[v], o[v + 1]);
+      }
+    } else if constexpr (BETA) {
+#pragma unroll
+      for (int v = 0; v < V; ++v) o[v] = OP::outb(OP::prod(al, va[u][v]), be, old[u][v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; ++v) o[v] = OP::out(OP::prod(al, va[u][v]));
+    }
+    TB* const dst = reinterpret_cast<TB*>(b + ob[u]);
+    if constexpr (UNAL) {
+      if (!BETA || skip[u] == 0) {
+        RowVec<TB, V> t;
+        __builtin_memcpy(&t, &o[0], sizeof(t));
+        *reinterpret_cast<RowVec<TB, V>*>(dst) = t;
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          if (v >= skip[u]) dst[v] = o[v];
+      }
+    } else {
+      vstore<TB, V, NT>(dst, o);
+    }
+  }
+  if constexpr (FP8) {
+    if (amax_out) block_amax_commit(amax, amax_out);
+  }
+}
+
 }  // namespace ttc

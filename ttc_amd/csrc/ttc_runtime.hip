@@ -109,6 +109,20 @@ const ttc_plan_s* variant_for(const ttc_plan_s* pl, const void* A, const void* B
   return nullptr;
 }
 
+// Row copy, one chunk per work-group.
+static ttc_status_t launch_row_chunks(const ttc_plan_s* use, const KernelEntry* e, int mode, const void* A, void* B,
+                                      double alpha, double beta, const float* scale_in, const float* amax_in,
+                                      float fp8_max, float scale, float* amax_out, float* scale_inv_out,
+                                      hipStream_t s) {
+  if (use->row1_unaligned)
+    e = find_kernel(use->type_a, use->type_b, use->row1_v, use->row1_v, mode, kFamRowUnaligned);
+  if (!e) return TTC_ERROR_UNSUPPORTED;
+  return e->launch_row_once(use->row1, A, B, alpha, beta, scale_in, amax_in, fp8_max, scale, amax_out, scale_inv_out,
+                            use->row1_grid, s) == hipSuccess
+             ? TTC_SUCCESS
+             : TTC_ERROR_HIP;
+}
+
 static bool is_fp8_type(int t) { return t == TTC_E4M3 || t == TTC_E5M2; }
 
 ttc_status_t launch_plan(const ttc_plan_s* pl, const void* A, void* B, double alpha, double beta, hipStream_t s) {
@@ -118,6 +132,8 @@ ttc_status_t launch_plan(const ttc_plan_s* pl, const void* A, void* B, double al
   const int mode = pl->beta_is_zero ? (pl->nt_store ? kModeBzNt : kModeBz) : kModeBeta;
   const KernelEntry* e = find_kernel(pl->type_a, pl->type_b, use->va, use->vb, mode, use->family);
   if (!e) return TTC_ERROR_UNSUPPORTED;
+  if (use->family == kFamRow && use->row1_grid)
+    return launch_row_chunks(use, e, mode, A, B, alpha, beta, nullptr, nullptr, 0.0f, 1.0f, nullptr, nullptr, s);
   if (use->family == kFamRow) {
     const unsigned grid = row_grid(use, pl->wg_per_cu, e->func);
     return e->launch_row(use->row, A, B, alpha, beta, nullptr, nullptr, 0.0f, 1.0f, nullptr, nullptr, grid, s) ==
@@ -229,6 +245,9 @@ extern "C" ttc_status_t ttc_execute_fp8(ttc_plan_t pl, const void* A, void* B, d
     amax_out = nullptr;
     d_scale_in = nullptr;
   }
+  if (use->family == kFamRow && use->row1_grid)
+    return launch_row_chunks(use, e, kModeFp8, A, B, alpha, 0.0, d_scale_in, amax_in, fp8_max, scale, amax_out,
+                             d_scale_inv_out, s);
   if (use->family == kFamRow) {
     const unsigned grid = row_grid(use, pl->wg_per_cu, e->func);
     return e->launch_row(use->row, A, B, alpha, 0.0, d_scale_in, amax_in, fp8_max, scale, amax_out, d_scale_inv_out,

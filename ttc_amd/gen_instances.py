@@ -48,6 +48,23 @@ def row_widths(na, nb):
     return w
 
 
+def row_unaligned_widths(na, nb):
+    """Same rule as ttc::row_unaligned_widths (csrc/ttc_plan.h): vector widths
+    of the row copy in unaligned vectors."""
+    w = []
+    v = 2
+    while v * max(na, nb) <= 16:
+        w.append(v)
+        v *= 2
+    return w
+
+
+def row_unaligned_modes(na, nb, modes):
+    """Store modes it is instantiated for (csrc/ttc_plan.h
+    row_unaligned_mode)."""
+    return [m for m in modes if m in ("kModeBz", "kModeFp8") or (m == "kModeBeta" and max(na, nb) <= 2)]
+
+
 def op_for(ta, tb):
     if ta in F32_CLASS and tb in F32_CLASS:
         return "OpF32<%s, %s>" % (TYPES[ta][0], TYPES[tb][0])
@@ -100,6 +117,9 @@ def instance_files(ta, tb):
     # row-copy family (perm[0] == 0), one file per pair
     lines = ["      make_row_entry<%s, %d, %s>(TTC_%s, TTC_%s)," % (op, v, m, ta, tb)
              for v in row_widths(TYPES[ta][1], TYPES[tb][1]) for m in modes]
+    lines += ["      make_row_unaligned_entry<%s, %d, %s>(TTC_%s, TTC_%s)," % (op, v, m, ta, tb)
+              for v in row_unaligned_widths(TYPES[ta][1], TYPES[tb][1])
+              for m in row_unaligned_modes(TYPES[ta][1], TYPES[tb][1], modes)]
     name = "inst_%s_%s_row" % (ta.lower(), tb.lower())
     src = ["// Generated by ttc_amd/gen_instances.py -- do not edit.", '#include "../ttc_launch.hpp"',
            "namespace ttc {", "const KernelEntry* %s(int* n) {" % name, "  static const KernelEntry entries[] = {"]
