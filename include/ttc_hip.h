@@ -181,8 +181,10 @@ void ttc_legacy_transpose(ttc_dtype_t type_a, ttc_dtype_t type_b, const void* A,
                           const int* ldb, const ttc_config_t* cfg, const char* name);
 
 /* Batched grouped transpositions (no counterpart in the reference, which
- * runs one transposition per host call).  All ops run in ONE persistent
- * kernel driven by a device-side work table built at creation. */
+ * runs one transposition per host call), driven by a device-side work table
+ * built at creation: ONE launch of one work-group per tile for all ops that
+ * take it, and a persistent launch per (kernel family, type) for the rest
+ * (box tiles, ops whose configuration sets lds_buffers). */
 typedef struct {
   ttc_dtype_t type_a, type_b; /* real or complex, A and B of the same class */
   int dim;
@@ -198,9 +200,9 @@ typedef struct {
 } ttc_batch_op_t;
 
 /* Creates the work table on the current device (allocates device memory).
- * wg_per_cu: work-group slices per CU in each group's grid (residency is
- * set by occupancy; more slices than resident work-groups balance uneven
- * ops); 0 = 96. */
+ * wg_per_cu: work-group slices per CU in the grid of each persistent launch
+ * (residency is set by occupancy; more slices than resident work-groups
+ * balance uneven ops); 0 = 96. */
 ttc_status_t ttc_batch_create(ttc_batch_t* batch, int nops, const ttc_batch_op_t* ops, int wg_per_cu);
 /* One grouped launch of every op. */
 ttc_status_t ttc_batch_execute(ttc_batch_t batch, ttc_stream_t stream);
@@ -223,8 +225,9 @@ ttc_status_t ttc_batch_destroy(ttc_batch_t batch);
  * GPU, of TTC_BATCH_WORKSPACE_BYTES, held until the process ends.  The table
  * is built on the host (host heap only) and copied with hipMemcpyAsync on
  * `stream`, ordered after that stream's earlier work; the call returns once
- * the kernels are enqueued.  A table larger than the workspace (about 24
- * bytes per tile plus about 1 KiB per op) returns TTC_ERROR_WORKSPACE.
+ * the kernels are enqueued.  A table larger than the workspace (about 1 KiB
+ * per op, plus about 24 bytes per tile of the ops in persistent launches)
+ * returns TTC_ERROR_WORKSPACE.
  * Every call on one GPU shares that GPU's workspace: calls on one stream
  * are ordered, but calls that overlap on one GPU (different streams or host
  * threads, without ordering between them) race. */

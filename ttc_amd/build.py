@@ -36,7 +36,7 @@ HIP_FLAGS = [
 ]
 CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-I" + INCLUDE, "-I" + CSRC]
 
-HEADERS = ["ttc_kernels.hpp", "ttc_rc.hpp", "ttc_lane.hpp", "ttc_row.hpp", "ttc_launch.hpp", "ttc_batch_kernels.hpp", "ttc_params.h",
+HEADERS = ["ttc_kernels.hpp", "ttc_rc.hpp", "ttc_lane.hpp", "ttc_row.hpp", "ttc_launch.hpp", "ttc_batch_kernels.hpp", "ttc_batch_one.hpp", "ttc_params.h",
            "ttc_plan.h", "ttc_runtime.h", "gen/inst_all.h"]
 VERSION = "0.2.0"
 
@@ -77,7 +77,7 @@ def _write_version():
 
 def _sources():
     inst, _ = gen_instances.generate()
-    batch = [os.path.join(CSRC, "ttc_batch_k_%s.hip" % pair) for pair in ("s", "d", "bf16", "f16", "c", "z")]
+    batch = [os.path.join(CSRC, "ttc_batch_k_%s.hip" % pair) for pair in ("one", "s", "d", "bf16", "f16", "c", "z")]
     hip = [os.path.join(CSRC, "ttc_runtime.hip"), os.path.join(CSRC, "ttc_batch.hip")] + batch + inst
     cxx = [os.path.join(CSRC, "ttc_plan.cpp"), _write_version()]
     return hip, cxx

@@ -3,20 +3,18 @@
 // replayed through a captured hipGraph.  The reference has no counterpart
 // (one transposition per host call, ttc/CUDAtranspose.py:395-429).
 //
-// Work table: one record per op (its tile parameters, pointers, scalars) and
-// one record per tile (origin offsets, partial-tile limits), ops grouped by
-// kernel family and type pair and ordered by variant (vector widths, beta
-// read or not) inside a group, each group's tiles numbered consecutively,
-// and a split of each group's tile range into one contiguous slice per
-// work-group, balanced by bytes moved.  One persistent launch per group
-// walks that group's slices, each op through its variant's walk (the
-// kernels are in ttc_batch_kernels.hpp).  Each op takes the family its own
-// plan chose: row x column tiles (a work-group rebuilds its LDS offset
-// tables when its slice crosses into the next op), row copies (dimension 0
-// in place; the unit of work is a chunk of vectors) or box tiles.  One
-// launch per group rather than per (group, variant): a graph of many small
-// independent launches runs them a few at a time (the hardware queues),
-// each with its own tail.
+// Every op that runs one work-group per tile (row x column tiles on the
+// lane-fixed walk, row copies) goes into ONE launch over all types
+// (ttc_batch_one.hpp): the work table holds a record per op, the first tile
+// of each, and the op each block of 64 tiles starts in.
+//
+// The others (box tiles, tiles the lane-fixed walk does not take, ops that
+// ask for lds_buffers) run in one persistent launch per (family, type pair):
+// a record per op and per tile (origin offsets, partial-tile limits), ops
+// ordered by variant (vector widths, beta read or not), and a split of the
+// group's tile range into one contiguous slice per work-group, balanced by
+// bytes moved.  A work-group rebuilds its LDS offset tables when its slice
+// crosses into the next row x column op.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,6 +25,7 @@
 #include <vector>
 
 #include "ttc_batch_kernels.hpp"
+#include "ttc_batch_one.hpp"
 #include "ttc_launch.hpp"
 #include "ttc_plan.h"
 #include "ttc_runtime.h"
@@ -54,9 +53,8 @@ static void fill_bases(const TileParams& p, TileBase* out) {
 }
 
 // Kernel of group key = family * kBPairs + pair (family 0 box tiles, 1 row
-// x column tiles, 2 row copies).
-enum GroupFamily { kGroupBox = 0, kGroupRC = 1, kGroupRow = 2 };
-static int group_of(int kind) { return kind / kVariantStride; }
+// x column tiles).
+enum GroupFamily { kGroupBox = 0, kGroupRC = 1 };
 static int group_family(int group) { return group / kBPairs; }
 
 static const BatchKernelSet& pair_kernels(int pair) {
@@ -66,11 +64,7 @@ static const BatchKernelSet& pair_kernels(int pair) {
 }
 static const void* group_kernel(int group) {
   const BatchKernelSet& k = pair_kernels(group % kBPairs);
-  switch (group_family(group)) {
-    case kGroupRC: return k.rc;
-    case kGroupRow: return k.row;
-    default: return k.box;
-  }
+  return group_family(group) == kGroupRC ? k.rc : k.box;
 }
 
 static int batch_pair(int ta, int tb) {
@@ -105,10 +99,12 @@ struct BatchGroup {
 // op records point at their tile records once the image's device address is
 // known (render).
 struct BatchImage {
-  enum { kBox, kRC, kRow, kWg, kBases, kRcTiles, kRcTables, kSections };
+  enum { kOne, kOneBegin, kOneBlocks, kBox, kRC, kWg, kBases, kRcTiles, kRcTables, kSections };
+  std::vector<BatchOneOp> one;          // ops of the one-work-group-per-tile launch
+  std::vector<uint32_t> one_begin;      // first tile of each
+  std::vector<uint32_t> one_block;      // the op each block of kOneBlock tiles starts in
   std::vector<BatchOpDev> box;
   std::vector<BatchRCOpDev> rcs;
-  std::vector<BatchRowOpDev> rows;
   std::vector<uint32_t> wg;
   std::vector<TileBase> bases;
   std::vector<RCTile> rct;
@@ -119,8 +115,9 @@ struct BatchImage {
   size_t bytes = 0;
 
   void layout() {
-    const size_t len[kSections] = {sizeof(BatchOpDev) * box.size(),   sizeof(BatchRCOpDev) * rcs.size(),
-                                   sizeof(BatchRowOpDev) * rows.size(), sizeof(uint32_t) * wg.size(),
+    const size_t len[kSections] = {sizeof(BatchOneOp) * one.size(),     sizeof(uint32_t) * one_begin.size(),
+                                   sizeof(uint32_t) * one_block.size(), sizeof(BatchOpDev) * box.size(),
+                                   sizeof(BatchRCOpDev) * rcs.size(),   sizeof(uint32_t) * wg.size(),
                                    sizeof(TileBase) * bases.size(),     sizeof(RCTile) * rct.size(),
                                    sizeof(int32_t) * rtab.size()};
     size_t o = 0;
@@ -145,9 +142,11 @@ struct BatchImage {
     auto put = [&](int s, const void* src, size_t n) {
       if (n) std::memcpy(out.data() + off[s], src, n);
     };
+    put(kOne, one.data(), sizeof(BatchOneOp) * one.size());
+    put(kOneBegin, one_begin.data(), sizeof(uint32_t) * one_begin.size());
+    put(kOneBlocks, one_block.data(), sizeof(uint32_t) * one_block.size());
     put(kBox, b2.data(), sizeof(BatchOpDev) * b2.size());
     put(kRC, r2.data(), sizeof(BatchRCOpDev) * r2.size());
-    put(kRow, rows.data(), sizeof(BatchRowOpDev) * rows.size());
     put(kWg, wg.data(), sizeof(uint32_t) * wg.size());
     put(kBases, bases.data(), sizeof(TileBase) * bases.size());
     put(kRcTiles, rct.data(), sizeof(RCTile) * rct.size());
@@ -160,6 +159,8 @@ struct BatchPlan {
   std::vector<ttc_plan_t> plans;  // per-op plans (also used by the per-op loop)
   std::vector<ttc_batch_op_t> ops;
   std::vector<BatchGroup> groups;
+  uint32_t one_tiles = 0;  // tiles of the one-work-group-per-tile launch
+  int one_lds = 0;
   BatchImage img;
   int nwg_total = 0;
   int64_t tiles = 0, bytes = 0;
@@ -206,6 +207,11 @@ static void fill_rc_tiles(const RCParams& p, RCTile* out) {
   }
 }
 
+// Kinds from here on are those of the grouped launches whose work-groups walk
+// several tiles: kGroupKind + group * kVariantStride + variant; below it
+// those of the one-work-group-per-tile launch (ttc_batch_one.hpp).
+constexpr int kGroupKind = kBPairs * kOneVariants;
+
 // One op of the work table while it is built.
 struct OpRec {
   int kind;
@@ -243,6 +249,10 @@ static std::vector<uint32_t> split_by_bytes(const std::vector<OpRec>& h, int op0
   return wgb;
 }
 
+// Work-groups of the one-work-group-per-tile launch (HIP counts a grid's
+// threads in 32 bits; past that each walks several tiles).
+static unsigned one_grid(uint32_t tiles) { return std::min<uint32_t>(tiles, 1u << 23); }
+
 constexpr int kBatchSlicesPerCu = 96;  // default work-group slices per CU in a group's grid
 
 // Plans every op and builds the work table on the host (no device memory).
@@ -262,20 +272,52 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       any_lda |= op.lda[k] != 0;
       any_ldb |= op.ldb[k] != 0;
     }
+    const int* lda = any_lda ? op.lda : nullptr;
+    const int* ldb = any_ldb ? op.ldb : nullptr;
+    const int wide = pair_kernels(pair).widest;
+    OpRec& r = rec[i];
+    r.src = i;
+    const int64_t sa = dtype_bytes(op.type_a), sb = dtype_bytes(op.type_b);
+    // one work-group per tile, where the op's plan takes such a launch
+    {
+      ttc_plan_t pl = nullptr;
+      ttc_status_t st = plan_create(&pl, op.type_a, op.type_b, op.dim, op.perm, op.size, lda, ldb, op.beta_is_zero,
+                                    &op.cfg, kPlanGroupTile);
+      if (st != TTC_SUCCESS) return st;
+      bp.plans[i] = pl;
+      if (pl->g.elements > 0 && (!op.A || !op.B)) return TTC_ERROR_INVALID_VALUE;
+      const ttc_plan_s* use = pl->g.elements > 0 ? variant_for(pl, op.A, op.B) : pl;
+      if (!use) return TTC_ERROR_INVALID_VALUE;
+      const int bz = pl->beta_is_zero ? 1 : 0;
+      int variant = -1;
+      if (use->family == kFamilyRC && use->lane_div == 2)
+        variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
+      else if (use->family == kFamilyRow && use->row1_unaligned)
+        variant = kOneRowUnaligned + __builtin_ctz((unsigned)use->row1_v) * 2 + bz;
+      else if (use->family == kFamilyRow)
+        variant = kOneRow + index_of_width(use->row1_v, wide) * 2 + bz;
+      if (variant >= 0) {
+        r.kind = pair * kOneVariants + variant;
+        r.ntiles = pl->g.elements == 0 ? 0 : (use->family == kFamilyRC ? use->lane.walk.ntiles : use->row1_grid);
+        r.weight = 0.0;
+        bp.bytes += pl->g.elements * (sa + sb * (bz ? 1 : 2));
+        continue;
+      }
+      bp.plans[i] = nullptr;
+      ttc_plan_destroy(pl);
+    }
     // vector widths the group kernels instantiate: 1, 2 and the widest on
-    // row x column tiles and row copies, 1 and the widest on box tiles
+    // row x column tiles, 1 and the widest on box tiles
     ttc_config_t cfg = op.cfg;
     if (cfg.tile_order > 2) cfg.tile_order = 2;  // grouped launches walk host-built tile records in B order
     if (cfg.lds_buffers == 0) cfg.lds_buffers = 1;  // one LDS buffer unless the op asks for two (measured faster)
-    const int wide = pair_kernels(pair).widest;
     auto width_ok = [wide](const ttc_plan_s* q, int v) {
       return v == 1 || v == wide || (v == 2 && wide > 2 && q->family != kFamilyBox);
     };
     for (int pass = 0; pass < 2; ++pass) {
       ttc_plan_t pl = nullptr;
-      ttc_status_t st = plan_create(&pl, op.type_a, op.type_b, op.dim, op.perm, op.size,
-                                    any_lda ? op.lda : nullptr, any_ldb ? op.ldb : nullptr, op.beta_is_zero, &cfg,
-                                    true);
+      ttc_status_t st = plan_create(&pl, op.type_a, op.type_b, op.dim, op.perm, op.size, lda, ldb, op.beta_is_zero,
+                                    &cfg, kPlanGroupWalk);
       if (st != TTC_SUCCESS) return st;
       const bool ok_a = width_ok(pl, pl->va), ok_b = width_ok(pl, pl->vb);
       if ((ok_a && ok_b) || pass == 1) {
@@ -289,20 +331,14 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
     }
     const ttc_plan_s* pl = bp.plans[i];
     if (!width_ok(pl, pl->va) || !width_ok(pl, pl->vb)) return TTC_ERROR_UNSUPPORTED;
-    if (pl->g.elements > 0 && (!op.A || !op.B)) return TTC_ERROR_INVALID_VALUE;
     const ttc_plan_s* use = pl->g.elements > 0 ? variant_for(pl, op.A, op.B) : pl;
     if (!use) return TTC_ERROR_INVALID_VALUE;
-    if (!width_ok(use, use->va) || !width_ok(use, use->vb)) return TTC_ERROR_UNSUPPORTED;
-    const int fam = use->family == kFamilyRC ? kGroupRC : (use->family == kFamilyRow ? kGroupRow : kGroupBox);
+    if (!width_ok(use, use->va) || !width_ok(use, use->vb) || use->family == kFamilyRow) return TTC_ERROR_UNSUPPORTED;
+    const int fam = use->family == kFamilyRC ? kGroupRC : kGroupBox;
     const int bz = pl->beta_is_zero ? 1 : 0;
-    const int ia = index_of_width(use->va, wide), ib = index_of_width(use->vb, wide);
-    OpRec& r = rec[i];
-    // a row copy has one width for both sides
-    const int variant = fam == kGroupRow ? ia * 2 + bz : (ia * 3 + ib) * 2 + bz;
-    r.kind = (fam * kBPairs + pair) * kVariantStride + variant;
+    const int variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
+    r.kind = kGroupKind + (fam * kBPairs + pair) * kVariantStride + variant;
     r.ntiles = pl->g.elements > 0 ? use->p.ntiles : 0;
-    r.src = i;
-    const int64_t sa = dtype_bytes(op.type_a), sb = dtype_bytes(op.type_b);
     r.weight = r.ntiles ? (double)pl->g.elements * (double)(sa + sb * (pl->beta_is_zero ? 1 : 2)) / r.ntiles : 0.0;
     bp.bytes += pl->g.elements * (sa + sb * (pl->beta_is_zero ? 1 : 2));
   }
@@ -313,14 +349,45 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
   const int cus = device_cus(dev);
   BatchImage& im = bp.img;
   bp.tiles = 0;
-  for (int j = 0; j < nops;) {
+  int j = 0;
+  uint64_t one_tiles = 0;
+  for (; j < nops && rec[j].kind < kGroupKind; ++j) {
+    const OpRec& r = rec[j];
+    if (r.ntiles == 0) continue;
+    const ttc_batch_op_t& op = ops[r.src];
+    const ttc_plan_s* use = variant_for(bp.plans[r.src], op.A, op.B);
+    BatchOneOp d;
+    std::memset(&d, 0, sizeof(d));
+    if (use->family == kFamilyRC) {
+      std::memcpy(&d.p, &use->lane, sizeof(use->lane));
+      d.p.lane.walk.grid_order = 0;  // the launch deals the tiles of all ops out to the XCDs
+      bp.one_lds = std::max(bp.one_lds, use->lane_lds);
+    } else {
+      std::memcpy(&d.p, &use->row1, sizeof(use->row1));
+    }
+    d.A = op.A;
+    d.B = op.B;
+    d.alpha = op.alpha;
+    d.beta = op.beta;
+    d.kind = r.kind;
+    const uint32_t first = (uint32_t)one_tiles;
+    one_tiles += r.ntiles;
+    if (one_tiles >= (1ull << 31)) return TTC_ERROR_UNSUPPORTED;
+    while ((uint64_t)im.one_block.size() * kOneBlock < one_tiles) im.one_block.push_back((uint32_t)im.one.size());
+    im.one.push_back(d);
+    im.one_begin.push_back(first);
+  }
+  bp.one_tiles = (uint32_t)one_tiles;
+  bp.tiles += (int64_t)one_tiles;
+  auto group_of = [](int kind) { return (kind - kGroupKind) / kVariantStride; };
+  while (j < nops) {
     int e = j;
     uint64_t tiles = 0;
     int lds = 16;
     const int group = group_of(rec[j].kind);
     const int family = group_family(group);
     const bool rc = family == kGroupRC;
-    const size_t op0 = rc ? im.rcs.size() : (family == kGroupRow ? im.rows.size() : im.box.size());
+    const size_t op0 = rc ? im.rcs.size() : im.box.size();
     while (e < nops && group_of(rec[e].kind) == group) {
       OpRec& r = rec[e];
       r.tile_begin = (uint32_t)tiles;
@@ -329,19 +396,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       const ttc_plan_s* pl = bp.plans[r.src];
       const ttc_plan_s* use = pl->g.elements > 0 ? variant_for(pl, op.A, op.B) : pl;
       lds = std::max(lds, use->lds_bytes);
-      if (family == kGroupRow) {
-        BatchRowOpDev d;
-        std::memset(&d, 0, sizeof(d));
-        d.p = use->row;
-        d.A = op.A;
-        d.B = op.B;
-        d.alpha = op.alpha;
-        d.beta = op.beta;
-        d.variant = r.kind % kVariantStride;
-        d.tile_begin = r.tile_begin;
-        d.ntiles = r.ntiles;  // chunks of kThreads * kRowUnroll vectors
-        im.rows.push_back(d);
-      } else if (rc) {
+      if (rc) {
         BatchRCOpDev d;
         std::memset(&d, 0, sizeof(d));
         d.p = use->rc;
@@ -357,7 +412,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
         d.B = op.B;
         d.alpha = op.alpha;
         d.beta = op.beta;
-        d.variant = r.kind % kVariantStride;
+        d.variant = (r.kind - kGroupKind) % kVariantStride;
         d.tile_begin = r.tile_begin;
         d.ntiles = r.ntiles;
         const size_t first = im.rct.size();
@@ -377,7 +432,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
         d.B = op.B;
         d.alpha = op.alpha;
         d.beta = op.beta;
-        d.variant = r.kind % kVariantStride;
+        d.variant = (r.kind - kGroupKind) % kVariantStride;
         d.tile_begin = r.tile_begin;
         d.ntiles = r.ntiles;
         const size_t first = im.bases.size();
@@ -413,6 +468,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
   }
   bp.nwg_total = 0;
   for (const BatchGroup& g : bp.groups) bp.nwg_total += g.nwg;
+  bp.nwg_total += (int)one_grid(bp.one_tiles);
   im.layout();
   return TTC_SUCCESS;
 }
@@ -426,23 +482,40 @@ struct GroupArgs {
 static GroupArgs group_args(const BatchPlan& bp, const BatchGroup& g, uintptr_t base) {
   const BatchImage& im = bp.img;
   GroupArgs a;
-  switch (group_family(g.group)) {
-    case kGroupRC:
-      a.ops = reinterpret_cast<const void*>(base + im.off[BatchImage::kRC] + g.op0 * sizeof(BatchRCOpDev));
-      break;
-    case kGroupRow:
-      a.ops = reinterpret_cast<const void*>(base + im.off[BatchImage::kRow] + g.op0 * sizeof(BatchRowOpDev));
-      break;
-    default:
-      a.ops = reinterpret_cast<const void*>(base + im.off[BatchImage::kBox] + g.op0 * sizeof(BatchOpDev));
-      break;
-  }
+  a.ops = group_family(g.group) == kGroupRC
+              ? reinterpret_cast<const void*>(base + im.off[BatchImage::kRC] + g.op0 * sizeof(BatchRCOpDev))
+              : reinterpret_cast<const void*>(base + im.off[BatchImage::kBox] + g.op0 * sizeof(BatchOpDev));
   a.nops = g.nops;
   a.wg = reinterpret_cast<const uint32_t*>(base + im.off[BatchImage::kWg] + g.wg0 * sizeof(uint32_t));
   return a;
 }
 
+// Arguments of the one-work-group-per-tile launch.
+struct OneArgs {
+  const void* ops;
+  const void* begin;
+  const void* block;
+  uint32_t nops, ntiles;
+};
+static OneArgs one_args(const BatchPlan& bp, uintptr_t base) {
+  const BatchImage& im = bp.img;
+  OneArgs a;
+  a.ops = reinterpret_cast<const void*>(base + im.off[BatchImage::kOne]);
+  a.begin = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneBegin]);
+  a.block = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneBlocks]);
+  a.nops = (uint32_t)im.one.size();
+  a.ntiles = bp.one_tiles;
+  return a;
+}
+
 static ttc_status_t launch_groups(const BatchPlan& bp, uintptr_t base, hipStream_t s) {
+  if (bp.one_tiles > 0) {
+    OneArgs a = one_args(bp, base);
+    void* args[] = {&a.ops, &a.begin, &a.block, &a.nops, &a.ntiles};
+    if (hipLaunchKernel(batch_one_func(), dim3(one_grid(bp.one_tiles)), dim3(kThreads), args, (size_t)bp.one_lds,
+                        s) != hipSuccess)
+      return TTC_ERROR_HIP;
+  }
   for (const BatchGroup& g : bp.groups) {
     GroupArgs a = group_args(bp, g, base);
     void* args[] = {&a.ops, &a.nops, &a.wg};
@@ -515,6 +588,22 @@ extern "C" ttc_status_t ttc_batch_graph_launch(ttc_batch_t b, ttc_stream_t strea
       // the grouped launch: one kernel node per kind, no edges between them
       // (they touch disjoint ops), so the graph may run kinds side by side
       if (hipGraphCreate(&g, 0) != hipSuccess) return TTC_ERROR_HIP;
+      if (b->bp.one_tiles > 0) {
+        OneArgs a = one_args(b->bp, reinterpret_cast<uintptr_t>(b->d_image));
+        void* args[] = {&a.ops, &a.begin, &a.block, &a.nops, &a.ntiles};
+        hipKernelNodeParams kp;
+        std::memset(&kp, 0, sizeof(kp));
+        kp.func = const_cast<void*>(batch_one_func());
+        kp.gridDim = dim3(one_grid(b->bp.one_tiles));
+        kp.blockDim = dim3(kThreads);
+        kp.sharedMemBytes = (unsigned)b->bp.one_lds;
+        kp.kernelParams = args;
+        hipGraphNode_t node;
+        if (hipGraphAddKernelNode(&node, g, nullptr, 0, &kp) != hipSuccess) {
+          (void)hipGraphDestroy(g);
+          return TTC_ERROR_HIP;
+        }
+      }
       for (const BatchGroup& gr : b->bp.groups) {
         GroupArgs a = group_args(b->bp, gr, reinterpret_cast<uintptr_t>(b->d_image));
         void* args[] = {&a.ops, &a.nops, &a.wg};
@@ -590,7 +679,7 @@ extern "C" ttc_status_t ttc_batch_execute_noalloc(int nops, const ttc_batch_op_t
   ttc_status_t st = plan_batch(nops, ops, wg_per_cu, bp);
   if (st != TTC_SUCCESS) return st;
   if (bp.img.bytes > (size_t)TTC_BATCH_WORKSPACE_BYTES) return TTC_ERROR_WORKSPACE;
-  if (bp.groups.empty()) return TTC_SUCCESS;  // every op is empty
+  if (bp.groups.empty() && bp.one_tiles == 0) return TTC_SUCCESS;  // every op is empty
   void* base = nullptr;
   st = scratch_address(&base);
   if (st != TTC_SUCCESS) return st;

@@ -1,0 +1,37 @@
+// Grouped launch of one work-group per tile: the kernel over all types.
+#include "ttc_batch_one.hpp"
+
+namespace ttc {
+
+using KIdx = const __attribute__((address_space(4))) uint32_t;
+
+__global__ void __launch_bounds__(kThreads)
+    batch_one_kernel(const BatchOneOp* __restrict__ ops, const uint32_t* __restrict__ begin,
+                     const uint32_t* __restrict__ block, uint32_t nops, uint32_t ntiles) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  KIdx* kbegin = (KIdx*)begin;
+  KIdx* kblock = (KIdx*)block;
+  for (uint32_t w = blockIdx.x; w < ntiles; w += gridDim.x) {
+    if (w != blockIdx.x) __syncthreads();  // the previous tile's LDS reads
+    const uint32_t id = uniform(one_tile_of(w, ntiles));
+    uint32_t op = uniform(kblock[id / kOneBlock]);
+    while (op + 1 < nops && kbegin[op + 1] <= id) ++op;
+    op = uniform(op);
+    KOneOp* o = (KOneOp*)ops + op;
+    const uint32_t tile = id - kbegin[op];
+    const int kind = o->kind, variant = kind % kOneVariants;
+    switch (kind / kOneVariants) {
+      case kBS: one_type<OpF32<float, float>, 4>(variant, o, tile, lds_raw); break;
+      case kBD: one_type<OpDD, 2>(variant, o, tile, lds_raw); break;
+      case kBBF16: one_type<OpF32<bf16s, bf16s>, 8>(variant, o, tile, lds_raw); break;
+      case kBF16: one_type<OpF32<f16s, f16s>, 8>(variant, o, tile, lds_raw); break;
+      case kBC: one_type<OpCC, 2>(variant, o, tile, lds_raw); break;
+      case kBZ: one_type<OpZZ, 1>(variant, o, tile, lds_raw); break;
+      default: break;
+    }
+  }
+}
+
+const void* batch_one_func() { return reinterpret_cast<const void*>(&batch_one_kernel); }
+
+}  // namespace ttc

@@ -1,5 +1,5 @@
-// Device side of the grouped batch: the work-table records and the three
-// persistent group kernels (box tiles, row x column tiles, row copies).
+// Device side of the grouped batch: the work-table records and the two
+// persistent group kernels (box tiles, row x column tiles).
 // The kernels of each type pair are instantiated in a file of their own
 // (ttc_batch_k_<pair>.hip), so that the six pairs compile in parallel; the
 // host side (ttc_batch.hip) reaches them through batch_kernels(pair).
@@ -10,7 +10,6 @@
 
 #include "ttc_kernels.hpp"
 #include "ttc_rc.hpp"
-#include "ttc_row.hpp"
 
 namespace ttc {
 
@@ -23,7 +22,6 @@ enum BatchPair : int { kBS = 0, kBD = 1, kBBF16 = 2, kBF16 = 3, kBC = 4, kBZ = 5
 // class.  A vector width is coded by its index in {1, 2, W} (W = the
 // pair's widest, 16 bytes): the three widths the planner ever picks.
 //   row x column: variant = (index_a * 3 + index_b) * 2 + beta_is_zero  (18)
-//   row copy:     variant = index * 2 + beta_is_zero                    (6)
 //   box tiles:    variant = (index_a * 3 + index_b) * 2 + beta_is_zero,
 //                 widths 1 and W only (index 1 is never used)
 // kind = (family * kBPairs + pair) * kVariantStride + variant.
@@ -63,21 +61,6 @@ struct BatchRCOpDev {
   const int32_t* tables;  // its LDS offset tables (rc_fill_tables: RCParams::ntab entries)
 };
 
-// Op record of a row-copy group (perm[0] == 0 after fusion, dimension 0
-// contiguous on both sides): rows move without LDS staging, as in the
-// single-op row kernel.  Its work unit is a chunk of kThreads * kRowUnroll
-// vectors of the op's row walk.
-struct BatchRowOpDev {
-  RowParams p;
-  const void* A;
-  void* B;
-  double alpha, beta;
-  int32_t variant;
-  int32_t pad_;
-  uint32_t tile_begin;  // first chunk of this op in its group
-  uint32_t ntiles;      // chunks
-};
-
 // Parameter records are copied out of the work table whole, one 32-bit word
 // at a time, so that no field can be left behind when a field is added (a
 // field-by-field copy once missed one, and a kernel then read an
@@ -86,11 +69,8 @@ static_assert(sizeof(TileParams) % 4 == 0 && std::is_trivially_copyable<TilePara
               "TileParams is copied as 32-bit words");
 static_assert(sizeof(RCParams) % 4 == 0 && std::is_trivially_copyable<RCParams>::value,
               "RCParams is copied as 32-bit words");
-static_assert(sizeof(RowParams) % 4 == 0 && std::is_trivially_copyable<RowParams>::value,
-              "RowParams is copied as 32-bit words");
 
 using KRCOp = const __attribute__((address_space(4))) BatchRCOpDev;
-using KRowOp = const __attribute__((address_space(4))) BatchRowOpDev;
 using KWord = const __attribute__((address_space(4))) uint32_t;
 
 __device__ __forceinline__ int32_t uni(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
@@ -224,121 +204,19 @@ __global__ void __launch_bounds__(kRcThreads) batch_rc_kernel(const BatchRCOpDev
   }
 }
 
-// ------------------------------------------------------------ row copies
-
-// Chunks [lo, hi) of one row op: lane l of chunk c moves vectors
-// c * kThreads * U + u * kThreads + l (u < U) of the op's walk (rows of
-// dimension 0 in B order, V elements per vector).
-template <class OP, int V, bool BETA>
-__device__ __forceinline__ void row_op_slice(KRowOp& o, uint32_t lo, uint32_t hi) {
-  using TA = typename OP::TA;
-  using TB = typename OP::TB;
-  constexpr int U = kRowUnroll;
-  RowParams p;
-  {
-    KWord* s = (KWord*)&o.p;
-    uint32_t* d = reinterpret_cast<uint32_t*>(&p);
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(RowParams) / 4); ++i) d[i] = s[i];
-  }
-  const typename OP::AL al = (typename OP::AL)o.alpha;
-  const typename OP::BE be = (typename OP::BE)o.beta;
-  const char* a = static_cast<const char*>(o.A);
-  char* b = static_cast<char*>(o.B);
-  for (uint32_t c = lo; c < hi; ++c) {
-    const uint32_t g0 = c * (uint32_t)(kThreads * U) + threadIdx.x;
-    int64_t ob[U];
-    bool ok[U];
-    TA va[U][V];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t g = g0 + (uint32_t)(u * kThreads);
-      ok[u] = g < p.total;
-      const uint32_t gg = ok[u] ? g : 0u;
-      const uint32_t row = fdiv(gg, p.dnv);
-      const uint32_t v = gg - row * p.nv;
-      int64_t xa = (int64_t)v * (int64_t)(V * sizeof(TA));
-      int64_t xb = (int64_t)v * (int64_t)(V * sizeof(TB));
-      uint32_t rem = row;
-#pragma unroll
-      for (int k = 0; k < kMaxDim; ++k) {
-        if (k < p.rank) {
-          const uint32_t q = fdiv(rem, p.dn[k]);
-          const uint32_t x = rem - q * p.dn[k].d;
-          rem = q;
-          xa += (int64_t)x * p.sa[k];
-          xb += (int64_t)x * p.sb[k];
-        }
-      }
-      ob[u] = xb;
-      if (ok[u]) vload<TA, V>(va[u], reinterpret_cast<const TA*>(a + xa));
-    }
-    TB old[U][V];
-    if constexpr (BETA) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (ok[u]) vload<TB, V>(old[u], reinterpret_cast<const TB*>(b + ob[u]));
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (!ok[u]) continue;
-      TB out[V];
-#pragma unroll
-      for (int v = 0; v < V; ++v) {
-        if constexpr (BETA) out[v] = OP::outb(OP::prod(al, va[u][v]), be, old[u][v]);
-        else out[v] = OP::out(OP::prod(al, va[u][v]));
-      }
-      vstore<TB, V, false>(reinterpret_cast<TB*>(b + ob[u]), out);
-    }
-  }
-}
-
-template <class OP, int W, int I = 0>
-__device__ __forceinline__ void row_dispatch(int v, KRowOp& o, uint32_t lo, uint32_t hi) {
-  if constexpr (I < 6) {
-    if constexpr (index_used(I / 2, W)) {
-      if (v == I) {
-        row_op_slice<OP, width_of_index(I / 2, W), (I & 1) == 0>(o, lo, hi);
-        return;
-      }
-    }
-    row_dispatch<OP, W, I + 1>(v, o, lo, hi);
-  }
-}
-
-template <class OP, int W>
-__global__ void __launch_bounds__(kThreads) batch_row_kernel(const BatchRowOpDev* __restrict__ ops, int nops,
-                                                             const uint32_t* __restrict__ wg_begin) {
-  const uint32_t t0 = wg_begin[blockIdx.x], t1 = wg_begin[blockIdx.x + 1];
-  if (t0 >= t1) return;
-  KRowOp* kops = (KRowOp*)ops;
-  uint32_t t = t0;
-  for (int op = first_op(ops, nops, t0); op < nops && t < t1; ++op) {
-    KRowOp& o = kops[op];
-    const uint32_t end = o.tile_begin + o.ntiles;
-    const uint32_t stop = end < t1 ? end : t1;
-    if (t < stop) {
-      row_dispatch<OP, W>(o.variant, o, t - o.tile_begin, stop - o.tile_begin);
-      t = stop;
-    }
-  }
-}
-
 // ------------------------------------------------------------- registry
 
-// The three group kernels of one type pair, W its widest vector width.
+// The two group kernels of one type pair, W its widest vector width.
 struct BatchKernelSet {
   const void* box;
   const void* rc;
-  const void* row;
   int widest;
 };
 
 template <class OP, int W>
 BatchKernelSet batch_kernel_set() {
   return BatchKernelSet{reinterpret_cast<const void*>(&batch_box_kernel<OP, W>),
-                        reinterpret_cast<const void*>(&batch_rc_kernel<OP, W>),
-                        reinterpret_cast<const void*>(&batch_row_kernel<OP, W>), W};
+                        reinterpret_cast<const void*>(&batch_rc_kernel<OP, W>), W};
 }
 
 // Defined one per file, ttc_batch_k_<pair>.hip.

@@ -51,10 +51,11 @@ struct RCLane {
     }
   }
 
-  // One tile; returns max |alpha * a| of this lane's elements (fp8 casts).
-  // after(amax): called between staging and the barrier.
+  // The tile of work-group `wg` of the launch (of the op, in a grouped one).
+  // after(amax): called between staging and the barrier with max |alpha * a|
+  // of this lane's elements (fp8 casts).
   template <class F>
-  __device__ __forceinline__ static void run(KLane* kp, const TA* __restrict__ A, TB* __restrict__ B,
+  __device__ __forceinline__ static void run(KLane* kp, uint32_t wg, const TA* __restrict__ A, TB* __restrict__ B,
                                              unsigned char* lds_raw, typename OP::AL alpha, typename OP::BE beta,
                                              F&& after) {
     const uint32_t tid = threadIdx.x;
@@ -71,7 +72,7 @@ struct RCLane {
       w.dband = FastDiv{kp->walk.dband.d, kp->walk.dband.m, kp->walk.dband.s, 0};
       w.dw = FastDiv{kp->walk.dw.d, kp->walk.dw.m, kp->walk.dw.s, 0};
       w.dwl = FastDiv{kp->walk.dwl.d, kp->walk.dwl.m, kp->walk.dwl.s, 0};
-      rem = uniform(rc_tile_of(w, blockIdx.x));
+      rem = uniform(rc_tile_of(w, wg));
     }
     int64_t bA = 0, bB = 0;
     uint32_t last = 0;
@@ -173,7 +174,7 @@ __global__ void __launch_bounds__(kRcThreads)
                           typename OP::TB* __restrict__ B, double alpha, double beta) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   KLane* kp = (KLane*)__builtin_amdgcn_kernarg_segment_ptr();
-  RCLane<OP, VA, VB, BETA, NT, DIV>::run(kp, A, B, lds_raw, (typename OP::AL)alpha, (typename OP::BE)beta,
+  RCLane<OP, VA, VB, BETA, NT, DIV>::run(kp, blockIdx.x, A, B, lds_raw, (typename OP::AL)alpha, (typename OP::BE)beta,
                                          [](float) {});
 }
 
@@ -201,7 +202,7 @@ __global__ void __launch_bounds__(kRcThreads)
   unsigned int* const am = reinterpret_cast<unsigned int*>(amax_out);
   unsigned int seen = 0;
   if (am && threadIdx.x == 0) seen = __hip_atomic_load(am, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  RCLane<OP, VA, VB, false, false, DIV>::run(kp, A, B, lds_raw, alpha, scale, [&](float m) {
+  RCLane<OP, VA, VB, false, false, DIV>::run(kp, blockIdx.x, A, B, lds_raw, alpha, scale, [&](float m) {
     if (!am) return;
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));

@@ -955,7 +955,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
   pl->row1_v = v;
   pl->row1_unaligned = 0;
   pl->row1_grid = 0;
-  if (pl->row.total == 0 || pl->wg_per_cu > 0) return;
+  if (pl->row.total == 0 || (pl->wg_per_cu > 0 && pl->min_div == 1)) return;
   const bool may = !pl->vec_given && row_unaligned_mode(szA, szB, !pl->beta_is_zero, pl->nt_store != 0);
   const int w = may ? row_unaligned_width(szA, szB, n0) : 1;
   if (w > v) {
@@ -1043,7 +1043,7 @@ static double lane_cost(const Geometry& g, const int* tile, int szA, int szB, in
 // sides, tiles covering short leading extents whole, and of each that the
 // walk does not fit, the largest that fits along a group's outermost
 // dimension; the cheapest by lane_cost.
-bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile) {
+bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile, int min_div) {
   if (g.elements == 0 || g.rank < 2 || g.perm[0] == 0) return false;
   const int szA = dtype_bytes(ta), szB = dtype_bytes(tb), vmax = max_rc_volume(ta, tb);
   double best = -1.0;
@@ -1065,7 +1065,7 @@ bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool be
   };
   auto consider = [&](const int* c) {
     LaneFit f;
-    for (int div = 2; div >= 1; --div) {
+    for (int div = 2; div >= min_div; --div) {
       if (!lane_fit(g, c, szA, szB, va, vb, div, f)) continue;
       const double cost = lane_cost(g, c, szA, szB, va, vb, div, beta, f);
       // (the plan keeps the family's parameters too, within its LDS budget)
@@ -1098,8 +1098,8 @@ bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool be
       consider(c);
       c[k] = keep;
     };
-    shrink(gb[nb - 1], R, C, va, vb, rc_elems(szA) / va);
-    shrink(ga[na - 1], C, R, vb, va, rc_elems(szB) / vb);
+    shrink(gb[nb - 1], R, C, va, vb, rc_elems(szA) / va / min_div);
+    shrink(ga[na - 1], C, R, vb, va, rc_elems(szB) / vb / min_div);
   };
   for (int ra = 1; ra <= vmax; ra *= 2)
     for (int rb = 1; rb <= vmax; rb *= 2) {
@@ -1243,7 +1243,7 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     int rc_tile[kMaxDim];
     double rc_score = -1.0;
     const bool lane = fam != kFamilyBox && pl->one_tile && run_a == 0 && run_b == 0 &&
-                      choose_lane_tile(g, pl->type_a, pl->type_b, va, vb, !pl->beta_is_zero, rc_tile);
+                      choose_lane_tile(g, pl->type_a, pl->type_b, va, vb, !pl->beta_is_zero, rc_tile, pl->min_div);
     // (a caller that names the family is refused the shapes choose_rc_tile refuses)
     if (lane && fam == kFamilyRC) {
       int t[kMaxDim];
@@ -1284,7 +1284,7 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     // work-groups or LDS buffers, which only the pipelined kernel has
     pl->lane_div = 0;
     if (pl->one_tile && st == TTC_SUCCESS)
-      for (int div = 2; div >= 1 && pl->lane_div == 0; --div)
+      for (int div = 2; div >= pl->min_div && pl->lane_div == 0; --div)
         if (build_lane_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->tile_order, div, pl->lane,
                               pl->lane_lds))
           pl->lane_div = div;
@@ -1303,12 +1303,12 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
 extern "C" ttc_status_t ttc_plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim,
                                         const int* perm, const int* size, const int* lda, const int* ldb,
                                         int beta_is_zero, const ttc_config_t* cfg) {
-  return plan_create(plan, type_a, type_b, dim, perm, size, lda, ldb, beta_is_zero, cfg, false);
+  return plan_create(plan, type_a, type_b, dim, perm, size, lda, ldb, beta_is_zero, cfg, kPlanSingle);
 }
 
 ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim, const int* perm,
                               const int* size, const int* lda, const int* ldb, int beta_is_zero,
-                              const ttc_config_t* cfg, bool grouped) {
+                              const ttc_config_t* cfg, PlanUse use) {
   if (!plan) return TTC_ERROR_INVALID_VALUE;
   *plan = nullptr;
   if (!pair_supported(type_a, type_b)) return TTC_ERROR_UNSUPPORTED;
@@ -1347,7 +1347,10 @@ ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t 
   bool explicit_tile = false;
   for (int k = 0; k < TTC_MAX_DIM; ++k) explicit_tile |= c.tile[k] != 0;
   pl->vec_given = c.vec_a != 0 || c.vec_b != 0;
-  pl->one_tile = !grouped && c.wg_per_cu == 0 && (c.lds_buffers == 0 || !explicit_tile);
+  pl->one_tile = c.wg_per_cu == 0 && (c.lds_buffers == 0 || !explicit_tile);
+  if (use == kPlanGroupTile) pl->one_tile = c.lds_buffers == 0;  // (wg_per_cu does not apply to an op of a group)
+  if (use == kPlanGroupWalk) pl->one_tile = 0;
+  pl->min_div = use == kPlanSingle ? 1 : 2;
   auto in_list = [](int w, int bytes) {
     for (int x : vec_widths(bytes))
       if (x == w) return true;

@@ -116,7 +116,7 @@ bool choose_rc_tile(const Geometry& g, int ta, int tb, int va, int vb, int run_a
 // kernel.  choose_lane_tile: the heuristic tile of such a launch.
 bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int va, int vb, int grid_order,
                        int tile_order, int div, RCLaneParams& p, int& lds_bytes);
-bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile);
+bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile, int min_div = 1);
 // The launch's LDS offset tables (p.ntab entries, the layout of RCParams),
 // as the kernel's setup() builds them.
 void rc_fill_tables(const RCParams& p, int32_t* out);
@@ -125,11 +125,13 @@ void rc_fill_tables(const RCParams& p, int32_t* out);
 // elements; TTC_ERROR_UNSUPPORTED when the shape does not fit the kernel.
 ttc_status_t build_row_params(const Geometry& g, int ta, int tb, int v, RowParams& p);
 
-// ttc_plan_create; grouped: for an op of a grouped launch, whose work-groups
-// walk several tiles each.
+// ttc_plan_create for one op of its own, for an op of the grouped launch of
+// one work-group per tile (whose kernel has the half-size instances only), or
+// for an op of the grouped launches whose work-groups walk several tiles.
+enum PlanUse { kPlanSingle, kPlanGroupTile, kPlanGroupWalk };
 ttc_status_t plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t type_b, int dim, const int* perm,
                          const int* size, const int* lda, const int* ldb, int beta_is_zero, const ttc_config_t* cfg,
-                         bool grouped);
+                         PlanUse use);
 
 }  // namespace ttc
 
@@ -148,6 +150,7 @@ struct ttc_plan_s {
   int tile_order;        // 1 A order, 2 B order, 3 / 4 grouped B order (row x column tiles only)
   int lds_buffers;       // LDS tile buffers of the row x column kernel
   ttc::RCParams rc;
+  int min_div;           // smallest RCLane DIV the launch has: 2 in grouped launches
   int vec_given;         // the caller chose the vector widths
   int one_tile;          // row x column tiles: one tile per work-group where the tile fits (ttc_lane.hpp)
   int lane_div;          // one tile per work-group: 1 / 2 = instance, 0 = the pipelined kernel on rc

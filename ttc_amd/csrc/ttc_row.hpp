@@ -125,12 +125,12 @@ template <class T, int V> struct __attribute__((packed, aligned(sizeof(T)))) Row
 // copy 4740 -> 6010; bf16 128 x 4096 x 32 x 8 perm (0,2,1,3) 4760 -> 5340;
 // fp32 rows of 127 3890 -> 4730, of 5 2210 -> 3040; bf16 rows of 127
 // 2180 -> 4070, of 5 1270 -> 2240.
-template <class OP, int V, int MODE, bool UNAL>
-__global__ void __launch_bounds__(kThreads)
-    row_once_kernel(const RowParams p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
-                    double alpha, double beta, const float* __restrict__ scale_in, const float* __restrict__ amax_in,
-                    float fp8_max, float scale_host, float* __restrict__ amax_out,
-                    float* __restrict__ scale_inv_out) {
+// P: RowParams as a kernel argument or in a grouped launch's work table.
+// Returns max |alpha * a| of this lane's elements (fp8 casts).
+template <class OP, int V, int MODE, bool UNAL, class P>
+__device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typename OP::TA* __restrict__ A,
+                                           typename OP::TB* __restrict__ B, typename OP::AL al, typename OP::BE be,
+                                           float scale) {
   using TA = typename OP::TA;
   using TB = typename OP::TB;
   using L = typename OP::L;
@@ -138,24 +138,6 @@ __global__ void __launch_bounds__(kThreads)
   constexpr bool BETA = MODE == kModeBeta;
   constexpr bool NT = MODE == kModeBzNt;
   constexpr int U = row_once_unroll((int)sizeof(TA), (int)sizeof(TB), V, FP8, UNAL);
-  float scale = 1.0f;
-  if constexpr (FP8) {
-    scale = scale_host;
-    if (scale_in) {
-      scale = *scale_in;
-    } else if (amax_in) {
-      const float m = *amax_in;
-      scale = (m > 0.0f && m <= 3.402823466e38f) ? fp8_max / m : 1.0f;
-    }
-    if (scale_inv_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_inv_out = 1.0f / scale;
-  }
-  const typename OP::AL al = (typename OP::AL)alpha;
-  const typename OP::BE be = (typename OP::BE)beta;
-  uint32_t w = blockIdx.x;
-  if (p.xcd_share) {
-    const uint32_t x = w % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
-    w = x * q + (x < r ? x : r) + w / kXcds;
-  }
   const uint32_t g0 = w * (uint32_t)(kThreads * U) + threadIdx.x;
   const char* a = reinterpret_cast<const char*>(A);
   char* b = reinterpret_cast<char*>(B);
@@ -169,7 +151,7 @@ __global__ void __launch_bounds__(kThreads)
     const uint32_t g = g0 + (uint32_t)(u * kThreads);
     ok[u] = g < p.total;
     const uint32_t gg = ok[u] ? g : 0u;
-    const uint32_t row = fdiv(gg, p.dnv);
+    const uint32_t row = fdiv(gg, p.dnv.m, p.dnv.s);
     int32_t e = (int32_t)(gg - row * p.nv) * V;
     skip[u] = 0;
     if constexpr (UNAL) {
@@ -181,7 +163,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
     for (int k = 0; k < kMaxDim; ++k) {
       if (k < p.rank) {
-        const uint32_t q = fdiv(rem, p.dn[k]);
+        const uint32_t q = fdiv(rem, p.dn[k].m, p.dn[k].s);
         const uint32_t x = rem - q * p.dn[k].d;
         rem = q;
         xa += (int64_t)x * p.sa[k];
@@ -242,6 +224,34 @@ __global__ void __launch_bounds__(kThreads)
       vstore<TB, V, NT>(dst, o);
     }
   }
+  return amax;
+}
+
+template <class OP, int V, int MODE, bool UNAL>
+__global__ void __launch_bounds__(kThreads)
+    row_once_kernel(const RowParams p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
+                    double alpha, double beta, const float* __restrict__ scale_in, const float* __restrict__ amax_in,
+                    float fp8_max, float scale_host, float* __restrict__ amax_out,
+                    float* __restrict__ scale_inv_out) {
+  constexpr bool FP8 = MODE == kModeFp8;
+  float scale = 1.0f;
+  if constexpr (FP8) {
+    scale = scale_host;
+    if (scale_in) {
+      scale = *scale_in;
+    } else if (amax_in) {
+      const float m = *amax_in;
+      scale = (m > 0.0f && m <= 3.402823466e38f) ? fp8_max / m : 1.0f;
+    }
+    if (scale_inv_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_inv_out = 1.0f / scale;
+  }
+  uint32_t w = blockIdx.x;
+  if (p.xcd_share) {
+    const uint32_t x = w % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
+    w = x * q + (x < r ? x : r) + w / kXcds;
+  }
+  const float amax =
+      row_chunk<OP, V, MODE, UNAL>(p, w, A, B, (typename OP::AL)alpha, (typename OP::BE)beta, scale);
   if constexpr (FP8) {
     if (amax_out) block_amax_commit(amax, amax_out);
   }
