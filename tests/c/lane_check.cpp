@@ -75,6 +75,10 @@ static bool check_tile(const RCLaneParams& p, int szA, int szB, int va, int vb, 
   CHECK(p.kA * (long long)p.la <= kRcThreads && p.kB * (long long)p.lb <= kRcThreads, "lanes");
   std::vector<long long> rA(p.R), rB(nB), cB(p.C), cA(nA);  // true offsets, -1: out of range
   std::vector<uint32_t> colS(nA), rowS(nB), rowA(p.R, 0x55555555u), colB(p.C, 0x55555555u);
+  for (long long e = 0; e < std::max(nA, nB); ++e) {
+    if (e < nA) CHECK(fdiv((uint32_t)e, p.kAm, p.kAs) == e / p.kA, "column step division");
+    if (e < nB) CHECK(fdiv((uint32_t)e, p.kBm, p.kBs) == e / p.kB, "row step division");
+  }
   for (long long e = 0; e < nA; ++e) {
     const long long j = e / NIA + (e % NIA) * p.kA;
     long long oa, ob;
@@ -226,6 +230,21 @@ int main(int argc, char** argv) {
     for (int cols : {64, 32})
       if (fits && !check_tile(p, 4, 2, 4, 8, 1, rows, cols, lds, 4)) return 1;
   }
+  // the units of an fp8 cast: every one taken once, in order
+  for (const bool amax : {false, true})
+    for (const uint32_t n : {1u, 2u, 63u, 64u, 65u, 66u, 127u, 255u, 256u, 257u, 258u, 259u, 4096u, 100001u, 0x7fffffffu}) {
+      const AmaxUnits u = amax_units(n, amax);
+      const uint32_t wgs = u.work_groups(), from = wgs > 200000 ? wgs - 1000 : 0;
+      bool ok = u.first(0) == 0 && u.first(wgs) == n;
+      for (uint32_t w = from; w < wgs; ++w) {
+        const uint32_t k = u.first(w + 1) - u.first(w);
+        ok = ok && k >= 1 && k <= (!amax || w < kAmaxHead ? 1u : 2u);
+      }
+      if (!ok) {
+        std::fprintf(stderr, "fp8 units: %u, amax %d\n", n, (int)amax);
+        return 1;
+      }
+    }
   std::printf("lane check: %lld walks, %lld banded, %lld full-size instances, %lld tiles, %lld partial, "
               "%lld with A spans past 2^30: ok\n", walks, banded, full_size, tiles, partial, far);
   return 0;

@@ -71,7 +71,6 @@ static_assert(sizeof(RCParams) % 4 == 0 && std::is_trivially_copyable<RCParams>:
               "RCParams is copied as 32-bit words");
 
 using KRCOp = const __attribute__((address_space(4))) BatchRCOpDev;
-using KWord = const __attribute__((address_space(4))) uint32_t;
 
 __device__ __forceinline__ int32_t uni(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 

@@ -27,7 +27,6 @@
 namespace ttc {
 
 using KLane = const __attribute__((address_space(4))) RCLaneParams;
-
 template <class OP, int VA, int VB, bool BETA, bool NT, int DIV>
 struct RCLane {
   using TA = typename OP::TA;
@@ -59,6 +58,7 @@ struct RCLane {
                                              unsigned char* lds_raw, typename OP::AL alpha, typename OP::BE beta,
                                              F&& after) {
     const uint32_t tid = threadIdx.x;
+    touch_lines<sizeof(RCLaneParams)>(kp);
     // tile origin
     uint32_t rem;
     {
@@ -94,19 +94,31 @@ struct RCLane {
     int32_t* const rowS = colS + kA * NIA;
     int32_t* const rowA = rowS + kB * NIB;
     int32_t* const colB = rowA + R;
-    for (int e = (int)tid; e < kA * NIA; e += kRcThreads) {
-      const int j = e / NIA + (e % NIA) * kA;
-      int32_t oa, ob;
-      offsets(kp, na, kp->nb, (uint32_t)j, oa, ob);
-      colS[e] = j < cols ? oa : (int32_t)kRcTabOOB;
-      if (j < C) colB[j] = j < cols ? ob : (int32_t)kRcTabOOB;
+    // (columns from the first wave on, rows from the last: each wave computes
+    // one kind, or none)
+    for (int j = (int)tid; j < kA * NIA; j += kRcThreads) {
+      const uint32_t it = fdiv((uint32_t)j, kp->kAm, kp->kAs);
+      int32_t* const slot = colS + (j - (int)it * kA) * NIA + it;
+      if (j < C) {
+        int32_t oa, ob;
+        offsets(kp, na, kp->nb, (uint32_t)j, oa, ob);
+        *slot = j < cols ? oa : (int32_t)kRcTabOOB;
+        colB[j] = j < cols ? ob : (int32_t)kRcTabOOB;
+      } else {
+        *slot = (int32_t)kRcTabOOB;
+      }
     }
-    for (int e = (int)(kRcThreads - 1 - tid); e < kB * NIB; e += kRcThreads) {
-      const int i = e / NIB + (e % NIB) * kB;
-      int32_t oa, ob;
-      offsets(kp, 0, na, (uint32_t)i, oa, ob);
-      rowS[e] = i < rows ? ob : (int32_t)kRcTabOOB;
-      if (i < R) rowA[i] = i < rows ? oa : (int32_t)kRcTabOOB;
+    for (int i = (int)(kRcThreads - 1 - tid); i < kB * NIB; i += kRcThreads) {
+      const uint32_t it = fdiv((uint32_t)i, kp->kBm, kp->kBs);
+      int32_t* const slot = rowS + (i - (int)it * kB) * NIB + it;
+      if (i < R) {
+        int32_t oa, ob;
+        offsets(kp, 0, na, (uint32_t)i, oa, ob);
+        *slot = i < rows ? ob : (int32_t)kRcTabOOB;
+        rowA[i] = i < rows ? oa : (int32_t)kRcTabOOB;
+      } else {
+        *slot = (int32_t)kRcTabOOB;
+      }
     }
     const uint32_t RP = (uint32_t)kp->RP;
     // this lane's place in the two walks
@@ -178,16 +190,18 @@ __global__ void __launch_bounds__(kRcThreads)
                                          [](float) {});
 }
 
-// fp8 cast-transpose (semantics: cast_fp8_rc_kernel).  amax only grows during
-// a launch: each work-group reads it as it starts, and one whose tile's max
-// is not above that value is done; the others look again and then commit one
-// atomic.
+// fp8 cast-transpose (semantics: cast_fp8_rc_kernel).  Where amax is asked
+// for, a work-group takes the tiles AmaxUnits gives it and commits their max
+// once (amax_commit_one).  With amax_in, a pass over A has just run: the tiles
+// are walked backwards, so that the part of A it read last is still in the
+// last-level cache (amax and cast of bf16 8192 x 14336: 113 -> 108 us, fp32:
+// 191 -> 184).
 template <class OP, int VA, int VB, int DIV>
 __global__ void __launch_bounds__(kRcThreads)
     cast_fp8_lane_kernel(const RCLaneParams p, const typename OP::TA* __restrict__ A,
                          typename OP::TB* __restrict__ B, float alpha, const float* __restrict__ scale_in,
                          const float* __restrict__ amax_in, float fp8_max, float scale_host,
-                         float* __restrict__ amax_out, float* __restrict__ scale_inv_out) {
+                         float* __restrict__ amax_out, float* __restrict__ scale_inv_out, AmaxUnits units) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ float red[kRcThreads / 64];
   KLane* kp = (KLane*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -199,22 +213,16 @@ __global__ void __launch_bounds__(kRcThreads)
     scale = (m > 0.0f && m <= 3.402823466e38f) ? fp8_max / m : 1.0f;
   }
   if (scale_inv_out && blockIdx.x == 0 && threadIdx.x == 0) *scale_inv_out = 1.0f / scale;
-  unsigned int* const am = reinterpret_cast<unsigned int*>(amax_out);
-  unsigned int seen = 0;
-  if (am && threadIdx.x == 0) seen = __hip_atomic_load(am, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  RCLane<OP, VA, VB, false, false, DIV>::run(kp, blockIdx.x, A, B, lds_raw, alpha, scale, [&](float m) {
-    if (!am) return;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
-  });
-  if (am && threadIdx.x == 0) {
-    float m = red[0];
-#pragma unroll
-    for (int w = 1; w < kRcThreads / 64; ++w) m = fmaxf(m, red[w]);
-    const unsigned int bits = __float_as_uint(m);
-    if (bits > seen && bits > __hip_atomic_load(am, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(am, bits);
+  float amax = 0.0f;
+  const uint32_t first = units.first(blockIdx.x), end = units.first(blockIdx.x + 1);
+  for (uint32_t t = first; t < end; ++t) {
+    if (t != first) __syncthreads();  // the previous tile's LDS reads
+    RCLane<OP, VA, VB, false, false, DIV>::run(kp, amax_in ? units.n - 1 - t : t, A, B, lds_raw, alpha, scale, [&](float m) {
+      amax = fmaxf(amax, m);
+      if (amax_out && t + 1 == end) wg_max_publish(amax, red);
+    });
   }
+  if (amax_out && threadIdx.x == 0) amax_commit_one(wg_max_collect(red), amax_out);
 }
 
 }  // namespace ttc

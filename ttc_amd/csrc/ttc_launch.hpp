@@ -113,10 +113,11 @@ hipError_t launch_fp8_lane(const RCLaneParams& p, const void* A, void* B, float 
                            float* scale_inv_out, size_t lds, hipStream_t s) {
   const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
   typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  AmaxUnits units = amax_units(p.walk.ntiles, amax_out != nullptr);
   void* args[] = {const_cast<RCLaneParams*>(&p), &a, &b, &alpha, &scale_in, &amax_in, &fp8_max, &scale_host,
-                  &amax_out, &scale_inv_out};
+                  &amax_out, &scale_inv_out, &units};
   return hipLaunchKernel(reinterpret_cast<const void*>(&cast_fp8_lane_kernel<OP, VA, VB, DIV>),
-                         dim3(p.walk.ntiles), dim3(kRcThreads), args, lds, s);
+                         dim3(units.work_groups()), dim3(kRcThreads), args, lds, s);
 }
 
 template <class OP, int VA, int VB, int MODE>
@@ -165,10 +166,11 @@ hipError_t launch_row_once(const RowParams& p, const void* A, void* B, double al
                            float* amax_out, float* scale_inv_out, unsigned grid, hipStream_t s) {
   const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
   typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  AmaxUnits units = amax_units(grid, amax_out != nullptr);
   void* args[] = {const_cast<RowParams*>(&p), &a, &b, &alpha, &beta, &scale_in, &amax_in, &fp8_max, &scale_host,
-                  &amax_out, &scale_inv_out};
-  return hipLaunchKernel(reinterpret_cast<const void*>(&row_once_kernel<OP, V, MODE, UNAL>), dim3(grid),
-                         dim3(kThreads), args, 0, s);
+                  &amax_out, &scale_inv_out, &units};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&row_once_kernel<OP, V, MODE, UNAL>),
+                         dim3(units.work_groups()), dim3(kThreads), args, 0, s);
 }
 
 template <class OP, int V, int MODE>

@@ -802,6 +802,8 @@ bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int v
   p.RP = (int32_t)(R | 1);
   p.kA = (int32_t)kA;
   p.kB = (int32_t)kB;
+  const FastDiv dkA = make_fastdiv((uint32_t)kA), dkB = make_fastdiv((uint32_t)kB);
+  p.kAm = dkA.m, p.kAs = dkA.s, p.kBm = dkB.m, p.kBs = dkB.s;
   const FastDiv dla = make_fastdiv((uint32_t)la), dlb = make_fastdiv((uint32_t)lb);
   p.la = dla.d, p.lam = dla.m, p.las = dla.s;
   p.lb = dlb.d, p.lbm = dlb.m, p.lbs = dlb.s;

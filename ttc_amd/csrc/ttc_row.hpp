@@ -232,8 +232,9 @@ __global__ void __launch_bounds__(kThreads)
     row_once_kernel(const RowParams p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
                     double alpha, double beta, const float* __restrict__ scale_in, const float* __restrict__ amax_in,
                     float fp8_max, float scale_host, float* __restrict__ amax_out,
-                    float* __restrict__ scale_inv_out) {
+                    float* __restrict__ scale_inv_out, AmaxUnits units) {
   constexpr bool FP8 = MODE == kModeFp8;
+  touch_lines<sizeof(RowParams)>(__builtin_amdgcn_kernarg_segment_ptr());
   float scale = 1.0f;
   if constexpr (FP8) {
     scale = scale_host;
@@ -250,10 +251,23 @@ __global__ void __launch_bounds__(kThreads)
     const uint32_t x = w % kXcds, q = gridDim.x / kXcds, r = gridDim.x % kXcds;
     w = x * q + (x < r ? x : r) + w / kXcds;
   }
-  const float amax =
-      row_chunk<OP, V, MODE, UNAL>(p, w, A, B, (typename OP::AL)alpha, (typename OP::BE)beta, scale);
   if constexpr (FP8) {
-    if (amax_out) block_amax_commit(amax, amax_out);
+    // the chunks AmaxUnits gives this work-group, one commit; backwards after
+    // an amax pass, which leaves the end of A in the last-level cache (bf16 128
+    // x 4096 x 32 x 8, both passes: 143 -> 130 us)
+    float amax = 0.0f;
+    const uint32_t end = units.first(w + 1);
+    for (uint32_t c = units.first(w); c < end; ++c)
+      amax = fmaxf(amax, row_chunk<OP, V, MODE, UNAL>(p, amax_in ? units.n - 1 - c : c, A, B,
+                                                      (typename OP::AL)alpha, (typename OP::BE)beta, scale));
+    if (amax_out) {
+      __shared__ float red[kThreads / 64];
+      wg_max_publish(amax, red);
+      __syncthreads();
+      if (threadIdx.x == 0) amax_commit_one(wg_max_collect(red), amax_out);
+    }
+  } else {
+    (void)row_chunk<OP, V, MODE, UNAL>(p, w, A, B, (typename OP::AL)alpha, (typename OP::BE)beta, scale);
   }
 }
 
