@@ -968,6 +968,19 @@ static void build_row_once(ttc_plan_s* pl, int v) {
     pl->row1.dnv = make_fastdiv(pl->row1.nv);
     pl->row1.total = rows * pl->row1.nv;
   }
+  // Rows of whole cache lines share none with their neighbours on either
+  // side: walked in A order, whose reads then run on (bf16 128 x 4096 x 32 x 8
+  // perm (0,2,1,3): 101 -> 94 us, to e4m3 96 -> 91; rows of 400 bytes lost a
+  // quarter that way).
+  const Geometry& g = pl->g;
+  bool lines = (long long)n0 * szA % 128 == 0 && (long long)n0 * szB % 128 == 0;
+  for (int k = 1; k < g.rank; ++k) lines = lines && g.sa[k] * szA % 128 == 0 && g.sb[k] * szB % 128 == 0;
+  if (lines)
+    for (int k = 1; k < g.rank; ++k) {
+      pl->row1.dn[k - 1] = make_fastdiv((uint32_t)g.size[k]);
+      pl->row1.sa[k - 1] = g.sa[k] * szA;
+      pl->row1.sb[k - 1] = g.sb[k] * szB;
+    }
   pl->row1.xcd_share = (long long)n0 * std::min(szA, szB) < 128;
   const long long chunk = (long long)kThreads * row_once_unroll(szA, szB, pl->row1_v, fp8, pl->row1_unaligned != 0);
   pl->row1_grid = (unsigned)((pl->row1.total + chunk - 1) / chunk);
