@@ -1037,21 +1037,41 @@ static int rc_whole_extent_tiles(const Geometry& g, int va, int vb, int vmax, in
   return std::min(n, max_out);
 }
 
-// Cost of a launch of one work-group per tile, in bytes of HBM traffic (a fit
-// of 79 shapes x ~190 tiles, measured: the tile it picks is 2.6% (mean) behind
-// each shape's fastest, the run-length score of choose_rc_tile's 8%): the
-// bytes moved plus what partial cache lines add to each contiguous run, each
-// tile's fixed cost and that of its slots (issued whether or not they hold an
-// element), and the latency of a tile, which the whole launch waits for once.
+// The power of two up to 128 that divides the byte offset of every contiguous
+// run of the tiles in B.
+static long long run_alignment_b(const Geometry& g, const int* tile, int szB) {
+  long long bits = 128;
+  bool in_run = true;
+  for (int q = 0; q < g.rank; ++q) {
+    const int k = g.perm[q];
+    if (!in_run || tile[k] != g.size[k]) bits |= (in_run ? tile[k] : 1) * g.sb[k] * szB;
+    in_run = in_run && tile[k] == g.size[k] && (q + 1 == g.rank || g.sb[g.perm[q + 1]] == g.sb[k] * g.size[k]);
+  }
+  return bits & -bits;
+}
+
+// Cost of a launch of one work-group per tile, in bytes of HBM traffic, fitted
+// to 173 shapes x ~100 tiles each: the tile it picks is measured 2.1% (mean)
+// and at most 10% behind each shape's fastest; with run lengths and slots
+// alone that was 4.9% and 92%, with the score of choose_rc_tile 8%.  In order:
+// the bytes moved; what each contiguous run adds, on B by how far it is off
+// the cache lines (lines written in parts; little of it in fp8 casts, which
+// write least); what a tile's group of rows or columns adds once; each tile's
+// slots, issued whether or not they hold an element; and the latency of a
+// tile, which the whole launch waits for once, longer with the slots of a
+// full-size instance, of which fewer are resident.
 static double lane_cost(const Geometry& g, const int* tile, int szA, int szB, int va, int vb, int div, bool beta,
                         const LaneFit& f) {
   long long ra, rb;
   tile_runs(g, tile, ra, rb);
   const double N = (double)g.elements, m = beta ? 2.0 : 1.0;
-  const double ba = std::min(8192.0, (double)ra * szA), bb = std::min(8192.0, (double)rb * szB);
+  const double ba = std::min(16384.0, (double)ra * szA), bb = std::min(16384.0, (double)rb * szB);
+  const double off = (double)(128 - run_alignment_b(g, tile, szB)) / 128.0;
   const double slots = rc_elems(szA) / va / div + rc_elems(szB) / vb / div * m;
-  return N * szA * (1.0 + 64.0 / ba) + N * szB * m * (1.0 + 180.0 / bb) + (double)f.ntiles * (600.0 + 1300.0 * slots) +
-         1000.0 * (double)(f.R * f.C) * (szA + szB * m);
+  return N * szA * (1.0 + 56.0 / ba + 7.0 / ((double)f.R * szA)) +
+         N * szB * m * (1.0 + ((szB == 1 ? 10.0 : 176.0) * off + 14.0) / bb + 14.0 / ((double)f.C * szB)) +
+         (double)f.ntiles * 850.0 * slots +
+         (div == 1 ? 795.0 : 425.0) * (double)(f.R * f.C) * (szA + szB * m);
 }
 
 // Tile of a launch of one work-group per tile: run-length targets on both
