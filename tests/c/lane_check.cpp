@@ -10,6 +10,7 @@
 //     nothing a padding slot stages lands where the tile's elements are.
 // Prints one summary line; exit status 1 on the first violation.
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <random>
@@ -154,13 +155,70 @@ static bool check_tile(const RCLaneParams& p, int szA, int szB, int va, int vb, 
   return true;
 }
 
+// The few-byte form of a launch against the full one: origins, partial groups
+// and the groups' offsets (sdiv itself is checked in main).
+static bool check_small(const RCLaneParams& p, const RCLaneSmall& s, int szA, int szB) {
+  CHECK(s.ntiles == p.walk.ntiles && s.R == p.R && s.C == p.C && s.Rl == p.Rl && s.Cl == p.Cl && s.kA == p.kA &&
+            s.kB == p.kB && s.tab16 * 16 == p.tab && s.spare == p.spare && (s.groups & 15) == p.na &&
+            s.groups >> 4 == p.nb && (s.R | 1) == p.RP,
+        "small fields");
+  const uint32_t step = p.walk.ntiles / 5000 + 1;
+  for (uint32_t w = 0; w < p.walk.ntiles; w += w < 64 || w + 64 > p.walk.ntiles ? 1 : step) {
+    uint32_t rem = rc_tile_of(p.walk, w), last = 0;
+    long long oa = 0, ob = 0;
+    for (int g = 0; g < p.grank; ++g) {
+      const uint32_t x = rem % p.grid[g].d;
+      rem /= p.grid[g].d;
+      oa += (long long)x * p.grid[g].tsa * szA;
+      ob += (long long)x * p.grid[g].tsb * szB;
+      if (x == p.grid[g].d - 1) last |= p.grid[g].part;
+    }
+    int64_t sa, sb;
+    const uint32_t sl = rc_small_origin(&s, w, sa, sb);
+    CHECK(sa == oa && sb == ob && sl == last, "small origin");
+  }
+  for (int side = 0; side < 2; ++side)
+    for (int l = 0; l < (side ? p.C : p.R); ++l) {
+      const int first = side ? p.na : 0, n = side ? p.nb : p.na;
+      int32_t oa = 0, ob = 0, sa, sb;
+      uint32_t r = (uint32_t)l;
+      for (int m = first; m < first + n; ++m) {
+        oa += (int32_t)(r % p.dim[m].d) * p.dim[m].sa;
+        ob += (int32_t)(r % p.dim[m].d) * p.dim[m].sb;
+        r /= p.dim[m].d;
+      }
+      rc_small_offsets(&s, first, n, (uint32_t)l, sa, sb);
+      CHECK(sa == oa && sb == ob, "small offsets");
+    }
+  return true;
+}
+
+// sdiv_by for every divisor and numerators at its quotients' edges, with
+// reciprocals 1 ulp off.
+static bool check_sdiv() {
+  std::mt19937_64 rng(7);
+  for (uint32_t d = 1; d < kSmallCount; d += d < 5000 ? 1 : 1 + (uint32_t)(rng() % 400)) {
+    const float inv = 1.0f / (float)d, nudged[3] = {inv, std::nextafterf(inv, 0.0f), std::nextafterf(inv, 2.0f)};
+    const uint32_t qmax = (kSmallCount - 1) / d;
+    for (int t = 0; t < 40; ++t) {
+      const uint32_t q = t == 0 ? 0 : t == 1 ? qmax : (uint32_t)(rng() % (qmax + 1));
+      for (const long long n : {(long long)q * d - 1, (long long)q * d, (long long)q * d + d - 1}) {
+        if (n < 0 || n >= kSmallCount) continue;
+        for (const float f : nudged) CHECK(sdiv_by((uint32_t)n, f) == (uint32_t)n / d, "sdiv");
+      }
+    }
+  }
+  return true;
+}
+
 int main(int argc, char** argv) {
   const int ncases = argc > 1 ? std::atoi(argv[1]) : 200;
   std::mt19937_64 rng(4242);
+  if (!check_sdiv()) return 1;
   const int pairs[][2] = {{TTC_S, TTC_S},       {TTC_D, TTC_D},    {TTC_C, TTC_C}, {TTC_Z, TTC_Z}, {TTC_BF16, TTC_BF16},
                           {TTC_S, TTC_BF16},    {TTC_F16, TTC_S},  {TTC_D, TTC_S}, {TTC_S, TTC_D}, {TTC_C, TTC_Z},
                           {TTC_BF16, TTC_E4M3}, {TTC_S, TTC_E5M2}};
-  long long walks = 0, tiles = 0, banded = 0, partial = 0, full_size = 0, far = 0;
+  long long walks = 0, tiles = 0, banded = 0, partial = 0, full_size = 0, far = 0, small = 0;
   for (int c = 0; c < ncases; ++c) {
     const int r = 2 + (int)(rng() % 5);
     int perm[8], size[8], lda[8], ldb[8];
@@ -196,6 +254,11 @@ int main(int argc, char** argv) {
                 continue;
               if (!build_lane_params(g, t, ta, tb, va, vb, grid, order, div, p, lds)) continue;
               bool ok = check_walk(g, t, p);
+              RCLaneSmall sp;
+              if (div == 2 && build_lane_small(g, t, ta, tb, order, p, sp)) {
+                ok = ok && check_small(p, sp, szA, szB);
+                ++small;
+              }
               ++walks;
               banded += p.walk.bandw != 0;
               full_size += div == 1;
@@ -246,6 +309,6 @@ int main(int argc, char** argv) {
       }
     }
   std::printf("lane check: %lld walks, %lld banded, %lld full-size instances, %lld tiles, %lld partial, "
-              "%lld with A spans past 2^30: ok\n", walks, banded, full_size, tiles, partial, far);
+              "%lld with A spans past 2^30, %lld in few bytes: ok\n", walks, banded, full_size, tiles, partial, far, small);
   return 0;
 }

@@ -27,18 +27,42 @@
 namespace ttc {
 
 using KLane = const __attribute__((address_space(4))) RCLaneParams;
-template <class OP, int VA, int VB, bool BETA, bool NT, int DIV>
-struct RCLane {
-  using TA = typename OP::TA;
-  using TB = typename OP::TB;
-  using L = typename OP::L;
-  static constexpr int NIA = rc_elems((int)sizeof(TA)) / VA / DIV;  // read slots per lane
-  static constexpr int NIB = rc_elems((int)sizeof(TB)) / VB / DIV;  // write slots per lane
-  static constexpr bool FP8 = is_fp8<OP>::value;
+using KLaneSmall = const __attribute__((address_space(4))) RCLaneSmall;
 
+// Where a tile's parameters come from: the same members over both forms.
+struct LaneFull {
+  KLane* kp;
+  __device__ __forceinline__ void touch() const { touch_lines<sizeof(RCLaneParams)>(kp); }
+  // offsets of tile `wg`'s origin (elements here; what `at` adds), and which
+  // groups are partial
+  __device__ __forceinline__ uint32_t origin(uint32_t wg, int64_t& bA, int64_t& bB) const {
+    RCWalk w;
+    w.ntiles = kp->walk.ntiles;
+    w.grid_order = kp->walk.grid_order;
+    w.bandw = kp->walk.bandw;
+    w.bandn = kp->walk.bandn;
+    w.bandin = kp->walk.bandin;
+    w.dper = FastDiv{kp->walk.dper.d, kp->walk.dper.m, kp->walk.dper.s, 0};
+    w.dband = FastDiv{kp->walk.dband.d, kp->walk.dband.m, kp->walk.dband.s, 0};
+    w.dw = FastDiv{kp->walk.dw.d, kp->walk.dw.m, kp->walk.dw.s, 0};
+    w.dwl = FastDiv{kp->walk.dwl.d, kp->walk.dwl.m, kp->walk.dwl.s, 0};
+    uint32_t rem = uniform(rc_tile_of(w, wg)), last = 0;
+    bA = bB = 0;
+    const int gr = kp->grank;
+#pragma unroll 1
+    for (int g = 0; g < gr; ++g) {
+      const uint32_t d = kp->grid[g].d, q = fdiv(rem, kp->grid[g].m, kp->grid[g].s), x = rem - q * d;
+      rem = q;
+      bA += (int64_t)x * kp->grid[g].tsa;
+      bB += (int64_t)x * kp->grid[g].tsb;
+      if (x == d - 1) last |= kp->grid[g].part;
+    }
+    return last;
+  }
+  template <class T> __device__ __forceinline__ static T* at(T* p, int64_t b) { return p + uniform64(b); }
   // Offsets of position l of a group: mixed-radix digits over its tile
   // extents times their byte strides.
-  __device__ __forceinline__ static void offsets(KLane* kp, int first, int n, uint32_t l, int32_t& oa, int32_t& ob) {
+  __device__ __forceinline__ void offsets(int first, int n, uint32_t l, int32_t& oa, int32_t& ob) const {
     oa = ob = 0;
 #pragma unroll 1
     for (int m = first; m < first + n; ++m) {
@@ -49,6 +73,50 @@ struct RCLane {
       ob += x * kp->dim[m].sb;
     }
   }
+  __device__ __forceinline__ uint32_t RP() const { return (uint32_t)kp->RP; }
+  __device__ __forceinline__ int na() const { return kp->na; }
+  __device__ __forceinline__ int nb() const { return kp->nb; }
+  __device__ __forceinline__ uint32_t tab() const { return (uint32_t)kp->tab; }
+  __device__ __forceinline__ uint32_t by_kA(uint32_t j) const { return fdiv(j, kp->kAm, kp->kAs); }
+  __device__ __forceinline__ uint32_t by_kB(uint32_t i) const { return fdiv(i, kp->kBm, kp->kBs); }
+  template <int VA> __device__ __forceinline__ uint32_t la() const { return kp->la; }
+  template <int VB> __device__ __forceinline__ uint32_t lb() const { return kp->lb; }
+  __device__ __forceinline__ uint32_t by_la(uint32_t t, uint32_t) const { return fdiv(t, kp->lam, kp->las); }
+  __device__ __forceinline__ uint32_t by_lb(uint32_t t, uint32_t) const { return fdiv(t, kp->lbm, kp->lbs); }
+};
+
+struct LaneSmall {
+  KLaneSmall* kp;
+  __device__ __forceinline__ void touch() const { touch_lines<sizeof(RCLaneSmall)>(kp); }
+  __device__ __forceinline__ uint32_t origin(uint32_t wg, int64_t& bA, int64_t& bB) const {
+    return rc_small_origin(kp, wg, bA, bB);
+  }
+  template <class T> __device__ __forceinline__ static T* at(T* p, int64_t b) {
+    return reinterpret_cast<T*>(const_cast<char*>(reinterpret_cast<const char*>(p)) + uniform64(b));
+  }
+  __device__ __forceinline__ void offsets(int first, int n, uint32_t l, int32_t& oa, int32_t& ob) const {
+    rc_small_offsets(kp, first, n, l, oa, ob);
+  }
+  __device__ __forceinline__ uint32_t RP() const { return (uint32_t)kp->R | 1u; }
+  __device__ __forceinline__ int na() const { return kp->groups & 15; }
+  __device__ __forceinline__ int nb() const { return kp->groups >> 4; }
+  __device__ __forceinline__ uint32_t tab() const { return (uint32_t)kp->tab16 * 16u; }
+  __device__ __forceinline__ uint32_t by_kA(uint32_t j) const { return sdiv(j, kp->kA); }
+  __device__ __forceinline__ uint32_t by_kB(uint32_t i) const { return sdiv(i, kp->kB); }
+  template <int VA> __device__ __forceinline__ uint32_t la() const { return (uint32_t)kp->R / VA; }
+  template <int VB> __device__ __forceinline__ uint32_t lb() const { return (uint32_t)kp->C / VB; }
+  __device__ __forceinline__ uint32_t by_la(uint32_t t, uint32_t la) const { return sdiv(t, la); }
+  __device__ __forceinline__ uint32_t by_lb(uint32_t t, uint32_t lb) const { return sdiv(t, lb); }
+};
+
+template <class OP, int VA, int VB, bool BETA, bool NT, int DIV>
+struct RCLane {
+  using TA = typename OP::TA;
+  using TB = typename OP::TB;
+  using L = typename OP::L;
+  static constexpr int NIA = rc_elems((int)sizeof(TA)) / VA / DIV;  // read slots per lane
+  static constexpr int NIB = rc_elems((int)sizeof(TB)) / VB / DIV;  // write slots per lane
+  static constexpr bool FP8 = is_fp8<OP>::value;
 
   // The tile of work-group `wg` of the launch (of the op, in a grouped one).
   // after(amax): called between staging and the barrier with max |alpha * a|
@@ -57,51 +125,34 @@ struct RCLane {
   __device__ __forceinline__ static void run(KLane* kp, uint32_t wg, const TA* __restrict__ A, TB* __restrict__ B,
                                              unsigned char* lds_raw, typename OP::AL alpha, typename OP::BE beta,
                                              F&& after) {
+    run(LaneFull{kp}, wg, A, B, lds_raw, alpha, beta, after);
+  }
+  template <class SRC, class F>
+  __device__ __forceinline__ static void run(const SRC src, uint32_t wg, const TA* __restrict__ A,
+                                             TB* __restrict__ B, unsigned char* lds_raw, typename OP::AL alpha,
+                                             typename OP::BE beta, F&& after) {
     const uint32_t tid = threadIdx.x;
-    touch_lines<sizeof(RCLaneParams)>(kp);
-    // tile origin
-    uint32_t rem;
-    {
-      RCWalk w;
-      w.ntiles = kp->walk.ntiles;
-      w.grid_order = kp->walk.grid_order;
-      w.bandw = kp->walk.bandw;
-      w.bandn = kp->walk.bandn;
-      w.bandin = kp->walk.bandin;
-      w.dper = FastDiv{kp->walk.dper.d, kp->walk.dper.m, kp->walk.dper.s, 0};
-      w.dband = FastDiv{kp->walk.dband.d, kp->walk.dband.m, kp->walk.dband.s, 0};
-      w.dw = FastDiv{kp->walk.dw.d, kp->walk.dw.m, kp->walk.dw.s, 0};
-      w.dwl = FastDiv{kp->walk.dwl.d, kp->walk.dwl.m, kp->walk.dwl.s, 0};
-      rem = uniform(rc_tile_of(w, wg));
-    }
-    int64_t bA = 0, bB = 0;
-    uint32_t last = 0;
-    const int gr = kp->grank;
-#pragma unroll 1
-    for (int g = 0; g < gr; ++g) {
-      const uint32_t d = kp->grid[g].d, q = fdiv(rem, kp->grid[g].m, kp->grid[g].s), x = rem - q * d;
-      rem = q;
-      bA += (int64_t)x * kp->grid[g].tsa;
-      bB += (int64_t)x * kp->grid[g].tsb;
-      if (x == d - 1) last |= kp->grid[g].part;
-    }
-    const int R = kp->R, C = kp->C, kA = kp->kA, kB = kp->kB, na = kp->na;
+    const auto kp = src.kp;
+    src.touch();
+    int64_t bA, bB;
+    const uint32_t last = src.origin(wg, bA, bB);
+    const int R = kp->R, C = kp->C, kA = kp->kA, kB = kp->kB, na = src.na();
     const int rows = (last & 1u) ? kp->Rl : R, cols = (last & 2u) ? kp->Cl : C;
     // tables: colS[jl * NIA + it] = A offset of column jl + it * kA, rowS its
     // mirror image for B; rowA and colB by row and column
     L* const data = reinterpret_cast<L*>(lds_raw);
-    int32_t* const colS = reinterpret_cast<int32_t*>(lds_raw + kp->tab);
+    int32_t* const colS = reinterpret_cast<int32_t*>(lds_raw + src.tab());
     int32_t* const rowS = colS + kA * NIA;
     int32_t* const rowA = rowS + kB * NIB;
     int32_t* const colB = rowA + R;
     // (columns from the first wave on, rows from the last: each wave computes
     // one kind, or none)
     for (int j = (int)tid; j < kA * NIA; j += kRcThreads) {
-      const uint32_t it = fdiv((uint32_t)j, kp->kAm, kp->kAs);
+      const uint32_t it = src.by_kA((uint32_t)j);
       int32_t* const slot = colS + (j - (int)it * kA) * NIA + it;
       if (j < C) {
         int32_t oa, ob;
-        offsets(kp, na, kp->nb, (uint32_t)j, oa, ob);
+        src.offsets(na, src.nb(), (uint32_t)j, oa, ob);
         *slot = j < cols ? oa : (int32_t)kRcTabOOB;
         colB[j] = j < cols ? ob : (int32_t)kRcTabOOB;
       } else {
@@ -109,21 +160,22 @@ struct RCLane {
       }
     }
     for (int i = (int)(kRcThreads - 1 - tid); i < kB * NIB; i += kRcThreads) {
-      const uint32_t it = fdiv((uint32_t)i, kp->kBm, kp->kBs);
+      const uint32_t it = src.by_kB((uint32_t)i);
       int32_t* const slot = rowS + (i - (int)it * kB) * NIB + it;
       if (i < R) {
         int32_t oa, ob;
-        offsets(kp, 0, na, (uint32_t)i, oa, ob);
+        src.offsets(0, na, (uint32_t)i, oa, ob);
         *slot = i < rows ? ob : (int32_t)kRcTabOOB;
         rowA[i] = i < rows ? oa : (int32_t)kRcTabOOB;
       } else {
         *slot = (int32_t)kRcTabOOB;
       }
     }
-    const uint32_t RP = (uint32_t)kp->RP;
+    const uint32_t RP = src.RP();
     // this lane's place in the two walks
-    const uint32_t jl = fdiv(tid, kp->lam, kp->las), ai = (tid - jl * kp->la) * VA;
-    const uint32_t il = fdiv(tid, kp->lbm, kp->lbs), bj = (tid - il * kp->lb) * VB;
+    const uint32_t la = src.template la<VA>(), lb = src.template lb<VB>();
+    const uint32_t jl = src.by_la(tid, la), ai = (tid - jl * la) * VA;
+    const uint32_t il = src.by_lb(tid, lb), bj = (tid - il * lb) * VB;
     const bool onA = jl < (uint32_t)kA, onB = il < (uint32_t)kB;
     const uint32_t sA = onA ? ai + jl * RP : (uint32_t)kp->spare, stepA = onA ? (uint32_t)kA * RP : 0u;
     const uint32_t sB = onB ? il + bj * RP : 0u, stepB = onB ? (uint32_t)kB : 0u;
@@ -131,7 +183,7 @@ struct RCLane {
     const uint32_t rowoff = onA ? (uint32_t)rowA[ai] : kRcTabOOB, coloff = onB ? (uint32_t)colB[bj] : kRcTabOOB;
     const int32_t* const cs = colS + (onA ? jl * NIA : 0u);
     const int32_t* const rs = rowS + (onB ? il * NIB : 0u);
-    const BufRes ra = make_res(A + uniform64(bA)), rb = make_res(B + uniform64(bB));
+    const BufRes ra = make_res(SRC::at(A, bA)), rb = make_res(SRC::at(B, bB));
     TA va[NIA][VA];
     TB old[NIB][VB];
     uint32_t ob[NIB];
@@ -188,6 +240,16 @@ __global__ void __launch_bounds__(kRcThreads)
   KLane* kp = (KLane*)__builtin_amdgcn_kernarg_segment_ptr();
   RCLane<OP, VA, VB, BETA, NT, DIV>::run(kp, blockIdx.x, A, B, lds_raw, (typename OP::AL)alpha, (typename OP::BE)beta,
                                          [](float) {});
+}
+
+template <class OP, int VA, int VB, bool BETA, bool NT, int DIV>
+__global__ void __launch_bounds__(kRcThreads)
+    transpose_small_kernel(const RCLaneSmall p, const typename OP::TA* __restrict__ A,
+                           typename OP::TB* __restrict__ B, double alpha, double beta) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  const LaneSmall src{(KLaneSmall*)__builtin_amdgcn_kernarg_segment_ptr()};
+  RCLane<OP, VA, VB, BETA, NT, DIV>::run(src, blockIdx.x, A, B, lds_raw, (typename OP::AL)alpha,
+                                         (typename OP::BE)beta, [](float) {});
 }
 
 // fp8 cast-transpose (semantics: cast_fp8_rc_kernel).  Where amax is asked

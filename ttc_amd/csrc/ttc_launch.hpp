@@ -33,6 +33,10 @@ using LaunchFp8LaneFn = hipError_t (*)(const RCLaneParams&, const void*, void*, 
 using LaunchRowFn = hipError_t (*)(const RowParams&, const void*, void*, double, double, const float*, const float*,
                                    float, float, float*, float*, unsigned, hipStream_t);
 
+using LaunchLaneSmallFn = hipError_t (*)(const RCLaneSmall&, const void*, void*, double, double, size_t, hipStream_t);
+
+using LaunchRowSmallFn = hipError_t (*)(const RowSmall&, const void*, void*, double, double, hipStream_t);
+
 struct KernelEntry {
   int ta, tb, va, vb, mode, family;
   LaunchFn launch;
@@ -49,6 +53,9 @@ struct KernelEntry {
   // row x column family, one tile per work-group: instance of DIV 1, 2
   LaunchLaneFn launch_lane[2];
   LaunchFp8LaneFn launch_fp8_lane[2];
+  // launches whose parameters fit kSmallArgs
+  LaunchLaneSmallFn launch_lane_small;  // DIV 2
+  LaunchRowSmallFn launch_row_small;
 };
 
 template <class OP, int VA, int VB, bool BETA, bool NT>
@@ -107,6 +114,16 @@ hipError_t launch_lane(const RCLaneParams& p, const void* A, void* B, double alp
                          dim3(p.walk.ntiles), dim3(kRcThreads), args, lds, s);
 }
 
+template <class OP, int VA, int VB, bool BETA, bool NT>
+hipError_t launch_lane_small(const RCLaneSmall& p, const void* A, void* B, double alpha, double beta, size_t lds,
+                             hipStream_t s) {
+  const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
+  typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  void* args[] = {const_cast<RCLaneSmall*>(&p), &a, &b, &alpha, &beta};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&transpose_small_kernel<OP, VA, VB, BETA, NT, 2>),
+                         dim3(p.ntiles), dim3(kRcThreads), args, lds, s);
+}
+
 template <class OP, int VA, int VB, int DIV>
 hipError_t launch_fp8_lane(const RCLaneParams& p, const void* A, void* B, float alpha, const float* scale_in,
                            const float* amax_in, float fp8_max, float scale_host, float* amax_out,
@@ -144,6 +161,7 @@ KernelEntry make_rc_entry(int ta, int tb) {
     }
     e.launch_lane[0] = &launch_lane<OP, VA, VB, beta, nt, 1>;
     e.launch_lane[1] = &launch_lane<OP, VA, VB, beta, nt, 2>;
+    e.launch_lane_small = &launch_lane_small<OP, VA, VB, beta, nt>;
   }
   return e;
 }
@@ -173,11 +191,21 @@ hipError_t launch_row_once(const RowParams& p, const void* A, void* B, double al
                          dim3(units.work_groups()), dim3(kThreads), args, 0, s);
 }
 
+template <class OP, int V, int MODE, bool UNAL>
+hipError_t launch_row_small(const RowSmall& p, const void* A, void* B, double alpha, double beta, hipStream_t s) {
+  const typename OP::TA* a = static_cast<const typename OP::TA*>(A);
+  typename OP::TB* b = static_cast<typename OP::TB*>(B);
+  void* args[] = {const_cast<RowSmall*>(&p), &a, &b, &alpha, &beta};
+  return hipLaunchKernel(reinterpret_cast<const void*>(&row_small_kernel<OP, V, MODE, UNAL>), dim3(p.grid),
+                         dim3(kThreads), args, 0, s);
+}
+
 template <class OP, int V, int MODE>
 KernelEntry make_row_entry(int ta, int tb) {
   KernelEntry e{ta, tb, V, V, MODE, kFamRow, nullptr, nullptr, nullptr, nullptr, nullptr};
   e.launch_row = &launch_row<OP, V, MODE>;
   e.launch_row_once = &launch_row_once<OP, V, MODE, false>;
+  if constexpr (MODE != kModeFp8) e.launch_row_small = &launch_row_small<OP, V, MODE, false>;
   e.func = reinterpret_cast<const void*>(&row_kernel<OP, V, MODE>);
   return e;
 }
@@ -187,6 +215,7 @@ template <class OP, int V, int MODE>
 KernelEntry make_row_unaligned_entry(int ta, int tb) {
   KernelEntry e{ta, tb, V, V, MODE, kFamRowUnaligned, nullptr, nullptr, nullptr, nullptr, nullptr};
   e.launch_row_once = &launch_row_once<OP, V, MODE, true>;
+  if constexpr (MODE != kModeFp8) e.launch_row_small = &launch_row_small<OP, V, MODE, true>;
   return e;
 }
 

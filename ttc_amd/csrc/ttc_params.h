@@ -259,6 +259,118 @@ struct RCTile {
   uint32_t flags, pad_;
 };
 
+// Launches of few dimensions in few bytes of arguments: with at most 112
+// (kSmallArgs and A, B, alpha, beta) the host's part of a launch takes 2.7 us,
+// with more 3.7-4.3 (an empty kernel), and the kernel reads two lines of
+// arguments instead of up to ten.  Tiles, and vectors of rows, are counted
+// below 2^20, so that divisions go through floats (sdiv).  A tile's chain of
+// divisions is longer than with FastDiv's constants: tiles take this form up
+// to kSmallBytes read and written, where the host is what a sequence of calls
+// waits for (fp32 1024 x 1024, 8 MiB: 4.5 -> 4.3 us per call, fp64 37 x 21 x 19
+// x 5 4.5 -> 4.3; complex64 96 x 80 x 110, 13 MB, 4.88 -> 4.98, fp32 2048 x 1024
+// 5.03 -> 5.10).  Rows take it wherever it fits (fp32 rows of 64, 31 MB: 5.1 ->
+// 4.8).
+constexpr uint32_t kSmallCount = 1u << 20;
+constexpr long long kSmallBytes = 8ll << 20;
+constexpr int kSmallArgs = 80, kSmallDims = 4, kSmallRowDims = 5;
+
+// n / d for n < 2^20: (n + 1/2) / d is at least 1 / 2d off every integer, the
+// error of the product below 2^-21 * n / d (a reciprocal within 1 ulp).
+TTC_HD inline uint32_t sdiv_by(uint32_t n, float inv) { return (uint32_t)(((float)n + 0.5f) * inv); }
+TTC_HD inline uint32_t sdiv(uint32_t n, uint32_t d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return sdiv_by(n, __builtin_amdgcn_rcpf((float)d));
+#else
+  return sdiv_by(n, 1.0f / (float)d);
+#endif
+}
+
+struct RCSmallDim {
+  int32_t sa, sb;  // A and B byte strides
+  uint16_t d, n;   // tile extent, tiles along the dimension
+};
+// RCLaneParams (which see) of up to kSmallDims dimensions.
+struct RCLaneSmall {
+  uint32_t ntiles;
+  uint16_t R, C, Rl, Cl, kA, kB;
+  uint16_t tab16, spare;   // byte offset of the tables / 16
+  uint32_t bandin_w;       // RCWalk::bandin, bandw << 24
+  uint16_t bandn;
+  uint8_t grid_order, groups;  // na, nb << 4
+  uint16_t grid;           // walk order: a nibble per tiled dimension, index in dim | RCGridDim::part << 2
+  uint8_t grank, pad_;
+  RCSmallDim dim[kSmallDims];  // row group, column group, other dimensions
+};
+static_assert(sizeof(RCLaneSmall) == kSmallArgs, "kernel arguments");
+
+// rc_tile_of, and the tile's origin: byte offsets and partial groups (bits of
+// RCGridDim::part).  P: a pointer to the parameters, in any address space.
+template <class P> TTC_HD inline uint32_t rc_small_tile_of(P p, uint32_t w) {
+  uint32_t id = w;
+  const uint32_t nt = p->ntiles, order = p->grid_order;
+  if (order == 3) {
+    const uint32_t x = w % kXcds, q = nt / kXcds, rem = nt % kXcds;
+    id = x * q + (x < rem ? x : rem) + w / kXcds;
+  } else if (order == 2) {
+    constexpr uint32_t kRound = 512, kPer = kRound / kXcds;
+    const uint32_t base = w / kRound * kRound, l = w - base;
+    if (base + kRound <= nt) id = base + l % kXcds * kPer + l / kXcds;
+  }
+  const uint32_t bandin = p->bandin_w & 0xffffffu, bandw = p->bandin_w >> 24, bandn = p->bandn;
+  if (bandw) {
+    const uint32_t per = bandn * bandin, band = bandw * bandin;
+    const uint32_t hi = sdiv(id, per);
+    uint32_t r = id - hi * per;
+    const uint32_t b = sdiv(r, band);
+    r -= b * band;
+    const uint32_t wide = bandn - b * bandw < bandw ? bandn - b * bandw : bandw;
+    const uint32_t low = sdiv(r, wide);
+    id = low + bandin * (b * bandw + (r - low * wide) + bandn * hi);
+  }
+  return id;
+}
+template <class P> TTC_HD inline uint32_t rc_small_origin(P p, uint32_t w, int64_t& oa, int64_t& ob) {
+  uint32_t rem = rc_small_tile_of(p, w), last = 0, map = p->grid;
+  oa = ob = 0;
+  const int gr = p->grank;
+#pragma unroll 1
+  for (int g = 0; g < gr; ++g, map >>= 4) {
+    const uint32_t k = map & 3u, n = p->dim[k].n, q = sdiv(rem, n), x = rem - q * n;
+    rem = q;
+    oa += (int64_t)(x * p->dim[k].d) * p->dim[k].sa;
+    ob += (int64_t)(x * p->dim[k].d) * p->dim[k].sb;
+    if (x == n - 1) last |= map >> 2 & 3u;
+  }
+  return last;
+}
+// Byte offsets of position l of a group (of n dimensions from `first` on).
+template <class P>
+TTC_HD inline void rc_small_offsets(P p, int first, int n, uint32_t l, int32_t& oa, int32_t& ob) {
+  oa = ob = 0;
+#pragma unroll 1
+  for (int m = first; m < first + n; ++m) {
+    const uint32_t d = p->dim[m].d, q = sdiv(l, d);
+    const int32_t x = (int32_t)(l - q * d);
+    l = q;
+    oa += x * p->dim[m].sa;
+    ob += x * p->dim[m].sb;
+  }
+}
+
+// RowParams of up to kSmallRowDims row dimensions.
+struct RowSmallDim {
+  int32_t sa, sb;  // byte strides
+  uint32_t d;
+};
+struct RowSmall {
+  uint32_t total, nv;
+  int32_t n0;
+  uint16_t rank, xcd_share;
+  RowSmallDim dim[kSmallRowDims];
+  uint32_t grid;
+};
+static_assert(sizeof(RowSmall) == kSmallArgs, "kernel arguments");
+
 // One-chunk-per-work-group row copy (row_once_kernel): vectors in flight per
 // lane.  16-byte vectors: one, so that a launch has the most work-groups (200
 // MiB fp32: 6.0 TB/s with one, 5.7 with two, 5.6 with four); narrower and

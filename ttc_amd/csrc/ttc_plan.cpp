@@ -945,6 +945,64 @@ ttc_status_t build_row_params(const Geometry& g, int ta, int tb, int v, RowParam
   return TTC_SUCCESS;
 }
 
+bool build_lane_small(const Geometry& g, const int* tile, int ta, int tb, int tile_order, const RCLaneParams& full,
+                      RCLaneSmall& p) {
+  const int szA = dtype_bytes(ta), szB = dtype_bytes(tb);
+  if (szB == 1 || full.walk.ntiles >= kSmallCount || full.walk.bandn > 65535u) return false;
+  int na, nb, ga[kMaxDim], gb[kMaxDim], dims[kSmallDims], n = 0, at[kMaxDim];
+  if (!rc_groups(g, tile, na, ga, nb, gb) || na + nb > kSmallDims) return false;
+  for (int k = 0; k < g.rank; ++k) at[k] = -1;
+  for (int m = 0; m < na; ++m) at[dims[n] = ga[m]] = n, ++n;
+  for (int m = 0; m < nb; ++m) at[dims[n] = gb[m]] = n, ++n;
+  for (int k = 0; k < g.rank; ++k)
+    if (at[k] < 0 && g.size[k] > tile[k]) {
+      if (n == kSmallDims) return false;
+      at[dims[n] = k] = n, ++n;
+    }
+  std::memset(&p, 0, sizeof(p));
+  for (int m = 0; m < n; ++m) {
+    const int k = dims[m];
+    const long long tiles = (g.size[k] + tile[k] - 1) / tile[k], sa = g.sa[k] * szA, sb = g.sb[k] * szB;
+    if (tiles > 65535 || tile[k] > 65535 || sa > INT_MAX || sb > INT_MAX) return false;
+    p.dim[m] = RCSmallDim{(int32_t)sa, (int32_t)sb, (uint16_t)tile[k], (uint16_t)tiles};
+  }
+  int grank = 0;
+  for (int q = 0; q < g.rank; ++q) {  // (as build_lane_params)
+    const int k = tile_order >= 2 ? g.perm[q] : q;
+    if (g.size[k] <= tile[k]) continue;
+    p.grid |= (uint16_t)((uint32_t)(at[k] | (int)full.grid[grank].part << 2) << (4 * grank));
+    ++grank;
+  }
+  if (full.spare > 65535 || full.tab / 16 > 65535 || full.walk.bandin > 0xffffffu) return false;
+  p.grank = (uint8_t)grank;
+  p.ntiles = full.walk.ntiles;
+  p.R = (uint16_t)full.R, p.C = (uint16_t)full.C, p.Rl = (uint16_t)full.Rl, p.Cl = (uint16_t)full.Cl;
+  p.kA = (uint16_t)full.kA, p.kB = (uint16_t)full.kB;
+  p.tab16 = (uint16_t)(full.tab / 16);
+  p.spare = (uint16_t)full.spare;
+  p.bandin_w = full.walk.bandin | full.walk.bandw << 24;
+  p.bandn = (uint16_t)full.walk.bandn;
+  p.grid_order = (uint8_t)full.walk.grid_order;
+  p.groups = (uint8_t)(na | nb << 4);
+  return true;
+}
+
+bool build_row_small(const RowParams& full, unsigned grid, RowSmall& p) {
+  if (full.total == 0 || full.total >= kSmallCount || full.rank > kSmallRowDims) return false;
+  std::memset(&p, 0, sizeof(p));
+  for (int k = 0; k < full.rank; ++k) {
+    if (full.sa[k] > INT_MAX || full.sb[k] > INT_MAX) return false;
+    p.dim[k] = RowSmallDim{(int32_t)full.sa[k], (int32_t)full.sb[k], full.dn[k].d};
+  }
+  p.total = full.total;
+  p.nv = full.nv;
+  p.n0 = full.n0;
+  p.rank = (uint16_t)full.rank;
+  p.xcd_share = (uint16_t)(full.xcd_share != 0);
+  p.grid = grid;
+  return true;
+}
+
 // The one-chunk-per-work-group launch of row copy p (aligned vectors of v
 // elements): unaligned vectors where they are wider.  Rows shorter than a
 // cache line share lines with their neighbours in A and B, which then meet in
@@ -957,6 +1015,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
   pl->row1_v = v;
   pl->row1_unaligned = 0;
   pl->row1_grid = 0;
+  pl->small = 0;
   if (pl->row.total == 0 || (pl->wg_per_cu > 0 && pl->min_div == 1)) return;
   const bool may = !pl->vec_given && row_unaligned_mode(szA, szB, !pl->beta_is_zero, pl->nt_store != 0);
   const int w = may ? row_unaligned_width(szA, szB, n0) : 1;
@@ -984,6 +1043,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
   pl->row1.xcd_share = (long long)n0 * std::min(szA, szB) < 128;
   const long long chunk = (long long)kThreads * row_once_unroll(szA, szB, pl->row1_v, fp8, pl->row1_unaligned != 0);
   pl->row1_grid = (unsigned)((pl->row1.total + chunk - 1) / chunk);
+  pl->small = !fp8 && build_row_small(pl->row1, pl->row1_grid, pl->row_small);
 }
 
 static int rc_whole_extent_tiles(const Geometry& g, int va, int vb, int vmax, int (*out)[kMaxDim], int max_out) {
@@ -1318,11 +1378,15 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     // one tile per work-group unless the caller asks for resident
     // work-groups or LDS buffers, which only the pipelined kernel has
     pl->lane_div = 0;
+    pl->small = 0;
     if (pl->one_tile && st == TTC_SUCCESS)
       for (int div = 2; div >= pl->min_div && pl->lane_div == 0; --div)
         if (build_lane_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->tile_order, div, pl->lane,
                               pl->lane_lds))
           pl->lane_div = div;
+    const long long moved = dtype_bytes(pl->type_a) + (pl->beta_is_zero ? 1ll : 2ll) * dtype_bytes(pl->type_b);
+    pl->small = pl->lane_div == 2 && g.elements <= kSmallBytes / moved &&
+                build_lane_small(g, tile, pl->type_a, pl->type_b, pl->tile_order, pl->lane, pl->lane_small);
   } else {
     std::memset(&pl->rc, 0, sizeof(pl->rc));
     st = build_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->p, pl->lds_bytes, pl->lds_pad);

@@ -116,6 +116,10 @@ bool choose_rc_tile(const Geometry& g, int ta, int tb, int va, int vb, int run_a
 // kernel.  choose_lane_tile: the heuristic tile of such a launch.
 bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int va, int vb, int grid_order,
                        int tile_order, int div, RCLaneParams& p, int& lds_bytes);
+// The same launch in few bytes of kernel arguments, where it fits.
+bool build_lane_small(const Geometry& g, const int* tile, int ta, int tb, int tile_order, const RCLaneParams& full,
+                      RCLaneSmall& p);
+bool build_row_small(const RowParams& full, unsigned grid, RowSmall& p);
 bool choose_lane_tile(const Geometry& g, int ta, int tb, int va, int vb, bool beta, int* tile, int min_div = 1);
 // The launch's LDS offset tables (p.ntab entries, the layout of RCParams),
 // as the kernel's setup() builds them.
@@ -160,5 +164,8 @@ struct ttc_plan_s {
   ttc::RowParams row1;   // one chunk per work-group (row_once_kernel)
   int row1_v, row1_unaligned;
   unsigned row1_grid;    // 0: row_kernel (wg_per_cu given)
+  int small;             // lane_small (one tile per work-group, DIV 2) or row_small is the launch's
+  ttc::RCLaneSmall lane_small;
+  ttc::RowSmall row_small;
   ttc_plan_s* fallback;  // scalar-vector plan for misaligned pointers (may be null)
 };

@@ -125,7 +125,8 @@ template <class T, int V> struct __attribute__((packed, aligned(sizeof(T)))) Row
 // copy 4740 -> 6010; bf16 128 x 4096 x 32 x 8 perm (0,2,1,3) 4760 -> 5340;
 // fp32 rows of 127 3890 -> 4730, of 5 2210 -> 3040; bf16 rows of 127
 // 2180 -> 4070, of 5 1270 -> 2240.
-// P: RowParams as a kernel argument or in a grouped launch's work table.
+// P: RowParams as a kernel argument or in a grouped launch's work table, or
+// RowSmall.
 // Returns max |alpha * a| of this lane's elements (fp8 casts).
 template <class OP, int V, int MODE, bool UNAL, class P>
 __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typename OP::TA* __restrict__ A,
@@ -134,6 +135,7 @@ __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typenam
   using TA = typename OP::TA;
   using TB = typename OP::TB;
   using L = typename OP::L;
+  constexpr bool kSmall = std::is_same<P, RowSmall>::value;
   constexpr bool FP8 = MODE == kModeFp8;
   constexpr bool BETA = MODE == kModeBeta;
   constexpr bool NT = MODE == kModeBzNt;
@@ -151,7 +153,9 @@ __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typenam
     const uint32_t g = g0 + (uint32_t)(u * kThreads);
     ok[u] = g < p.total;
     const uint32_t gg = ok[u] ? g : 0u;
-    const uint32_t row = fdiv(gg, p.dnv.m, p.dnv.s);
+    uint32_t row;
+    if constexpr (kSmall) row = sdiv(gg, p.nv);
+    else row = fdiv(gg, p.dnv.m, p.dnv.s);
     int32_t e = (int32_t)(gg - row * p.nv) * V;
     skip[u] = 0;
     if constexpr (UNAL) {
@@ -161,13 +165,20 @@ __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typenam
     int64_t xa = (int64_t)e * (int64_t)sizeof(TA), xb = (int64_t)e * (int64_t)sizeof(TB);
     uint32_t rem = row;
 #pragma unroll
-    for (int k = 0; k < kMaxDim; ++k) {
+    for (int k = 0; k < (kSmall ? kSmallRowDims : kMaxDim); ++k) {
       if (k < p.rank) {
-        const uint32_t q = fdiv(rem, p.dn[k].m, p.dn[k].s);
-        const uint32_t x = rem - q * p.dn[k].d;
-        rem = q;
-        xa += (int64_t)x * p.sa[k];
-        xb += (int64_t)x * p.sb[k];
+        if constexpr (kSmall) {
+          const uint32_t q = sdiv(rem, p.dim[k].d), x = rem - q * p.dim[k].d;
+          rem = q;
+          xa += (int64_t)x * p.dim[k].sa;
+          xb += (int64_t)x * p.dim[k].sb;
+        } else {
+          const uint32_t q = fdiv(rem, p.dn[k].m, p.dn[k].s);
+          const uint32_t x = rem - q * p.dn[k].d;
+          rem = q;
+          xa += (int64_t)x * p.sa[k];
+          xb += (int64_t)x * p.sb[k];
+        }
       }
     }
     ob[u] = xb;
@@ -269,6 +280,20 @@ __global__ void __launch_bounds__(kThreads)
   } else {
     (void)row_chunk<OP, V, MODE, UNAL>(p, w, A, B, (typename OP::AL)alpha, (typename OP::BE)beta, scale);
   }
+}
+
+// The same with few bytes of arguments (RowSmall), without casts to fp8.
+template <class OP, int V, int MODE, bool UNAL>
+__global__ void __launch_bounds__(kThreads)
+    row_small_kernel(const RowSmall p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
+                     double alpha, double beta) {
+  touch_lines<sizeof(RowSmall)>(__builtin_amdgcn_kernarg_segment_ptr());
+  uint32_t w = blockIdx.x;
+  if (p.xcd_share) {
+    const uint32_t x = w % kXcds, q = p.grid / kXcds, r = p.grid % kXcds;
+    w = x * q + (x < r ? x : r) + w / kXcds;
+  }
+  (void)row_chunk<OP, V, MODE, UNAL>(p, w, A, B, (typename OP::AL)alpha, (typename OP::BE)beta, 1.0f);
 }
 
 }  // namespace ttc

@@ -128,6 +128,8 @@ static ttc_status_t launch_row_chunks(const ttc_plan_s* use, const KernelEntry* 
   if (use->row1_unaligned)
     e = find_kernel(use->type_a, use->type_b, use->row1_v, use->row1_v, mode, kFamRowUnaligned);
   if (!e) return TTC_ERROR_UNSUPPORTED;
+  if (use->small && mode != kModeFp8)
+    return e->launch_row_small(use->row_small, A, B, alpha, beta, s) == hipSuccess ? TTC_SUCCESS : TTC_ERROR_HIP;
   return e->launch_row_once(use->row1, A, B, alpha, beta, scale_in, amax_in, fp8_max, scale, amax_out, scale_inv_out,
                             use->row1_grid, s) == hipSuccess
              ? TTC_SUCCESS
@@ -152,6 +154,10 @@ ttc_status_t launch_plan(const ttc_plan_s* pl, const void* A, void* B, double al
                ? TTC_SUCCESS
                : TTC_ERROR_HIP;
   }
+  if (use->family == kFamRC && use->lane_div && use->small)
+    return e->launch_lane_small(use->lane_small, A, B, alpha, beta, (size_t)use->lane_lds, s) == hipSuccess
+               ? TTC_SUCCESS
+               : TTC_ERROR_HIP;
   if (use->family == kFamRC && use->lane_div)
     return e->launch_lane[use->lane_div - 1](use->lane, A, B, alpha, beta, (size_t)use->lane_lds, s) == hipSuccess
                ? TTC_SUCCESS
