@@ -373,11 +373,14 @@ static_assert(sizeof(RowSmall) == kSmallArgs, "kernel arguments");
 
 // One-chunk-per-work-group row copy (row_once_kernel): vectors in flight per
 // lane.  16-byte vectors: one, so that a launch has the most work-groups (200
-// MiB fp32: 6.0 TB/s with one, 5.7 with two, 5.6 with four); narrower and
-// unaligned ones: two (fp64 rows of 9 with beta: 4.5 with one, 4.9 with two);
-// fp8 casts: four (fp32 128 x 4096 x 32 x 8: 159 us with one, 143, 135).
+// MiB fp32: 6.0 TB/s with one, 5.7 with two, 5.6 with four); unaligned ones
+// and those of 8 bytes: two (fp64 rows of 447 with beta, 1.3 GB: 250 us with
+// one, 240, 253 with four); of 4 bytes and less: four (fp32 rows of 127 with
+// beta, 422 MB: 106, 116, 92; of 9: 73, 70, 62); fp8 casts: four (fp32 128 x
+// 4096 x 32 x 8: 159 us with one, 143, 135).
 constexpr int row_once_unroll(int bytes_a, int bytes_b, int v, bool fp8, bool unaligned) {
-  return fp8 ? 4 : ((v * bytes_a == 16 || v * bytes_b == 16) && !unaligned ? 1 : 2);
+  const int bytes = v * (bytes_a > bytes_b ? bytes_a : bytes_b);
+  return fp8 ? 4 : unaligned ? 2 : bytes >= 16 ? 1 : bytes >= 8 ? 2 : 4;
 }
 
 // Which units (tiles, chunks) a work-group of an fp8 cast takes.  Without
