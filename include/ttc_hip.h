@@ -226,8 +226,8 @@ ttc_status_t ttc_batch_destroy(ttc_batch_t batch);
  * is built on the host (host heap only) and copied with hipMemcpyAsync on
  * `stream`, ordered after that stream's earlier work; the call returns once
  * the kernels are enqueued.  A table larger than the workspace (about 1 KiB
- * per op, plus about 24 bytes per tile of the ops in persistent launches)
- * returns TTC_ERROR_WORKSPACE.
+ * per op, 0.3 KiB per row copy, plus about 24 bytes per tile of the ops in
+ * persistent launches) returns TTC_ERROR_WORKSPACE.
  * Every call on one GPU shares that GPU's workspace: calls on one stream
  * are ordered, but calls that overlap on one GPU (different streams or host
  * threads, without ordering between them) race. */

@@ -39,3 +39,18 @@ def test_rows_on_both_sides(gpu, code):
         for beta in (0.0, 0.75):
             check(gpu, tA, tB, perm, size, 1.25, beta, seed=n)
         check(gpu, tA, tB, perm, size, 1.0, 0.0, seed=n, offset_a=1, offset_b=1)
+
+
+def test_many_small_rows_fit_the_workspace(gpu):
+    """40000 row copies in one allocation-free grouped launch: 336 bytes of
+    work table per op is what it held before its records were split."""
+    import torch
+    from ttc_amd import runtime as rt
+    nops, size = 40000, [4, 3, 2]
+    A = torch.randn(nops, 24, device=gpu)
+    B = torch.zeros(nops, 24, device=gpu)
+    a, b = A.data_ptr(), B.data_ptr()
+    rt.batch_execute_noalloc([dict(type_a=rt.S, perm=[0, 2, 1], size=size, alpha=1.0, beta=0.0, A=a + 96 * i,
+                                   B=b + 96 * i) for i in range(nops)])
+    torch.cuda.synchronize()
+    assert torch.equal(B.view(nops, 3, 2, 4), A.view(nops, 2, 3, 4).transpose(1, 2))

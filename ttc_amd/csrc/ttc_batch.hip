@@ -99,9 +99,10 @@ struct BatchGroup {
 // op records point at their tile records once the image's device address is
 // known (render).
 struct BatchImage {
-  enum { kOne, kOneBegin, kOneBlocks, kBox, kRC, kWg, kBases, kRcTiles, kRcTables, kSections };
-  std::vector<BatchOneOp> one;          // ops of the one-work-group-per-tile launch
-  std::vector<uint32_t> one_begin;      // first tile of each
+  enum { kOne, kOneRows, kOneIndex, kOneBlocks, kBox, kRC, kWg, kBases, kRcTiles, kRcTables, kSections };
+  std::vector<OneLane> one;             // ops of the one-work-group-per-tile launch: row x column
+  std::vector<OneRow> one_rows;         // and row copies
+  std::vector<OneIndex> one_index;      // first tile and record of each
   std::vector<uint32_t> one_block;      // the op each block of kOneBlock tiles starts in
   std::vector<BatchOpDev> box;
   std::vector<BatchRCOpDev> rcs;
@@ -115,8 +116,9 @@ struct BatchImage {
   size_t bytes = 0;
 
   void layout() {
-    const size_t len[kSections] = {sizeof(BatchOneOp) * one.size(),     sizeof(uint32_t) * one_begin.size(),
-                                   sizeof(uint32_t) * one_block.size(), sizeof(BatchOpDev) * box.size(),
+    const size_t len[kSections] = {sizeof(OneLane) * one.size(),        sizeof(OneRow) * one_rows.size(),
+                                   sizeof(OneIndex) * one_index.size(), sizeof(uint32_t) * one_block.size(),
+                                   sizeof(BatchOpDev) * box.size(),
                                    sizeof(BatchRCOpDev) * rcs.size(),   sizeof(uint32_t) * wg.size(),
                                    sizeof(TileBase) * bases.size(),     sizeof(RCTile) * rct.size(),
                                    sizeof(int32_t) * rtab.size()};
@@ -142,8 +144,9 @@ struct BatchImage {
     auto put = [&](int s, const void* src, size_t n) {
       if (n) std::memcpy(out.data() + off[s], src, n);
     };
-    put(kOne, one.data(), sizeof(BatchOneOp) * one.size());
-    put(kOneBegin, one_begin.data(), sizeof(uint32_t) * one_begin.size());
+    put(kOne, one.data(), sizeof(OneLane) * one.size());
+    put(kOneRows, one_rows.data(), sizeof(OneRow) * one_rows.size());
+    put(kOneIndex, one_index.data(), sizeof(OneIndex) * one_index.size());
     put(kOneBlocks, one_block.data(), sizeof(uint32_t) * one_block.size());
     put(kBox, b2.data(), sizeof(BatchOpDev) * b2.size());
     put(kRC, r2.data(), sizeof(BatchRCOpDev) * r2.size());
@@ -356,26 +359,35 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
     if (r.ntiles == 0) continue;
     const ttc_batch_op_t& op = ops[r.src];
     const ttc_plan_s* use = variant_for(bp.plans[r.src], op.A, op.B);
-    BatchOneOp d;
-    std::memset(&d, 0, sizeof(d));
+    OneIndex at = {(uint32_t)one_tiles, 0};
+    const OneHead h = {op.A, op.B, op.alpha, op.beta, r.kind, {0, 0, 0}};
     if (use->family == kFamilyRC) {
-      std::memcpy(&d.p, &use->lane, sizeof(use->lane));
-      d.p.lane.walk.grid_order = 0;  // the launch deals the tiles of all ops out to the XCDs
+      OneLane d;
+      std::memset(&d, 0, sizeof(d));
+      d.h = h;
+      d.p = use->lane;
+      d.p.walk.grid_order = 0;  // the launch deals the tiles of all ops out to the XCDs
       bp.one_lds = std::max(bp.one_lds, use->lane_lds);
+      at.rec = (uint32_t)im.one.size();
+      im.one.push_back(d);
     } else {
-      std::memcpy(&d.p, &use->row1, sizeof(use->row1));
+      const RowParams& q = use->row1;
+      OneRow d;
+      std::memset(&d, 0, sizeof(d));
+      d.h = h;
+      d.p.total = q.total, d.p.nv = q.nv, d.p.n0 = q.n0, d.p.rank = q.rank;
+      d.p.dnv.m = q.dnv.m, d.p.dnv.s = q.dnv.s;
+      for (int k = 0; k < kMaxDim; ++k) {
+        d.p.dn[k].d = q.dn[k].d, d.p.dn[k].m = q.dn[k].m, d.p.dn[k].s = q.dn[k].s;
+        d.p.sa[k] = q.sa[k], d.p.sb[k] = q.sb[k];
+      }
+      at.rec = (uint32_t)im.one_rows.size() | kOneIsRow;
+      im.one_rows.push_back(d);
     }
-    d.A = op.A;
-    d.B = op.B;
-    d.alpha = op.alpha;
-    d.beta = op.beta;
-    d.kind = r.kind;
-    const uint32_t first = (uint32_t)one_tiles;
     one_tiles += r.ntiles;
     if (one_tiles >= (1ull << 31)) return TTC_ERROR_UNSUPPORTED;
-    while ((uint64_t)im.one_block.size() * kOneBlock < one_tiles) im.one_block.push_back((uint32_t)im.one.size());
-    im.one.push_back(d);
-    im.one_begin.push_back(first);
+    while ((uint64_t)im.one_block.size() * kOneBlock < one_tiles) im.one_block.push_back((uint32_t)im.one_index.size());
+    im.one_index.push_back(at);
   }
   bp.one_tiles = (uint32_t)one_tiles;
   bp.tiles += (int64_t)one_tiles;
@@ -492,18 +504,17 @@ static GroupArgs group_args(const BatchPlan& bp, const BatchGroup& g, uintptr_t 
 
 // Arguments of the one-work-group-per-tile launch.
 struct OneArgs {
-  const void* ops;
-  const void* begin;
-  const void* block;
+  const void *lanes, *rows, *index, *block;
   uint32_t nops, ntiles;
 };
 static OneArgs one_args(const BatchPlan& bp, uintptr_t base) {
   const BatchImage& im = bp.img;
   OneArgs a;
-  a.ops = reinterpret_cast<const void*>(base + im.off[BatchImage::kOne]);
-  a.begin = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneBegin]);
+  a.lanes = reinterpret_cast<const void*>(base + im.off[BatchImage::kOne]);
+  a.rows = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneRows]);
+  a.index = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneIndex]);
   a.block = reinterpret_cast<const void*>(base + im.off[BatchImage::kOneBlocks]);
-  a.nops = (uint32_t)im.one.size();
+  a.nops = (uint32_t)im.one_index.size();
   a.ntiles = bp.one_tiles;
   return a;
 }
@@ -511,7 +522,7 @@ static OneArgs one_args(const BatchPlan& bp, uintptr_t base) {
 static ttc_status_t launch_groups(const BatchPlan& bp, uintptr_t base, hipStream_t s) {
   if (bp.one_tiles > 0) {
     OneArgs a = one_args(bp, base);
-    void* args[] = {&a.ops, &a.begin, &a.block, &a.nops, &a.ntiles};
+    void* args[] = {&a.lanes, &a.rows, &a.index, &a.block, &a.nops, &a.ntiles};
     if (hipLaunchKernel(batch_one_func(), dim3(one_grid(bp.one_tiles)), dim3(kThreads), args, (size_t)bp.one_lds,
                         s) != hipSuccess)
       return TTC_ERROR_HIP;
@@ -590,7 +601,7 @@ extern "C" ttc_status_t ttc_batch_graph_launch(ttc_batch_t b, ttc_stream_t strea
       if (hipGraphCreate(&g, 0) != hipSuccess) return TTC_ERROR_HIP;
       if (b->bp.one_tiles > 0) {
         OneArgs a = one_args(b->bp, reinterpret_cast<uintptr_t>(b->d_image));
-        void* args[] = {&a.ops, &a.begin, &a.block, &a.nops, &a.ntiles};
+        void* args[] = {&a.lanes, &a.rows, &a.index, &a.block, &a.nops, &a.ntiles};
         hipKernelNodeParams kp;
         std::memset(&kp, 0, sizeof(kp));
         kp.func = const_cast<void*>(batch_one_func());

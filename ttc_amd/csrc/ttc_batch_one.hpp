@@ -25,27 +25,52 @@ namespace ttc {
 // (index: of the vector width in {1, 2, widest}); kind = type pair * 32 + variant.
 constexpr int kOneVariants = 32, kOneRow = 18, kOneRowUnaligned = 24;
 
-// Op record, 1 KiB: the parameters are read with scalar loads from its front.
-struct alignas(1024) BatchOneOp {
-  union Params {
-    RCLaneParams lane;
-    RowParams row;
-  } p;
+// Op records, read with scalar loads: what both kinds of op have, then the
+// row x column or the row copy's parameters.
+struct OneHead {
   const void* A;
   void* B;
   double alpha, beta;
   int32_t kind;
-  int32_t pad_;
+  int32_t pad_[3];
 };
-static_assert(sizeof(BatchOneOp) == 1024, "one record per KiB of the work table");
-static_assert(std::is_trivially_copyable<RCLaneParams>::value && std::is_trivially_copyable<RowParams>::value,
+struct alignas(1024) OneLane {
+  OneHead h;
+  RCLaneParams p;
+};
+// RowParams without the words row_chunk does not read, so that a work table
+// of the fixed workspace's size holds as many small row copies as it can.
+struct OneRow {
+  OneHead h;
+  struct Params {
+    uint32_t total, nv;
+    int32_t n0, rank;
+    struct {
+      uint32_t m, s;
+    } dnv;
+    struct {
+      uint32_t d, m, s;
+    } dn[kMaxDim];
+    int64_t sa[kMaxDim], sb[kMaxDim];
+  } p;
+};
+static_assert(sizeof(OneLane) == 1024 && sizeof(OneRow) == 296, "bytes per op of the work table");
+static_assert(std::is_trivially_copyable<OneLane>::value && std::is_trivially_copyable<OneRow>::value,
               "records are copied as bytes");
+
+// Per op, in launch order: its first tile, and its record among those of its
+// kind, with kOneIsRow for row copies.
+struct OneIndex {
+  uint32_t first, rec;
+};
+constexpr uint32_t kOneIsRow = 1u << 31;
 
 // Tiles per entry of the table that gives the op a block of tiles starts in.
 constexpr uint32_t kOneBlock = 64;
 
-using KOneOp = const __attribute__((address_space(4))) BatchOneOp;
-using KRow = const __attribute__((address_space(4))) RowParams;
+using KHead = const __attribute__((address_space(4))) OneHead;
+using KOneLane = const __attribute__((address_space(4))) OneLane;
+using KOneRow = const __attribute__((address_space(4))) OneRow;
 
 // The launch's tile of work-group w: rounds of 2048 tiles, in which each XCD
 // takes 256 consecutive ones, so that neighbours meet in one L2 and every XCD
@@ -57,7 +82,7 @@ TTC_HD inline uint32_t one_tile_of(uint32_t w, uint32_t ntiles) {
 }
 
 template <class OP, int W, int I>
-__device__ __forceinline__ void one_variant(KOneOp* o, uint32_t tile, unsigned char* lds) {
+__device__ __forceinline__ void one_variant(KHead* o, uint32_t tile, unsigned char* lds) {
   using TA = typename OP::TA;
   using TB = typename OP::TB;
   constexpr bool BETA = (I & 1) == 0;
@@ -65,7 +90,7 @@ __device__ __forceinline__ void one_variant(KOneOp* o, uint32_t tile, unsigned c
     constexpr int ia = I / 6, ib = (I / 2) % 3;
     if constexpr (index_used(ia, W) && index_used(ib, W))
       RCLane<OP, width_of_index(ia, W), width_of_index(ib, W), BETA, false, 2>::run(
-          (KLane*)&o->p.lane, tile, static_cast<const TA*>(o->A), static_cast<TB*>(o->B), lds,
+          (KLane*)&((KOneLane*)o)->p, tile, static_cast<const TA*>(o->A), static_cast<TB*>(o->B), lds,
           (typename OP::AL)o->alpha, (typename OP::BE)o->beta, [](float) {});
   } else {
     constexpr bool UNAL = I >= kOneRowUnaligned;
@@ -74,13 +99,13 @@ __device__ __forceinline__ void one_variant(KOneOp* o, uint32_t tile, unsigned c
                                : index_used((I - kOneRow) / 2, W);
     if constexpr (used)
       (void)row_chunk<OP, V, BETA ? kModeBeta : kModeBz, UNAL>(
-          *(KRow*)&o->p.row, tile, static_cast<const TA*>(o->A), static_cast<TB*>(o->B), (typename OP::AL)o->alpha,
+          ((KOneRow*)o)->p, tile, static_cast<const TA*>(o->A), static_cast<TB*>(o->B), (typename OP::AL)o->alpha,
           (typename OP::BE)o->beta, 1.0f);
   }
 }
 
 template <class OP, int W>
-__device__ __forceinline__ void one_type(int variant, KOneOp* o, uint32_t tile, unsigned char* lds) {
+__device__ __forceinline__ void one_type(int variant, KHead* o, uint32_t tile, unsigned char* lds) {
   switch (variant) {
 #define TTC_ONE(I) \
   case I: one_variant<OP, W, I>(o, tile, lds); break;
@@ -92,11 +117,12 @@ __device__ __forceinline__ void one_type(int variant, KOneOp* o, uint32_t tile, 
   }
 }
 
-// begin: first tile of each op (nops entries); block: the op that holds tile
-// kOneBlock * i, per i.
+// lanes, rows: the records; index: the ops, by kind; block: the op that holds
+// tile kOneBlock * i, per i.
 __global__ void __launch_bounds__(kThreads)
-    batch_one_kernel(const BatchOneOp* __restrict__ ops, const uint32_t* __restrict__ begin,
-                     const uint32_t* __restrict__ block, uint32_t nops, uint32_t ntiles);
+    batch_one_kernel(const OneLane* __restrict__ lanes, const OneRow* __restrict__ rows,
+                     const OneIndex* __restrict__ index, const uint32_t* __restrict__ block, uint32_t nops,
+                     uint32_t ntiles);
 
 // Defined in ttc_batch_k_one.hip.
 const void* batch_one_func();
