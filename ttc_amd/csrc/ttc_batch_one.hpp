@@ -6,7 +6,7 @@
 // Bound by HBM on large ops, by the one launch's latency on small ones.
 // Against one persistent kernel per (family, type), one after the other on
 // the stream: 26 ops of up to 0.3 MiB 54 -> 8 us, 30 ops of up to 2.2 MiB (17
-// MB) 59 -> 18 us, 64 ops of up to 64 MiB (1.03 GB) 327 -> 223 us.
+// MB) 59 -> 17 us, 64 ops of up to 64 MiB (1.03 GB) 327 -> 212 us.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -7,12 +7,12 @@
 // written back once; work-groups that stride over many tiles each (the
 // pipelined kernel of ttc_rc.hpp) drift apart and lose that.  Time per
 // launch, pipelined -> one tile per work-group (copy of 200 MiB: 5.5 TB/s):
-//   fp32 6507 x 8057, padded              110 -> 95 us  (4.4 TB/s)
-//   fp32 rank 6, odd extents, 200 MiB     131 -> 103    (4.1)
-//   fp64 rank 5, beta = 1, 200 MiB        133 -> 117    (5.4)
-//   fp32 -> bf16 rank 4 with beta, 2.4 GB 1129 -> 980   (4.9)
-//   complex64 96 x 80 x 110               6.3 -> 5.3
-//   fp64 37 x 21 x 19 x 5, beta = 1       7.5 -> 5.0
+//   fp32 6507 x 8057, padded              110 -> 94 us  (4.5 TB/s)
+//   fp32 rank 6, odd extents, 200 MiB     131 -> 102    (4.1)
+//   fp64 rank 5, beta = 1, 200 MiB        133 -> 118    (5.3)
+//   fp32 -> bf16 rank 4 with beta, 2.4 GB 1129 -> 950   (5.1)
+//   complex64 96 x 80 x 110               6.3 -> 4.9
+//   fp64 37 x 21 x 19 x 5, beta = 1       7.5 -> 4.4 (in few bytes of arguments)
 //
 // Each lane keeps one vector of rows for the whole read walk and one vector
 // of columns for the whole write walk (RCLaneParams), for any row and column
