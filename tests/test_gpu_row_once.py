@@ -43,3 +43,35 @@ def test_row_lengths_fp8(gpu, tA, tB):
         rt.Plan(tA, tB, [0, 2, 1], size, beta_is_zero=True).execute_fp8(dA, dB, 0.5, scale=3.5, amax_out=amax)
         torch.cuda.synchronize()
         assert same_bits(dB.cpu().numpy(), want) and float(amax.item()) == want_amax, (tA, tB, n0)
+
+
+@pytest.mark.parametrize("n", [2 ** 31 - 1, 2 ** 31 - 7])
+def test_rows_of_almost_2_31_elements(gpu, n):
+    """One row whose vectors end within a vector of 2^31: every element, and
+    nothing behind the row."""
+    import torch
+    from ttc_amd import runtime as rt
+    A = torch.randn(n, dtype=torch.bfloat16, device=gpu)
+    B = torch.full((n + 64,), 3.0, dtype=torch.bfloat16, device=gpu)
+    step = 1 << 28
+    rt.Plan(BF16, BF16, [0], [n], beta_is_zero=True).execute(A, B, 1.0, 0.0)
+    torch.cuda.synchronize()
+    assert torch.equal(B[:n], A) and bool((B[n:] == 3.0).all())
+    rt.Plan(BF16, BF16, [0], [n]).execute(A, B, 1.0, 0.5)
+    torch.cuda.synchronize()
+    for i in range(0, n, step):
+        a = A[i:min(i + step, n)].float()
+        assert torch.equal(B[i:min(i + step, n)], (a + 0.5 * a).to(torch.bfloat16)), i
+    assert bool((B[n:] == 3.0).all())
+    del B
+    Q = torch.full((n + 64,), 7, dtype=torch.uint8, device=gpu)
+    amax = torch.zeros(1, device=gpu)
+    rt.Plan(BF16, E4M3, [0], [n], beta_is_zero=True).execute_fp8(A, Q, 1.0, scale=32.0, amax_out=amax)
+    torch.cuda.synchronize()
+    top = 0.0
+    for i in range(0, n, step):
+        a = A[i:min(i + step, n)].float()
+        top = max(top, float(a.abs().max()))
+        want = (a * 32.0).clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8)
+        assert torch.equal(Q[i:min(i + step, n)], want), i
+    assert bool((Q[n:] == 7).all()) and float(amax) == top

@@ -238,6 +238,12 @@ constexpr int rc_elems(int bytes) { return 128 / bytes > 32 ? 32 : 128 / bytes; 
 // order, and each lane moves one vector of V elements of dimension 0.
 constexpr int kRowUnroll = 4;  // vectors in flight per lane in the row-copy kernel
 
+// Rows of n0 >= v elements in unaligned vectors of v: vectors per row, and how
+// far the one that would start at element e is shifted back to end with its
+// row.  n0 may lie within v of 2^31: neither n0 + v nor e + v fits an int32.
+TTC_HD inline uint32_t row_vectors(int32_t n0, int32_t v) { return ((uint32_t)n0 + (uint32_t)v - 1u) / (uint32_t)v; }
+TTC_HD inline int32_t row_shift(int32_t e, int32_t v, int32_t n0) { return e > n0 - v ? e - (n0 - v) : 0; }
+
 struct RowParams {
   uint32_t total;         // rows * nv (< 2^31)
   uint32_t nv;            // vectors per row: extent of dimension 0 / V (rounded up on unaligned vectors)

@@ -1023,7 +1023,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
     const uint32_t rows = pl->row.total / pl->row.nv;
     pl->row1_v = w;
     pl->row1_unaligned = 1;
-    pl->row1.nv = (uint32_t)((n0 + w - 1) / w);
+    pl->row1.nv = row_vectors(n0, w);  // rows * nv stays below 2^31: w >= 2 v
     pl->row1.dnv = make_fastdiv(pl->row1.nv);
     pl->row1.total = rows * pl->row1.nv;
   }

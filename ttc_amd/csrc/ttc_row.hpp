@@ -159,7 +159,7 @@ __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typenam
     int32_t e = (int32_t)(gg - row * p.nv) * V;
     skip[u] = 0;
     if constexpr (UNAL) {
-      skip[u] = e + V > p.n0 ? e + V - p.n0 : 0;
+      skip[u] = row_shift(e, V, p.n0);
       e -= skip[u];
     }
     int64_t xa = (int64_t)e * (int64_t)sizeof(TA), xb = (int64_t)e * (int64_t)sizeof(TB);
