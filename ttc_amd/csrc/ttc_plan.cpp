@@ -201,15 +201,17 @@ int max_tile_volume(int ta, int tb, int va, int vb) {
 }
 
 // -------------------------------------------------------------- tile choice
-static int round_up(int x, int m) { return (x + m - 1) / m * m; }
+// Tiles of t along an extent n (n + t may pass 2^31).
+static long long tiles_of(long long n, long long t) { return (n + t - 1) / t; }
+
+static int round_up(int x, int m) { return (int)(tiles_of(x, m) * m); }
 
 // Split extent n into pieces of about `want`, balanced so the last piece is
 // not a sliver, then rounded up to `align` (which divides n).
 static int split_extent(int n, int want, int align) {
   want = std::max(want, 1);
   if (want >= n) return n;
-  const int pieces = (n + want - 1) / want;
-  int t = (n + pieces - 1) / pieces;
+  int t = (int)tiles_of(n, tiles_of(n, want));
   t = round_up(t, align);
   return std::min(t, n);
 }
@@ -330,7 +332,7 @@ double tile_score(const Geometry& g, const int* tile, int szA, int szB) {
   long long V = 1, ntiles = 1;
   for (int k = 0; k < g.rank; ++k) {
     V *= tile[k];
-    ntiles *= (g.size[k] + tile[k] - 1) / std::max(tile[k], 1);
+    ntiles *= tiles_of(g.size[k], std::max(tile[k], 1));
   }
   if (V <= 0 || ntiles <= 0) return 0.0;
   long long ra, rb;
@@ -405,7 +407,7 @@ ttc_status_t build_params(const Geometry& g, const int* tile, int ta, int tb, in
     p.tsa[k] = (int64_t)t * g.sa[k];
     p.tsb[k] = (int64_t)t * g.sb[k];
     p.tdiv[k] = make_fastdiv((uint32_t)t);
-    const long long gk = n > 0 ? (n + t - 1) / t : 1;
+    const long long gk = n > 0 ? tiles_of(n, t) : 1;
     ntiles *= gk;
     if (ntiles > INT_MAX) return TTC_ERROR_UNSUPPORTED;
     p.gdiv[k] = make_fastdiv((uint32_t)gk);
@@ -574,7 +576,7 @@ ttc_status_t build_rc_params(const Geometry& g, const int* tile, int ta, int tb,
     if (t < 1 || (n > 0 && t > n)) return TTC_ERROR_INVALID_VALUE;
     spanA += (long long)(t - 1) * g.sa[k];
     spanB += (long long)(t - 1) * g.sb[k];
-    gk[k] = n > 0 ? (n + t - 1) / t : 1;
+    gk[k] = n > 0 ? tiles_of(n, t) : 1;
     if (n == 0) ntiles = 0;
     ntiles *= gk[k];
     if (ntiles > INT_MAX) return TTC_ERROR_UNSUPPORTED;
@@ -685,7 +687,7 @@ ttc_status_t build_rc_params(const Geometry& g, const int* tile, int ta, int tb,
   long long gi = 1, outer = 1;
   if (kg >= 0) {
     gi = std::min<long long>(G, gk[kg]);
-    outer = (gk[kg] + gi - 1) / gi;
+    outer = tiles_of(gk[kg], gi);
     const int pos = p.grank++;
     p.n[pos] = outer > 1 ? (int32_t)(gi * tile[kg]) : g.size[kg];  // never partial when split
     p.t[pos] = tile[kg];
@@ -760,7 +762,7 @@ static bool lane_fit(const Geometry& g, const int* tile, int szA, int szB, int v
   for (int m = 0; m < f.nb; ++m) f.C *= tile[f.gb[m]];
   for (int k = 0; k < g.rank; ++k) {
     if (tile[k] < 1 || tile[k] > g.size[k]) return false;
-    f.ntiles *= (g.size[k] + tile[k] - 1) / tile[k];
+    f.ntiles *= tiles_of(g.size[k], tile[k]);
     if (f.ntiles > kLaneMaxTiles) return false;
   }
   const long long la = f.R / va, lb = f.C / vb, nia = rc_elems(szA) / va / div, nib = rc_elems(szB) / vb / div;
@@ -794,7 +796,7 @@ bool build_lane_params(const Geometry& g, const int* tile, int ta, int tb, int v
   const long long R = f.R, C = f.C, Rl = f.Rl, Cl = f.Cl, kA = f.kA, kB = f.kB;
   const long long la = R / va, lb = C / vb, nia = rc_elems(szA) / va / div, nib = rc_elems(szB) / vb / div;
   long long gk[kMaxDim];
-  for (int k = 0; k < g.rank; ++k) gk[k] = (g.size[k] + tile[k] - 1) / tile[k];
+  for (int k = 0; k < g.rank; ++k) gk[k] = tiles_of(g.size[k], tile[k]);
   p.R = (int32_t)R;
   p.C = (int32_t)C;
   p.Rl = (int32_t)Rl;
@@ -962,7 +964,7 @@ bool build_lane_small(const Geometry& g, const int* tile, int ta, int tb, int ti
   std::memset(&p, 0, sizeof(p));
   for (int m = 0; m < n; ++m) {
     const int k = dims[m];
-    const long long tiles = (g.size[k] + tile[k] - 1) / tile[k], sa = g.sa[k] * szA, sb = g.sb[k] * szB;
+    const long long tiles = tiles_of(g.size[k], tile[k]), sa = g.sa[k] * szA, sb = g.sb[k] * szB;
     if (tiles > 65535 || tile[k] > 65535 || sa > INT_MAX || sb > INT_MAX) return false;
     p.dim[m] = RCSmallDim{(int32_t)sa, (int32_t)sb, (uint16_t)tile[k], (uint16_t)tiles};
   }
