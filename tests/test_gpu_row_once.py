@@ -75,3 +75,31 @@ def test_rows_of_almost_2_31_elements(gpu, n):
         want = (a * 32.0).clamp(-448.0, 448.0).to(torch.float8_e4m3fn).view(torch.uint8)
         assert torch.equal(Q[i:min(i + step, n)], want), i
     assert bool((Q[n:] == 7).all()) and float(amax) == top
+
+
+@pytest.mark.parametrize("code", ["s", "d", "c", "b", "h"])
+def test_scaling_in_place(gpu, code):
+    """An identity permutation whose A is its B: rows that are no whole number
+    of vectors, dense and padded, alone, misaligned and in a grouped launch."""
+    import torch
+    from common import from_device, make_case, oracle_run
+    from ttc_amd import runtime as rt
+    t, _ = CODE[code]
+    for n0 in (3, 9, 127, 100003):
+        for size, ld in (([n0], None), ([n0, 41], [n0 + 2, 41])):
+            perm = list(range(len(size)))
+            for beta in (0.0, 0.5):
+                A, _ = make_case(t, t, perm, size, ld, ld, seed=n0)
+                want = oracle_run(t, t, A, A, 1.25, beta, perm, size, ld, ld)
+                plan = rt.Plan(t, t, perm, size, ld, ld, beta == 0.0)
+                for off in (0, A.itemsize):
+                    X = torch.zeros(A.nbytes + off, dtype=torch.uint8, device=gpu)
+                    X[off:] = to_device(A, gpu)
+                    plan.execute(X.data_ptr() + off, X.data_ptr() + off, 1.25, beta)
+                    torch.cuda.synchronize()
+                    assert same_bits(X[off:].cpu().numpy().view(A.dtype), want), (code, size, ld, beta, off)
+                X = to_device(A, gpu)
+                rt.Batch([dict(type_a=t, perm=perm, size=size, lda=ld, ldb=ld, alpha=1.25, beta=beta, A=X,
+                               B=X)]).execute()
+                torch.cuda.synchronize()
+                assert same_bits(from_device(X, A), want), (code, size, ld, beta, "grouped")

@@ -295,13 +295,13 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       int variant = -1;
       if (use->family == kFamilyRC && use->lane_div == 2)
         variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
-      else if (use->family == kFamilyRow && use->row1_unaligned)
-        variant = kOneRowUnaligned + __builtin_ctz((unsigned)use->row1_v) * 2 + bz;
-      else if (use->family == kFamilyRow)
-        variant = kOneRow + index_of_width(use->row1_v, wide) * 2 + bz;
+      const RowChunks c = use->family == kFamilyRow ? row_chunks(use, op.A, op.B) : RowChunks{};
+      if (use->family == kFamilyRow)
+        variant = c.unaligned ? kOneRowUnaligned + __builtin_ctz((unsigned)c.v) * 2 + bz
+                              : kOneRow + index_of_width(c.v, wide) * 2 + bz;
       if (variant >= 0) {
         r.kind = pair * kOneVariants + variant;
-        r.ntiles = pl->g.elements == 0 ? 0 : (use->family == kFamilyRC ? use->lane.walk.ntiles : use->row1_grid);
+        r.ntiles = pl->g.elements == 0 ? 0 : (use->family == kFamilyRC ? use->lane.walk.ntiles : c.grid);
         r.weight = 0.0;
         bp.bytes += pl->g.elements * (sa + sb * (bz ? 1 : 2));
         continue;
@@ -371,7 +371,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       at.rec = (uint32_t)im.one.size();
       im.one.push_back(d);
     } else {
-      const RowParams& q = use->row1;
+      const RowParams& q = *row_chunks(use, op.A, op.B).p;
       OneRow d;
       std::memset(&d, 0, sizeof(d));
       d.h = h;

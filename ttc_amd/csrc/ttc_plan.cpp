@@ -1005,6 +1005,22 @@ bool build_row_small(const RowParams& full, unsigned grid, RowSmall& p) {
   return true;
 }
 
+static unsigned row_chunk_count(const RowParams& p, int szA, int szB, int v, bool fp8, bool unaligned) {
+  const long long chunk = (long long)kThreads * row_once_unroll(szA, szB, v, fp8, unaligned);
+  return (unsigned)((p.total + chunk - 1) / chunk);
+}
+
+// With beta == 0 the unaligned vectors at a row's end overlap and both write
+// what they have read: in place (A == B, an identity permutation that scales)
+// one of them could read what the other has written.  Aligned vectors do not
+// overlap.
+RowChunks row_chunks(const ttc_plan_s* use, const void* A, const void* B) {
+  if (!(A == B && use->beta_is_zero && use->row1_unaligned))
+    return RowChunks{&use->row1, use->row1_v, use->row1_unaligned != 0, use->row1_grid};
+  const int szA = dtype_bytes(use->type_a), szB = dtype_bytes(use->type_b);
+  return RowChunks{&use->row, use->va, false, row_chunk_count(use->row, szA, szB, use->va, szB == 1, false)};
+}
+
 // The one-chunk-per-work-group launch of row copy p (aligned vectors of v
 // elements): unaligned vectors where they are wider.  Rows shorter than a
 // cache line share lines with their neighbours in A and B, which then meet in
@@ -1043,8 +1059,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
       pl->row1.sb[k - 1] = g.sb[k] * szB;
     }
   pl->row1.xcd_share = (long long)n0 * std::min(szA, szB) < 128;
-  const long long chunk = (long long)kThreads * row_once_unroll(szA, szB, pl->row1_v, fp8, pl->row1_unaligned != 0);
-  pl->row1_grid = (unsigned)((pl->row1.total + chunk - 1) / chunk);
+  pl->row1_grid = row_chunk_count(pl->row1, szA, szB, pl->row1_v, fp8, pl->row1_unaligned != 0);
   pl->small = !fp8 && build_row_small(pl->row1, pl->row1_grid, pl->row_small);
 }
 

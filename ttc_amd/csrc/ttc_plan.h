@@ -169,3 +169,16 @@ struct ttc_plan_s {
   ttc::RowSmall row_small;
   ttc_plan_s* fallback;  // scalar-vector plan for misaligned pointers (may be null)
 };
+
+namespace ttc {
+
+// The row copy's launch of one chunk per work-group on the given buffers.
+struct RowChunks {
+  const RowParams* p;
+  int v;
+  bool unaligned;
+  unsigned grid;  // chunks
+};
+RowChunks row_chunks(const ttc_plan_s* use, const void* A, const void* B);
+
+}  // namespace ttc

@@ -125,13 +125,13 @@ static ttc_status_t launch_row_chunks(const ttc_plan_s* use, const KernelEntry* 
                                       double alpha, double beta, const float* scale_in, const float* amax_in,
                                       float fp8_max, float scale, float* amax_out, float* scale_inv_out,
                                       hipStream_t s) {
-  if (use->row1_unaligned)
-    e = find_kernel(use->type_a, use->type_b, use->row1_v, use->row1_v, mode, kFamRowUnaligned);
+  const RowChunks c = row_chunks(use, A, B);
+  if (c.unaligned) e = find_kernel(use->type_a, use->type_b, c.v, c.v, mode, kFamRowUnaligned);
   if (!e) return TTC_ERROR_UNSUPPORTED;
-  if (use->small && mode != kModeFp8)
+  if (use->small && mode != kModeFp8 && c.p == &use->row1)
     return e->launch_row_small(use->row_small, A, B, alpha, beta, s) == hipSuccess ? TTC_SUCCESS : TTC_ERROR_HIP;
-  return e->launch_row_once(use->row1, A, B, alpha, beta, scale_in, amax_in, fp8_max, scale, amax_out, scale_inv_out,
-                            use->row1_grid, s) == hipSuccess
+  return e->launch_row_once(*c.p, A, B, alpha, beta, scale_in, amax_in, fp8_max, scale, amax_out, scale_inv_out,
+                            c.grid, s) == hipSuccess
              ? TTC_SUCCESS
              : TTC_ERROR_HIP;
 }
