@@ -3,7 +3,8 @@
 // elements and of the last extents below 2^31: the vectors of a row, shifted as
 // the kernel shifts the last one, start inside the row, follow each other
 // without a gap and end with the row; the chunks cover all vectors, whose count
-// stays below 2^31.  Prints one summary line; exit status 1 on a violation.
+// stays below 2^31; and the launch in few bytes of arguments, where there is
+// one, takes every vector to the same row.  Prints one summary line; exit status 1 on a violation.
 #include <climits>
 #include <cstdio>
 
@@ -20,7 +21,8 @@ using namespace ttc;
     }                                                                                                            \
   } while (0)
 
-static bool check_row(const ttc_plan_s* pl, int ta, int tb, int beta, int n0, long long rows, long long& unaligned) {
+static bool check_row(const ttc_plan_s* pl, int ta, int tb, int beta, int n0, long long rows, long long& unaligned,
+                      long long& small) {
   const RowParams& p = pl->row1;
   const long long V = pl->row1_v, nv = p.nv;
   CHECK(pl->family == kFamilyRow && p.n0 == n0);
@@ -42,6 +44,26 @@ static bool check_row(const ttc_plan_s* pl, int ta, int tb, int beta, int n0, lo
     if (i > 0) CHECK(start(i) > start(i - 1) && start(i) <= start(i - 1) + V);
   }
   CHECK(start(nv - 1) + V == n0);
+  // the few-byte form of the launch stands for the same rows
+  if (pl->small) {
+    const RowSmall& q = pl->row_small;
+    CHECK(p.total < kSmallCount && q.total == p.total && q.nv == p.nv && q.n0 == p.n0 && q.rank == p.rank);
+    CHECK((q.xcd_share != 0) == (p.xcd_share != 0) && q.grid == pl->row1_grid);
+    for (uint32_t i = 0; i < p.total; ++i) {
+      const uint32_t row = fdiv(i, p.nvm, p.nvs);
+      CHECK(row == i / p.nv && sdiv(i, q.nv) == row);
+      uint32_t rem = row, rem2 = row;
+      for (int k = 0; k < p.rank; ++k) {
+        const uint32_t x = rem % p.dn[k].d, d2 = sdiv(rem2, q.dim[k].d), x2 = rem2 - d2 * q.dim[k].d;
+        CHECK(fdiv(rem, p.dn[k].m, p.dn[k].s) == rem / p.dn[k].d && x == x2);
+        CHECK(p.sa[k] == q.dim[k].sa && p.sb[k] == q.dim[k].sb);
+        rem /= p.dn[k].d;
+        rem2 = d2;
+      }
+      CHECK(rem == 0 && rem2 == 0);
+    }
+    ++small;
+  }
   const int szA = dtype_bytes(ta), szB = dtype_bytes(tb);
   const long long chunk = 256ll * row_once_unroll(szA, szB, (int)V, szB == 1, pl->row1_unaligned != 0);
   CHECK(pl->row1_grid * chunk >= (long long)p.total && (pl->row1_grid - 1) * chunk < (long long)p.total);
@@ -49,7 +71,7 @@ static bool check_row(const ttc_plan_s* pl, int ta, int tb, int beta, int n0, lo
 }
 
 int main() {
-  long long plans = 0, unaligned = 0, last = 0;
+  long long plans = 0, unaligned = 0, last = 0, small = 0;
   for (int ta = 0; ta < 8; ++ta)
     for (int tb = 0; tb < 8; ++tb) {
       if (!pair_supported(ta, tb)) continue;
@@ -71,7 +93,7 @@ int main() {
               return std::fprintf(stderr, "FAIL plan %d %d %d\n", ta, tb, n0), 1;
             for (const ttc_plan_s* q : {(const ttc_plan_s*)pl, (const ttc_plan_s*)pl->fallback})
               if (q) {
-                if (!check_row(q, ta, tb, beta, c.n0, c.rows, unaligned)) return 1;
+                if (!check_row(q, ta, tb, beta, c.n0, c.rows, unaligned, small)) return 1;
                 ++plans;
                 last += huge && q->row1_unaligned;
               }
@@ -80,6 +102,6 @@ int main() {
         }
       }
     }
-  std::printf("%lld plans, %lld unaligned, %lld of them near 2^31\n", plans, unaligned, last);
+  std::printf("%lld plans, %lld unaligned, %lld of them near 2^31, %lld in few bytes\n", plans, unaligned, last, small);
   return 0;
 }

@@ -19,5 +19,5 @@ def test_row_vectors_cover_each_row(tmp_path):
         pytest.fail("g++ failed:\n" + p.stdout)
     r = subprocess.run([exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
     assert r.returncode == 0, r.stdout
-    plans, unaligned, last = [int(w) for w in r.stdout.replace(",", " ").split() if w.isdigit()][:3]
-    assert plans > 5000 and unaligned > 1000 and last > 100, r.stdout
+    plans, unaligned, last, small = [int(w) for w in r.stdout.replace(",", " ").split() if w.isdigit()][:4]
+    assert plans > 5000 and unaligned > 1000 and last > 100 and small > 1000, r.stdout

@@ -371,16 +371,10 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       at.rec = (uint32_t)im.one.size();
       im.one.push_back(d);
     } else {
-      const RowParams& q = *row_chunks(use, op.A, op.B).p;
       OneRow d;
       std::memset(&d, 0, sizeof(d));
       d.h = h;
-      d.p.total = q.total, d.p.nv = q.nv, d.p.n0 = q.n0, d.p.rank = q.rank;
-      d.p.dnv.m = q.dnv.m, d.p.dnv.s = q.dnv.s;
-      for (int k = 0; k < kMaxDim; ++k) {
-        d.p.dn[k].d = q.dn[k].d, d.p.dn[k].m = q.dn[k].m, d.p.dn[k].s = q.dn[k].s;
-        d.p.sa[k] = q.sa[k], d.p.sb[k] = q.sb[k];
-      }
+      d.p = *row_chunks(use, op.A, op.B).p;
       at.rec = (uint32_t)im.one_rows.size() | kOneIsRow;
       im.one_rows.push_back(d);
     }

@@ -38,25 +38,18 @@ struct alignas(1024) OneLane {
   OneHead h;
   RCLaneParams p;
 };
-// RowParams without the words row_chunk does not read, so that a work table
-// of the fixed workspace's size holds as many small row copies as it can.
+// (RowWalk alone, so that a work table of the fixed workspace's size holds as
+// many small row copies as it can.)
 struct OneRow {
   OneHead h;
-  struct Params {
-    uint32_t total, nv;
-    int32_t n0, rank;
-    struct {
-      uint32_t m, s;
-    } dnv;
-    struct {
-      uint32_t d, m, s;
-    } dn[kMaxDim];
-    int64_t sa[kMaxDim], sb[kMaxDim];
-  } p;
+  RowWalk p;
 };
 static_assert(sizeof(OneLane) == 1024 && sizeof(OneRow) == 296, "bytes per op of the work table");
+// Parameter records enter the table whole and are read in place: no field can
+// be left behind.
 static_assert(std::is_trivially_copyable<OneLane>::value && std::is_trivially_copyable<OneRow>::value,
               "records are copied as bytes");
+static_assert(std::is_base_of<RowWalk, RowParams>::value, "a row copy's record is a slice of its parameters");
 
 // Per op, in launch order: its first tile, and its record among those of its
 // kind, with kOneIsRow for row copies.

@@ -22,6 +22,8 @@
 // few KB: a small launch waits for its instructions, so straight-line code
 // for every case would cost more than it saves.
 #pragma once
+#include <type_traits>
+
 #include "ttc_rc.hpp"
 
 namespace ttc {
@@ -36,16 +38,12 @@ struct LaneFull {
   // offsets of tile `wg`'s origin (elements here; what `at` adds), and which
   // groups are partial
   __device__ __forceinline__ uint32_t origin(uint32_t wg, int64_t& bA, int64_t& bB) const {
-    RCWalk w;
-    w.ntiles = kp->walk.ntiles;
-    w.grid_order = kp->walk.grid_order;
-    w.bandw = kp->walk.bandw;
-    w.bandn = kp->walk.bandn;
-    w.bandin = kp->walk.bandin;
-    w.dper = FastDiv{kp->walk.dper.d, kp->walk.dper.m, kp->walk.dper.s, 0};
-    w.dband = FastDiv{kp->walk.dband.d, kp->walk.dband.m, kp->walk.dband.s, 0};
-    w.dw = FastDiv{kp->walk.dw.d, kp->walk.dw.m, kp->walk.dw.s, 0};
-    w.dwl = FastDiv{kp->walk.dwl.d, kp->walk.dwl.m, kp->walk.dwl.s, 0};
+    RCWalk w;  // copied whole, as 32-bit words: no field can be left behind
+    static_assert(sizeof(RCWalk) % 4 == 0 && std::is_trivially_copyable<RCWalk>::value, "RCWalk is copied as words");
+    KWord* const s = (KWord*)&kp->walk;
+    uint32_t* const d = reinterpret_cast<uint32_t*>(&w);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(RCWalk) / 4); ++i) d[i] = s[i];
     uint32_t rem = uniform(rc_tile_of(w, wg)), last = 0;
     bA = bB = 0;
     const int gr = kp->grank;

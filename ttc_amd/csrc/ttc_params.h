@@ -52,6 +52,15 @@ TTC_HD inline uint32_t fdiv(uint32_t n, uint32_t m, uint32_t s) {
 }
 TTC_HD inline uint32_t fdiv(uint32_t n, const FastDiv& f) { return fdiv(n, f.m, f.s); }
 
+// FastDiv without its padding.
+struct DivBy {
+  uint32_t d, m, s;
+};
+inline DivBy make_divby(uint32_t d) {
+  const FastDiv f = make_fastdiv(d);
+  return DivBy{f.d, f.m, f.s};
+}
+
 // Work-groups are dispatched round-robin over the 8 XCDs (work-group w runs
 // on XCD w % 8), each XCD with its own L2.
 constexpr uint32_t kXcds = 8;
@@ -244,18 +253,26 @@ constexpr int kRowUnroll = 4;  // vectors in flight per lane in the row-copy ker
 TTC_HD inline uint32_t row_vectors(int32_t n0, int32_t v) { return ((uint32_t)n0 + (uint32_t)v - 1u) / (uint32_t)v; }
 TTC_HD inline int32_t row_shift(int32_t e, int32_t v, int32_t n0) { return e > n0 - v ? e - (n0 - v) : 0; }
 
-struct RowParams {
+// What a work-group needs of its rows: the part of RowParams that a grouped
+// launch's work table holds, assigned whole.
+struct RowWalk {
   uint32_t total;         // rows * nv (< 2^31)
   uint32_t nv;            // vectors per row: extent of dimension 0 / V (rounded up on unaligned vectors)
-  FastDiv dnv;
-  int32_t rank;           // row dimensions, in B order
   int32_t n0;             // extent of dimension 0
-  int32_t xcd_share;      // one chunk per work-group: XCDs take contiguous shares of the chunks
-  int32_t pad_;
-  FastDiv dn[kMaxDim];    // their extents
+  int32_t rank;           // row dimensions, in B order
+  uint32_t nvm, nvs;      // division by nv
+  DivBy dn[kMaxDim];      // their extents
   int64_t sa[kMaxDim];    // A byte strides
   int64_t sb[kMaxDim];    // B byte strides
 };
+struct RowParams : RowWalk {
+  int32_t xcd_share;      // one chunk per work-group: XCDs take contiguous shares of the chunks
+  int32_t pad_;
+};
+inline void row_set_vectors(RowWalk& p, uint32_t rows, uint32_t nv) {
+  const FastDiv f = make_fastdiv(nv);
+  p.total = rows * nv, p.nv = nv, p.nvm = f.m, p.nvs = f.s;
+}
 
 // One row x column tile of a grouped launch: element offsets of its origin
 // in A and B; flags bit 0: last (partial) tile along the row group, bit 1:

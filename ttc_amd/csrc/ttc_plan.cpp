@@ -933,16 +933,14 @@ ttc_status_t build_row_params(const Geometry& g, int ta, int tb, int v, RowParam
   p.rank = g.rank - 1;
   for (int q = 1; q < g.rank; ++q) {
     const int k = g.perm[q];
-    p.dn[q - 1] = make_fastdiv((uint32_t)g.size[k]);
+    p.dn[q - 1] = make_divby((uint32_t)g.size[k]);
     p.sa[q - 1] = g.sa[k] * szA;
     p.sb[q - 1] = g.sb[k] * szB;
     rows *= g.size[k];
   }
   const long long total = rows * nv;
   if (total >= (1ll << 31)) return TTC_ERROR_UNSUPPORTED;
-  p.total = (uint32_t)total;
-  p.nv = (uint32_t)nv;
-  p.dnv = make_fastdiv((uint32_t)nv);
+  row_set_vectors(p, (uint32_t)rows, (uint32_t)nv);
   p.n0 = g.size[0];
   return TTC_SUCCESS;
 }
@@ -1041,9 +1039,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
     const uint32_t rows = pl->row.total / pl->row.nv;
     pl->row1_v = w;
     pl->row1_unaligned = 1;
-    pl->row1.nv = row_vectors(n0, w);  // rows * nv stays below 2^31: w >= 2 v
-    pl->row1.dnv = make_fastdiv(pl->row1.nv);
-    pl->row1.total = rows * pl->row1.nv;
+    row_set_vectors(pl->row1, rows, row_vectors(n0, w));  // still below 2^31: w >= 2 v
   }
   // Rows of whole cache lines share none with their neighbours on either
   // side: walked in A order, whose reads then run on (bf16 128 x 4096 x 32 x 8
@@ -1054,7 +1050,7 @@ static void build_row_once(ttc_plan_s* pl, int v) {
   for (int k = 1; k < g.rank; ++k) lines = lines && g.sa[k] * szA % 128 == 0 && g.sb[k] * szB % 128 == 0;
   if (lines)
     for (int k = 1; k < g.rank; ++k) {
-      pl->row1.dn[k - 1] = make_fastdiv((uint32_t)g.size[k]);
+      pl->row1.dn[k - 1] = make_divby((uint32_t)g.size[k]);
       pl->row1.sa[k - 1] = g.sa[k] * szA;
       pl->row1.sb[k - 1] = g.sb[k] * szB;
     }

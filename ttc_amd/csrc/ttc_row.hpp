@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(kThreads)
       const uint32_t g = g0 + (uint32_t)u * stride;
       ok[u] = g < p.total;
       const uint32_t gg = ok[u] ? g : 0u;
-      const uint32_t row = fdiv(gg, p.dnv);
+      const uint32_t row = fdiv(gg, p.nvm, p.nvs);
       const uint32_t v = gg - row * p.nv;
       int64_t xa = (int64_t)v * (int64_t)(V * sizeof(TA));
       int64_t xb = (int64_t)v * (int64_t)(V * sizeof(TB));
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int k = 0; k < kMaxDim; ++k) {
         if (k < p.rank) {
-          const uint32_t q = fdiv(rem, p.dn[k]);
+          const uint32_t q = fdiv(rem, p.dn[k].m, p.dn[k].s);
           const uint32_t x = rem - q * p.dn[k].d;
           rem = q;
           xa += (int64_t)x * p.sa[k];
@@ -125,8 +125,8 @@ template <class T, int V> struct __attribute__((packed, aligned(sizeof(T)))) Row
 // copy 4740 -> 6010; bf16 128 x 4096 x 32 x 8 perm (0,2,1,3) 4760 -> 5340;
 // fp32 rows of 127 3890 -> 4730, of 5 2210 -> 3040; bf16 rows of 127
 // 2180 -> 4070, of 5 1270 -> 2240.
-// P: RowParams as a kernel argument or in a grouped launch's work table, or
-// RowSmall.
+// P: RowParams as a kernel argument, RowWalk in a grouped launch's work table,
+// or RowSmall.
 // Returns max |alpha * a| of this lane's elements (fp8 casts).
 template <class OP, int V, int MODE, bool UNAL, class P>
 __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typename OP::TA* __restrict__ A,
@@ -155,7 +155,7 @@ __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typenam
     const uint32_t gg = ok[u] ? g : 0u;
     uint32_t row;
     if constexpr (kSmall) row = sdiv(gg, p.nv);
-    else row = fdiv(gg, p.dnv.m, p.dnv.s);
+    else row = fdiv(gg, p.nvm, p.nvs);
     int32_t e = (int32_t)(gg - row * p.nv) * V;
     skip[u] = 0;
     if constexpr (UNAL) {
