@@ -92,10 +92,9 @@ struct BatchGroup {
   int lds_bytes;
 };
 
-// Host copy of a batch's device work table.  Its sections (box op records,
-// row x column op records, work-group slices, box tile records, row x
-// column tile records, offset tables) sit 256-byte aligned in one image, so
-// that one allocation (or the fixed workspace) and one copy hold all of it;
+// Host copy of a batch's device work table.  Its sections sit
+// kTableAlign-aligned in one image, so that one allocation (or the fixed
+// workspace) and one copy hold all of it;
 // op records point at their tile records once the image's device address is
 // known (render).
 struct BatchImage {
@@ -125,7 +124,7 @@ struct BatchImage {
     size_t o = 0;
     for (int s = 0; s < kSections; ++s) {
       off[s] = o;
-      o += (len[s] + 255) / 256 * 256;
+      o += (len[s] + kTableAlign - 1) / kTableAlign * kTableAlign;
     }
     bytes = o;
   }
@@ -657,7 +656,7 @@ extern "C" ttc_status_t ttc_batch_destroy(ttc_batch_t b) {
 // `scratch` is only a stand-in, never a device address: scratch_address()
 // looks up the current device's copy once (hipGetSymbolAddress) and all
 // later uses (the table copy, the kernels' arguments) go through that.
-static __device__ __align__(256) unsigned char scratch[TTC_BATCH_WORKSPACE_BYTES];
+static __device__ __align__(kTableAlign) unsigned char scratch[TTC_BATCH_WORKSPACE_BYTES];
 
 static constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;

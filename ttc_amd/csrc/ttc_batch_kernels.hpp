@@ -35,6 +35,10 @@ __host__ __device__ constexpr bool index_used(int idx, int W) {
   return idx == 0 || (idx == 1 && W > 2) || (idx == 2 && W > 1);
 }
 
+// A work table's sections start at multiples of this, in memory from
+// hipMalloc and in the fixed workspace.
+constexpr size_t kTableAlign = 256;
+
 struct BatchOpDev {
   TileParams p;
   const void* A;

@@ -34,9 +34,11 @@ struct OneHead {
   int32_t kind;
   int32_t pad_[3];
 };
-struct alignas(1024) OneLane {
+// (1 KiB each, so that no record shares a line with another.)
+struct alignas(64) OneLane {
   OneHead h;
   RCLaneParams p;
+  unsigned char pad_[1024 - sizeof(OneHead) - sizeof(RCLaneParams)];
 };
 // (RowWalk alone, so that a work table of the fixed workspace's size holds as
 // many small row copies as it can.)
@@ -44,19 +46,21 @@ struct OneRow {
   OneHead h;
   RowWalk p;
 };
-static_assert(sizeof(OneLane) == 1024 && sizeof(OneRow) == 296, "bytes per op of the work table");
-// Parameter records enter the table whole and are read in place: no field can
-// be left behind.
-static_assert(std::is_trivially_copyable<OneLane>::value && std::is_trivially_copyable<OneRow>::value,
-              "records are copied as bytes");
-static_assert(std::is_base_of<RowWalk, RowParams>::value, "a row copy's record is a slice of its parameters");
-
 // Per op, in launch order: its first tile, and its record among those of its
 // kind, with kOneIsRow for row copies.
 struct OneIndex {
   uint32_t first, rec;
 };
 constexpr uint32_t kOneIsRow = 1u << 31;
+
+static_assert(sizeof(OneLane) == 1024 && sizeof(OneRow) == 296, "bytes per op of the work table");
+static_assert(alignof(OneLane) <= kTableAlign && alignof(OneRow) <= kTableAlign && alignof(OneIndex) <= kTableAlign,
+              "the sections of a work table start at multiples of kTableAlign");
+// Parameter records enter the table whole and are read in place: no field can
+// be left behind.
+static_assert(std::is_trivially_copyable<OneLane>::value && std::is_trivially_copyable<OneRow>::value,
+              "records are copied as bytes");
+static_assert(std::is_base_of<RowWalk, RowParams>::value, "a row copy's record is a slice of its parameters");
 
 // Tiles per entry of the table that gives the op a block of tiles starts in.
 constexpr uint32_t kOneBlock = 64;
