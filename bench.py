@@ -46,24 +46,26 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def kernel_name(info):
+def kernel_name(plan):
     """The kernel a plan launches, spelled as rocprof shows its template
-    (ttc::<family kernel><Op, VA, VB, BETA, NT[, FAST or DIV]>)."""
+    (ttc::<kernel><Op, VA, VB, BETA, NT[, FAST or DIV]>, row copies ttc::
+    <kernel><Op, V, MODE[, UNAL]>)."""
+    from ttc_amd import runtime as rt
+    info, launch = plan.info(), plan.launch()
     ops = {(0, 0): "ttc::OpF32<float, float>", (1, 1): "ttc::OpDD"}
     tf = lambda x: "true" if x else "false"
     op = ops.get((info["type_a"], info["type_b"]), "?")
-    if info["family"] == 2 and info["lane_fixed"]:  # one work-group per tile; DIV 2 where half the slots do
-        va, vb, r, c = info["vec_a"], info["vec_b"], info["rows"], info["cols"]
-        ea, eb = info["slots_a"] * va, info["slots_b"] * vb
-        half = 256 // (r // va) * (ea // va // 2) >= c and 256 // (c // vb) * (eb // vb // 2) >= r
-        return "ttc::transpose_lane_kernel<%s, %d, %d, %s, %s, %d>" % (
-            op, va, vb, tf(not info["beta_is_zero"]), tf(info["nt_store"]), 2 if half else 1)
-    if info["family"] == 2:
-        return "ttc::transpose_rc_kernel<%s, %d, %d, %s, %s, %s>" % (
-            op, info["vec_a"], info["vec_b"], tf(not info["beta_is_zero"]), tf(info["nt_store"]),
-            tf(info["lane_fixed"]))
-    return "ttc::transpose_kernel<%s, %d, %d, %s, %s>" % (op, info["vec_a"], info["vec_b"],
-                                                        tf(not info["beta_is_zero"]), tf(info["nt_store"]))
+    bz, nt, kernel = bool(info["beta_is_zero"]), bool(info["nt_store"]), launch["kernel"]
+    if kernel in (rt.KERNEL_ROW_WALK, rt.KERNEL_ROW, rt.KERNEL_ROW_SMALL):
+        mode = (2 if nt else 1) if bz else 0
+        name = {rt.KERNEL_ROW_WALK: "row_kernel", rt.KERNEL_ROW: "row_once_kernel"}.get(kernel, "row_small_kernel")
+        last = "" if kernel == rt.KERNEL_ROW_WALK else ", " + tf(launch["unaligned"])
+        return "ttc::%s<%s, %d, %d%s>" % (name, op, launch["vec_a"], mode, last)
+    name, last = {rt.KERNEL_TILE: ("transpose_lane_kernel", ", %d" % launch["slot_div"]),
+                  rt.KERNEL_TILE_SMALL: ("transpose_small_kernel", ", 2"),
+                  rt.KERNEL_TILE_WALK: ("transpose_rc_kernel", ", " + tf(launch["lane_fixed"]))}.get(
+                      kernel, ("transpose_kernel", ""))
+    return "ttc::%s<%s, %d, %d, %s, %s%s>" % (name, op, launch["vec_a"], launch["vec_b"], tf(not bz), tf(nt), last)
 
 
 def build_c2(torch, rt, wl, dev, tune=0):
@@ -105,7 +107,7 @@ def build_c2(torch, rt, wl, dev, tune=0):
                 ops.append({"k": case["k"], "es": es, "bz": bz, "plan": plan, "plan0": plan0, "A": A, "B": B,
                             "alpha": 1.0, "beta": 0.0 if bz else 1.0, "perm": case["perm"], "size": size,
                             "lda": lda, "ldb": ldb, "bytes": info["bytes_algorithmic"], "info": info,
-                            "kernel": kernel_name(info)})
+                            "kernel": kernel_name(plan)})
     # beta = 0 ops first, then beta = 1 ops
     ops.sort(key=lambda o: (not o["bz"], o["k"], o["es"]))
     return ops, bufs

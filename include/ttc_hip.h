@@ -92,7 +92,10 @@ typedef struct {
                             with wg_per_cu, or where a tile does not fit a launch of one work-group per tile */
 } ttc_config_t;
 
-/* What a plan resolved to (fused geometry, tile, launch shape). */
+/* What a plan resolved to (fused geometry, tile, numbering).  slots_a,
+ * slots_b, tiles, lds_bytes, lds_buffers and lane_fixed describe the launch
+ * of work-groups that walk several tiles, which the configuration stands for
+ * whatever kernel the plan launches; ttc_plan_get_launch tells that one. */
 typedef struct {
   int rank;                      /* after index fusion */
   int perm[TTC_MAX_DIM];
@@ -103,7 +106,8 @@ typedef struct {
   int vec_a, vec_b;
   int threads;                   /* work-group size (256) */
   int slots_a, slots_b;          /* vectors per thread per tile, read / write side */
-  int64_t tiles;                 /* number of tiles */
+  int64_t tiles;                 /* number of tiles (tile_order 3 / 4: with the padding ids of the last group); rows
+                                    of a row copy */
   int tile_volume;               /* elements per full tile */
   int lds_bytes;                 /* dynamic LDS per work-group */
   int lds_pad;                   /* LDS padding (elements) on B's stride-1 dimension */
@@ -121,6 +125,31 @@ typedef struct {
   int lds_buffers;               /* LDS tile buffers of the row x column kernel (1 for other families) */
   int lane_fixed;                /* row x column kernel: tiles take a lane-fixed walk (1) or the general one */
 } ttc_plan_info_t;
+
+/* The kernel that a call of a plan launches. */
+typedef enum {
+  TTC_KERNEL_NONE = 0,       /* no elements: nothing is launched */
+  TTC_KERNEL_BOX = 1,        /* box tiles */
+  TTC_KERNEL_TILE_WALK = 2,  /* row x column tiles, work-groups that walk several */
+  TTC_KERNEL_TILE = 3,       /* row x column tiles, one per work-group */
+  TTC_KERNEL_TILE_SMALL = 4, /* the same with few bytes of arguments */
+  TTC_KERNEL_ROW_WALK = 5,   /* row copy, work-groups that walk the tensor */
+  TTC_KERNEL_ROW = 6,        /* row copy, one chunk of vectors per work-group */
+  TTC_KERNEL_ROW_SMALL = 7   /* the same with few bytes of arguments */
+} ttc_kernel_t;
+
+typedef struct {
+  int kernel;           /* ttc_kernel_t */
+  int vec_a, vec_b;     /* elements per lane vector */
+  int unaligned;        /* row copy: its vectors are aligned to one element only */
+  int64_t units;        /* tiles (padding ids included) or chunks of the launch; on TTC_KERNEL_TILE* and ROW* one
+                           work-group each, in an fp8 cast with amax of more than 256 two for most */
+  int slots_a, slots_b; /* vectors per thread and unit, read / write side */
+  int slot_div;         /* row x column tiles, one per work-group: 2 = the instance of half the slots, else 1 */
+  int lds_bytes;        /* dynamic LDS per work-group */
+  int lds_buffers;      /* LDS tile buffers (0: none) */
+  int lane_fixed;       /* row x column tiles: full tiles take the lane-fixed walk (1) or the general one (0) */
+} ttc_plan_launch_t;
 
 /* Library version string. */
 const char* ttc_version(void);
@@ -144,6 +173,8 @@ ttc_status_t ttc_plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t t
                              const int* size, const int* lda, const int* ldb, int beta_is_zero,
                              const ttc_config_t* cfg);
 ttc_status_t ttc_plan_get_info(ttc_plan_t plan, ttc_plan_info_t* info);
+/* The launch of a call on buffers aligned to the plan's vectors. */
+ttc_status_t ttc_plan_get_launch(ttc_plan_t plan, ttc_plan_launch_t* launch);
 ttc_status_t ttc_plan_destroy(ttc_plan_t plan);
 
 /* Asynchronous execution on `stream`.  Replaces the kernel launch of the

@@ -1572,6 +1572,43 @@ extern "C" ttc_status_t ttc_plan_get_info(ttc_plan_t pl, ttc_plan_info_t* info) 
   return TTC_SUCCESS;
 }
 
+extern "C" ttc_status_t ttc_plan_get_launch(ttc_plan_t pl, ttc_plan_launch_t* out) {
+  if (!pl || !out) return TTC_ERROR_INVALID_VALUE;
+  std::memset(out, 0, sizeof(*out));
+  if (pl->g.elements == 0) return TTC_SUCCESS;
+  const int szA = dtype_bytes(pl->type_a), szB = dtype_bytes(pl->type_b);
+  out->vec_a = pl->va;
+  out->vec_b = pl->vb;
+  out->slot_div = 1;
+  if (pl->family == kFamilyRow) {
+    const bool once = pl->row1_grid != 0;
+    out->kernel = !once ? TTC_KERNEL_ROW_WALK : pl->small ? TTC_KERNEL_ROW_SMALL : TTC_KERNEL_ROW;
+    out->units = once ? pl->row1_grid : pl->p.ntiles;
+    out->unaligned = once && pl->row1_unaligned;
+    if (once) out->vec_a = out->vec_b = pl->row1_v;
+    out->slots_a = out->slots_b =
+        once ? row_once_unroll(szA, szB, pl->row1_v, szB == 1, pl->row1_unaligned != 0) : kRowUnroll;
+  } else if (pl->family == kFamilyRC) {
+    const bool lane = pl->lane_div != 0;
+    out->kernel = !lane ? TTC_KERNEL_TILE_WALK : pl->small ? TTC_KERNEL_TILE_SMALL : TTC_KERNEL_TILE;
+    out->units = lane ? pl->lane.walk.ntiles : pl->rc.ntiles;
+    out->slot_div = lane ? pl->lane_div : 1;
+    out->slots_a = rc_elems(szA) / pl->va / out->slot_div;
+    out->slots_b = rc_elems(szB) / pl->vb / out->slot_div;
+    out->lds_bytes = lane ? pl->lane_lds : pl->lds_bytes;
+    out->lds_buffers = lane ? 1 : pl->rc.nbuf;
+    out->lane_fixed = lane || pl->rc.fast;
+  } else {
+    out->kernel = TTC_KERNEL_BOX;
+    out->units = pl->p.ntiles;
+    out->slots_a = (pl->p.V / pl->va + kThreads - 1) / kThreads;
+    out->slots_b = (pl->p.V / pl->vb + kThreads - 1) / kThreads;
+    out->lds_bytes = pl->lds_bytes;
+    out->lds_buffers = 1;
+  }
+  return TTC_SUCCESS;
+}
+
 extern "C" ttc_status_t ttc_plan_destroy(ttc_plan_t pl) {
   if (!pl) return TTC_ERROR_INVALID_VALUE;
   delete pl->fallback;

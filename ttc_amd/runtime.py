@@ -87,6 +87,21 @@ class PlanInfo(ctypes.Structure):
                 "lane_fixed": self.lane_fixed}
 
 
+# ttc_kernel_t: the kernel that a call of a plan launches
+(KERNEL_NONE, KERNEL_BOX, KERNEL_TILE_WALK, KERNEL_TILE, KERNEL_TILE_SMALL, KERNEL_ROW_WALK, KERNEL_ROW,
+ KERNEL_ROW_SMALL) = range(8)
+
+
+class PlanLaunch(ctypes.Structure):
+    _fields_ = [("kernel", ctypes.c_int), ("vec_a", ctypes.c_int), ("vec_b", ctypes.c_int),
+                ("unaligned", ctypes.c_int), ("units", ctypes.c_int64), ("slots_a", ctypes.c_int),
+                ("slots_b", ctypes.c_int), ("slot_div", ctypes.c_int), ("lds_bytes", ctypes.c_int),
+                ("lds_buffers", ctypes.c_int), ("lane_fixed", ctypes.c_int)]
+
+    def as_dict(self):
+        return {name: getattr(self, name) for name, _ in self._fields_}
+
+
 class BatchOp(ctypes.Structure):
     _fields_ = [("type_a", ctypes.c_int), ("type_b", ctypes.c_int), ("dim", ctypes.c_int),
                 ("perm", ctypes.c_int * MAX_INPUT_DIM), ("size", ctypes.c_int * MAX_INPUT_DIM),
@@ -98,7 +113,7 @@ class BatchOp(ctypes.Structure):
 # Every symbol include/ttc_hip.h declares (checked by the CPU tests).
 EXPORTS = [
     "ttc_version", "ttc_status_string", "ttc_dtype_size", "ttc_fuse_indices", "ttc_plan_create",
-    "ttc_plan_get_info", "ttc_plan_destroy", "ttc_execute", "ttc_execute_fp8", "ttc_legacy_transpose",
+    "ttc_plan_get_info", "ttc_plan_get_launch", "ttc_plan_destroy", "ttc_execute", "ttc_execute_fp8", "ttc_legacy_transpose",
     "ttc_batch_create", "ttc_batch_execute", "ttc_batch_graph_launch", "ttc_batch_execute_loop",
     "ttc_batch_get_info", "ttc_batch_destroy", "ttc_batch_execute_noalloc",
 ]
@@ -131,6 +146,8 @@ def _load():
     L.ttc_plan_create.restype = ctypes.c_int
     L.ttc_plan_get_info.argtypes = [vp, ctypes.POINTER(PlanInfo)]
     L.ttc_plan_get_info.restype = ctypes.c_int
+    L.ttc_plan_get_launch.argtypes = [vp, ctypes.POINTER(PlanLaunch)]
+    L.ttc_plan_get_launch.restype = ctypes.c_int
     L.ttc_plan_destroy.argtypes = [vp]
     L.ttc_plan_destroy.restype = ctypes.c_int
     L.ttc_execute.argtypes = [vp, vp, vp, ctypes.c_double, ctypes.c_double, vp]
@@ -242,6 +259,13 @@ class Plan:
     def info(self):
         i = PlanInfo()
         _check(self._lib.ttc_plan_get_info(self._h, ctypes.byref(i)), "ttc_plan_get_info")
+        return i.as_dict()
+
+    def launch(self):
+        """The kernel that a call on buffers aligned to the plan's vectors
+        launches (ttc_plan_get_launch)."""
+        i = PlanLaunch()
+        _check(self._lib.ttc_plan_get_launch(self._h, ctypes.byref(i)), "ttc_plan_get_launch")
         return i.as_dict()
 
     def extent_bytes(self):
