@@ -184,3 +184,29 @@ def test_command_line_flags_reach_the_emitted_configuration(workdir):
     src = (workdir / "ttc_transpositions" / (name + ".hip")).read_text()
     want = rt.Plan(rt.S, rt.S, [1, 0], [1000, 768], beta_is_zero=True, config={"run_a": 16, "run_b": 256}).info()
     assert "{{%s}" % ", ".join(str(t) for t in want["tile"] + [0] * 6) in src
+
+
+@pytest.mark.parametrize("perm,size,beta", [([1, 0], [4000, 4100], True), ([2, 0, 1], [640, 40, 300], False),
+                                            ([3, 1, 0, 2], [40, 12, 30, 9], True), ([1, 0], [300, 20000], False)])
+def test_candidates_are_distinct_launches(perm, size, beta):
+    """Launches of one work-group per tile walk tile orders 2 and 3 alike: no
+    candidate is timed twice, bands of 16 tiles are tried where there are more
+    than 8 to a band, and work-groups that walk several tiles keep order 3."""
+    rt.lib()
+    walks, n16 = {}, 0
+    cands = autotune.candidates(rt.S, rt.S, perm, size, beta_is_zero=not beta, max_impl=200)
+    assert len(cands) > 20
+    for cfg in cands:
+        if cfg.get("family") != 2:
+            continue
+        plan = rt.Plan(rt.S, rt.S, perm, size, beta_is_zero=not beta, config=cfg)
+        one = plan.launch()["kernel"] in (rt.KERNEL_TILE, rt.KERNEL_TILE_SMALL)
+        order = cfg["tile_order"]
+        if one:
+            assert order in (1, 2, 4), cfg
+            n16 += order == 4
+        key = (tuple(cfg["tile"]), cfg["vec_a"], cfg["vec_b"], cfg["grid_order"], cfg.get("nt_store"),
+               cfg.get("wg_per_cu"), cfg.get("lds_buffers"), one, 2 if one and order == 3 else order)
+        assert key not in walks, (cfg, walks[key])
+        walks[key] = cfg
+    assert n16 or size == [40, 12, 30, 9]

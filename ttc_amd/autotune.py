@@ -78,6 +78,23 @@ def tile_walk_cost(info, tile_order):
     return ttc_util.walkCost(list(reversed(inner_first)))
 
 
+def tile_orders(info, one_tile):
+    """The tile orders worth timing for a row x column plan, cheapest walk
+    first.  Work-groups that walk several tiles (one_tile false): 2, 3 and 1.
+    Launches of one work-group per tile walk orders 2 and 3 alike, in bands of
+    8 tiles along the rows' outermost tiled dimension (4: of 16) unless that
+    dimension is B's first tiled one: 2 and 1, and 4 where it differs from 2."""
+    if not one_tile:
+        return sorted((2, 3, 1), key=lambda o: (tile_walk_cost(info, o), o))
+    g = [-(-n // t) if n else 1 for n, t in zip(info["size"], info["tile"])]
+    band = next((k for k in reversed(_row_group(info)) if g[k] > 1), None)
+    first = next((k for k in info["perm"] if g[k] > 1), None)
+    bands = band is not None and band != first
+    cost = {1: tile_walk_cost(info, 1), 2: tile_walk_cost(info, 3 if bands else 2), 4: tile_walk_cost(info, 4)}
+    orders = (2, 4, 1) if bands and g[band] > 8 else (2, 1)
+    return sorted(orders, key=lambda o: (cost[o], o))
+
+
 def candidates(type_a, type_b, perm, size, lda=None, ldb=None, beta_is_zero=False, max_impl=200,
                nt_stores=False, blockings=None):
     """List of config dicts, best-first by the model, at most max_impl.  The
@@ -112,9 +129,11 @@ def candidates(type_a, type_b, perm, size, lda=None, ldb=None, beta_is_zero=Fals
             for ra, rb in targets:
                 cfg = {"vec_a": va, "vec_b": vb, "run_a": int(ra), "run_b": int(rb), "family": fam}
                 try:
-                    info = rt.Plan(type_a, type_b, perm, size, lda, ldb, beta_is_zero, cfg).info()
+                    plan = rt.Plan(type_a, type_b, perm, size, lda, ldb, beta_is_zero, cfg)
                 except rt.TTCError:
                     continue
+                info = plan.info()
+                info["one_tile"] = plan.launch()["kernel"] in (rt.KERNEL_TILE, rt.KERNEL_TILE_SMALL)
                 key = (fam, tuple(info["tile"]), va, vb)
                 if key not in tiles:
                     tiles[key] = (tile_score(info, sa, sb),
@@ -153,7 +172,7 @@ def candidates(type_a, type_b, perm, size, lda=None, ldb=None, beta_is_zero=Fals
         out += [{"family": 3, "wg_per_cu": w} for w in (4, 2)]
     for t, info in ranked:
         if t["family"] == 2:
-            tords = sorted((2, 3, 1), key=lambda o: (tile_walk_cost(info, o), o))
+            tords = tile_orders(info, info["one_tile"])
         else:
             tords = (2,)  # box tiles have one numbering
         launch = [{"grid_order": go, "tile_order": to, "nt_store": nt}
@@ -167,7 +186,7 @@ def candidates(type_a, type_b, perm, size, lda=None, ldb=None, beta_is_zero=Fals
     if ranked:
         t0, i0 = ranked[0]
         l0 = {"grid_order": grid_orders[0], "nt_store": nts[0],
-              "tile_order": min((2, 3, 1), key=lambda o: (tile_walk_cost(i0, o), o)) if t0["family"] == 2 else 2}
+              "tile_order": tile_orders(i0, False)[0] if t0["family"] == 2 else 2}  # (wg_per_cu, lds_buffers: walks)
         for w in (2, 3):
             if len(out) < max_impl:
                 c = dict(t0)
