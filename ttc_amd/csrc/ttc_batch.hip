@@ -280,6 +280,28 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
     OpRec& r = rec[i];
     r.src = i;
     const int64_t sa = dtype_bytes(op.type_a), sb = dtype_bytes(op.type_b);
+    // puts the op into the launch of one work-group per tile, if its plan takes it
+    auto take_one = [&](const ttc_plan_s* use) {
+      const int bz = use->beta_is_zero ? 1 : 0;
+      int variant;
+      uint32_t ntiles;
+      if (use->family == kFamilyRC && use->lane_div == 2) {
+        variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
+        ntiles = use->lane.walk.ntiles;
+      } else if (use->family == kFamilyRow) {
+        const RowChunks c = row_chunks(use, op.A, op.B);
+        variant = c.unaligned ? kOneRowUnaligned + __builtin_ctz((unsigned)c.v) * 2 + bz
+                              : kOneRow + index_of_width(c.v, wide) * 2 + bz;
+        ntiles = c.grid;
+      } else {
+        return false;
+      }
+      r.kind = pair * kOneVariants + variant;
+      r.ntiles = use->g.elements == 0 ? 0 : ntiles;
+      r.weight = 0.0;
+      bp.bytes += use->g.elements * (sa + sb * (bz ? 1 : 2));
+      return true;
+    };
     // one work-group per tile, where the op's plan takes such a launch
     {
       ttc_plan_t pl = nullptr;
@@ -290,21 +312,7 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
       if (pl->g.elements > 0 && (!op.A || !op.B)) return TTC_ERROR_INVALID_VALUE;
       const ttc_plan_s* use = pl->g.elements > 0 ? variant_for(pl, op.A, op.B) : pl;
       if (!use) return TTC_ERROR_INVALID_VALUE;
-      const int bz = pl->beta_is_zero ? 1 : 0;
-      int variant = -1;
-      if (use->family == kFamilyRC && use->lane_div == 2)
-        variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
-      const RowChunks c = use->family == kFamilyRow ? row_chunks(use, op.A, op.B) : RowChunks{};
-      if (use->family == kFamilyRow)
-        variant = c.unaligned ? kOneRowUnaligned + __builtin_ctz((unsigned)c.v) * 2 + bz
-                              : kOneRow + index_of_width(c.v, wide) * 2 + bz;
-      if (variant >= 0) {
-        r.kind = pair * kOneVariants + variant;
-        r.ntiles = pl->g.elements == 0 ? 0 : (use->family == kFamilyRC ? use->lane.walk.ntiles : c.grid);
-        r.weight = 0.0;
-        bp.bytes += pl->g.elements * (sa + sb * (bz ? 1 : 2));
-        continue;
-      }
+      if (take_one(use)) continue;
       bp.plans[i] = nullptr;
       ttc_plan_destroy(pl);
     }
@@ -335,7 +343,8 @@ static ttc_status_t plan_batch(int nops, const ttc_batch_op_t* ops, int wg_per_c
     if (!width_ok(pl, pl->va) || !width_ok(pl, pl->vb)) return TTC_ERROR_UNSUPPORTED;
     const ttc_plan_s* use = pl->g.elements > 0 ? variant_for(pl, op.A, op.B) : pl;
     if (!use) return TTC_ERROR_INVALID_VALUE;
-    if (!width_ok(use, use->va) || !width_ok(use, use->vb) || use->family == kFamilyRow) return TTC_ERROR_UNSUPPORTED;
+    if (!width_ok(use, use->va) || !width_ok(use, use->vb)) return TTC_ERROR_UNSUPPORTED;
+    if (take_one(use)) continue;  // without the tile its widths ruled out, a row copy
     const int fam = use->family == kFamilyRC ? kGroupRC : kGroupBox;
     const int bz = pl->beta_is_zero ? 1 : 0;
     const int variant = (index_of_width(use->va, wide) * 3 + index_of_width(use->vb, wide)) * 2 + bz;
