@@ -291,3 +291,10 @@ def test_row_copy_family_for_perm0():
     for bad in ({"vec_a": 4, "vec_b": 2}, {"vec_a": 8}, {"vec_b": 16}):
         with pytest.raises(rt.TTCError):
             rt.Plan(S, rt.BF16, [0, 2, 1], [64, 48, 80], config=dict(bad, family=3))
+
+
+@pytest.mark.parametrize("perm,size", [([1, 0], [0, 4]), ([1, 0], [4, 0]), ([2, 1, 0], [3, 0, 5]), ([2, 0, 1], [0, 0, 8])])
+def test_row_column_tiles_of_no_elements_are_refused(perm, size):
+    # an empty tensor's own extents as a tile: 0 along its empty dimensions
+    with pytest.raises(rt.TTCError):
+        rt.Plan(S, S, perm, size, config={"family": 2, "tile": size})

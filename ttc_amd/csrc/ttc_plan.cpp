@@ -512,6 +512,8 @@ bool rc_groups(const Geometry& g, const int* tile, int& na, int* ga, int& nb, in
   const int p0 = g.perm[0];
   na = nb = 0;
   if (p0 == 0 || r < 2) return false;
+  for (int k = 0; k < r; ++k)
+    if (tile[k] < 1) return false;
   bool in_a[kMaxDim] = {false}, in_b[kMaxDim] = {false};
   for (int k = 0; k < r && k != p0; ++k) {
     if (k > 0 && (tile[k] == 1 || g.size[k - 1] % tile[k - 1] != 0)) break;
