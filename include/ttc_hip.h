@@ -143,7 +143,8 @@ typedef struct {
   int vec_a, vec_b;     /* elements per lane vector */
   int unaligned;        /* row copy: its vectors are aligned to one element only */
   int64_t units;        /* tiles (padding ids included) or chunks of the launch; on TTC_KERNEL_TILE* and ROW* one
-                           work-group each, in an fp8 cast with amax of more than 256 two for most */
+                           work-group each, in an fp8 cast with amax of more than 256 two for most (of 257 to 512
+                           chunks it takes TTC_KERNEL_ROW_WALK) */
   int slots_a, slots_b; /* vectors per thread and unit, read / write side */
   int slot_div;         /* row x column tiles, one per work-group: 2 = the instance of half the slots, else 1 */
   int lds_bytes;        /* dynamic LDS per work-group */

@@ -65,8 +65,10 @@ static bool check_row(const ttc_plan_s* pl, int ta, int tb, int beta, int n0, lo
     ++small;
   }
   const int szA = dtype_bytes(ta), szB = dtype_bytes(tb);
-  const long long chunk = 256ll * row_once_unroll(szA, szB, (int)V, szB == 1, pl->row1_unaligned != 0);
-  CHECK(pl->row1_grid * chunk >= (long long)p.total && (pl->row1_grid - 1) * chunk < (long long)p.total);
+  const bool once = pl->row1_grid != 0;  // else work-groups walk the chunks
+  const long long chunk = 256ll * (once ? row_once_unroll(szA, szB, (int)V, szB == 1, pl->row1_unaligned != 0) : kRowUnroll);
+  const long long chunks = once ? pl->row1_grid : pl->p.ntiles;
+  CHECK(chunks * chunk >= (long long)p.total && (chunks - 1) * chunk < (long long)p.total);
   return true;
 }
 

@@ -61,6 +61,27 @@ def test_row_copies_and_boxes():
     assert launch(S, S, [1, 0], [300, 0])[0]["kernel"] == rt.KERNEL_NONE
 
 
+@pytest.mark.parametrize("tA,tB,perm,size,beta,kernel", [
+    # casts on aligned vectors, from 4 MiB to below 384 MiB moved
+    (BF16, E4M3, [0, 2, 1], [128, 100, 100], False, "KERNEL_ROW"),
+    (BF16, E4M3, [0, 2, 1], [64, 72, 512], False, "KERNEL_ROW_WALK"),
+    (BF16, E4M3, [0, 2, 1], [128, 4096, 255], False, "KERNEL_ROW_WALK"),
+    (BF16, E4M3, [0, 2, 1], [128, 4096, 256], False, "KERNEL_ROW"),
+    (S, E4M3, [0], [4000000], False, "KERNEL_ROW_WALK"),
+    (BF16, E4M3, [0, 2, 1], [127, 300, 121], False, "KERNEL_ROW"),  # unaligned
+    # accumulation of 4- and 2-byte elements one at a time
+    (S, BF16, [0], [2000001], True, "KERNEL_ROW_WALK"),
+    (BF16, S, [0, 2, 1], [21, 330, 481], True, "KERNEL_ROW_WALK"),
+    (S, BF16, [0], [2000001], False, "KERNEL_ROW_SMALL"),
+    (S, BF16, [0], [4000000], True, "KERNEL_ROW_SMALL"),
+    (S, D, [0], [2000001], True, "KERNEL_ROW"),
+    (S, BF16, [0], [20001], True, "KERNEL_ROW_SMALL"),
+])
+def test_row_copies_that_are_walked(tA, tB, perm, size, beta, kernel):
+    one, _ = launch(tA, tB, perm, size, beta)
+    assert one["kernel"] == getattr(rt, kernel), one
+
+
 def test_bench_names_the_kernel():
     import bench
     name = lambda *a, **k: bench.kernel_name(rt.Plan(*a, **k))

@@ -1021,6 +1021,21 @@ RowChunks row_chunks(const ttc_plan_s* use, const void* A, const void* B) {
   return RowChunks{&use->row, use->va, false, row_chunk_count(use->row, szA, szB, use->va, szB == 1, false)};
 }
 
+// Aligned row copies of v elements that work-groups walking the tensor
+// (row_kernel) do faster than one chunk per work-group:
+// - casts to fp8 of 4 to 384 MiB moved (bf16 64 x 72 x 512, 7 MB: 9.0 us in
+//   chunks, 7.3 walked; 64 x 179 x 69 x 72, 171 MB: 44.7 and 40.6; bf16 1024 x
+//   48 x 1024 x 4, 604 MB: the other way round, 5-10% on one row). Below they
+//   are within 3%.
+// - accumulation of elements of 4 and 2 bytes one at a time (fp32 -> bf16, one
+//   row of 35828715: 99 us in chunks, 71 walked; from 1 MiB on).
+static bool row_walks(const ttc_plan_s* pl, int v) {
+  const int szA = dtype_bytes(pl->type_a), szB = dtype_bytes(pl->type_b);
+  const long long moved = pl->g.elements * (szA + (pl->beta_is_zero ? 1ll : 2ll) * szB);
+  if (szB == 1) return moved >= (4ll << 20) && moved < (384ll << 20);
+  return !pl->beta_is_zero && v == 1 && szA != szB && szA + szB == 6 && moved >= (1ll << 20);
+}
+
 // The one-chunk-per-work-group launch of row copy p (aligned vectors of v
 // elements): unaligned vectors where they are wider.  Rows shorter than a
 // cache line share lines with their neighbours in A and B, which then meet in
@@ -1034,9 +1049,10 @@ static void build_row_once(ttc_plan_s* pl, int v) {
   pl->row1_unaligned = 0;
   pl->row1_grid = 0;
   pl->small = 0;
-  if (pl->row.total == 0 || (pl->wg_per_cu > 0 && pl->min_div == 1)) return;
+  if (pl->row.total == 0) return;
   const bool may = !pl->vec_given && row_unaligned_mode(szA, szB, !pl->beta_is_zero, pl->nt_store != 0);
   const int w = may ? row_unaligned_width(szA, szB, n0) : 1;
+  if (!pl->in_group && (pl->wg_per_cu > 0 || (w <= v && row_walks(pl, v)))) return;
   if (w > v) {
     const uint32_t rows = pl->row.total / pl->row.nv;
     pl->row1_v = w;
@@ -1464,7 +1480,8 @@ ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t 
   pl->one_tile = c.wg_per_cu == 0 && (c.lds_buffers == 0 || !explicit_tile);
   if (use == kPlanGroupTile) pl->one_tile = c.lds_buffers == 0;  // (wg_per_cu does not apply to an op of a group)
   if (use == kPlanGroupWalk) pl->one_tile = 0;
-  pl->min_div = use == kPlanSingle ? 1 : 2;
+  pl->in_group = use != kPlanSingle;
+  pl->min_div = pl->in_group ? 2 : 1;
   auto in_list = [](int w, int bytes) {
     for (int x : vec_widths(bytes))
       if (x == w) return true;

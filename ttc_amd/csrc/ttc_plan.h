@@ -154,6 +154,7 @@ struct ttc_plan_s {
   int tile_order;        // 1 A order, 2 B order, 3 / 4 grouped B order (row x column tiles only)
   int lds_buffers;       // LDS tile buffers of the row x column kernel
   ttc::RCParams rc;
+  int in_group;          // an op of a grouped launch
   int min_div;           // smallest RCLane DIV the launch has: 2 in grouped launches
   int vec_given;         // the caller chose the vector widths
   int one_tile;          // row x column tiles: one tile per work-group where the tile fits (ttc_lane.hpp)
@@ -163,7 +164,7 @@ struct ttc_plan_s {
   ttc::RowParams row;
   ttc::RowParams row1;   // one chunk per work-group (row_once_kernel)
   int row1_v, row1_unaligned;
-  unsigned row1_grid;    // 0: row_kernel (wg_per_cu given)
+  unsigned row1_grid;    // 0: row_kernel (wg_per_cu given, or row_walks)
   int small;             // lane_small (one tile per work-group, DIV 2) or row_small is the launch's
   ttc::RCLaneSmall lane_small;
   ttc::RowSmall row_small;
