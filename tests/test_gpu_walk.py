@@ -6,7 +6,8 @@ case first asserts that this kernel is the one launched."""
 import numpy as np
 import pytest
 
-from common import BF16, CODE, F16, S, _real_update, first_diff, same_bits, to_device
+from common import (BF16, CODE, F16, S, _real_update, first_diff, from_device, make_case, oracle_run, same_bits,
+                    to_device)
 from oracle import oracle as orc
 from test_gpu_cast_batch import E4M3, E5M2, FP8_MAX, _heavy_input
 from test_gpu_parity import RANDOM_SHAPES, check
@@ -110,3 +111,21 @@ def test_fp8_casts(gpu, tA, tB):
         plan.execute_fp8(dA, dB, 0.5, amax_out=amax, mode=rt.SCALE_CURRENT)
         torch.cuda.synchronize()
         assert same_bits(dB.cpu().numpy(), want) and float(amax.item()) == top, (tA, tB, size, "current")
+
+
+@pytest.mark.parametrize("code", ["s", "d", "b", "c", "sb"])
+@pytest.mark.parametrize("perm,size", [([1, 0], [2, 1600001]), ([1, 0], [1600001, 3]), ([1, 2, 0], [3, 249, 7000])])
+def test_slivers(gpu, code, perm, size):
+    """Short groups, whose tiles are walked where one work-group per tile would
+    leave slivers."""
+    import torch
+    from ttc_amd import runtime as rt
+    tA, tB = CODE[code]
+    for beta in (0.0, 0.75):
+        A, B = make_case(tA, tB, perm, size, seed=len(size))
+        dA, dB = to_device(A, gpu), to_device(B, gpu)
+        plan = rt.Plan(tA, tB, perm, size, beta_is_zero=beta == 0.0)
+        plan.execute(dA, dB, 1.25, beta)
+        torch.cuda.synchronize()
+        got, want = from_device(dB, B), oracle_run(tA, tB, A, B, 1.25, beta, perm, size)
+        assert same_bits(got, want), (plan.launch(), first_diff(got, want))

@@ -82,6 +82,15 @@ def test_row_copies_that_are_walked(tA, tB, perm, size, beta, kernel):
     assert one["kernel"] == getattr(rt, kernel), one
 
 
+def test_slivers_are_walked():
+    walks = (rt.KERNEL_TILE_WALK, rt.KERNEL_BOX)
+    assert launch(BF16, BF16, [1, 4, 3, 0, 2], [2, 540, 723, 5, 28], True)[0]["kernel"] in walks
+    assert launch(BF16, BF16, [1, 0], [2, 1600001])[0]["kernel"] in walks
+    assert launch(BF16, BF16, [1, 0], [2, 1600001], family=2)[0]["kernel"] == rt.KERNEL_TILE_WALK
+    assert launch(BF16, BF16, [1, 0], [2, 400001])[0]["kernel"] == rt.KERNEL_TILE_SMALL  # few tiles
+    assert launch(BF16, BF16, [1, 0], [16, 200001])[0]["kernel"] == rt.KERNEL_TILE
+
+
 def test_bench_names_the_kernel():
     import bench
     name = lambda *a, **k: bench.kernel_name(rt.Plan(*a, **k))

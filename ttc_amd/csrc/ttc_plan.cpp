@@ -1141,6 +1141,11 @@ static long long run_alignment_b(const Geometry& g, const int* tile, int szB) {
   return bits & -bits;
 }
 
+// What issuing every slot of the tiles costs, as lane_cost counts it.
+static double slot_cost(int szA, int szB, int va, int vb, int div, bool beta, double ntiles) {
+  return ntiles * 850.0 * (rc_elems(szA) / va / div + rc_elems(szB) / vb / div * (beta ? 2.0 : 1.0));
+}
+
 // Cost of a launch of one work-group per tile, in bytes of HBM traffic, fitted
 // to 173 shapes x ~100 tiles each: the tile it picks is measured 2.1% (mean)
 // and at most 10% behind each shape's fastest; with run lengths and slots
@@ -1158,11 +1163,36 @@ static double lane_cost(const Geometry& g, const int* tile, int szA, int szB, in
   const double N = (double)g.elements, m = beta ? 2.0 : 1.0;
   const double ba = std::min(16384.0, (double)ra * szA), bb = std::min(16384.0, (double)rb * szB);
   const double off = (double)(128 - run_alignment_b(g, tile, szB)) / 128.0;
-  const double slots = rc_elems(szA) / va / div + rc_elems(szB) / vb / div * m;
   return N * szA * (1.0 + 56.0 / ba + 7.0 / ((double)f.R * szA)) +
          N * szB * m * (1.0 + ((szB == 1 ? 10.0 : 176.0) * off + 14.0) / bb + 14.0 / ((double)f.C * szB)) +
-         (double)f.ntiles * 850.0 * slots +
+         slot_cost(szA, szB, va, vb, div, beta, (double)f.ntiles) +
          (div == 1 ? 795.0 : 425.0) * (double)(f.R * f.C) * (szA + szB * m);
+}
+
+// Whether the tile picked for one work-group per tile is a sliver: one group
+// of up to 5 positions, and the other cut to the work-group's lanes, so that
+// its slots cost more than twice the bytes moved.  The work-groups that walk
+// several tiles take longer tiles there (`walk`).  Over 1500 shapes, the 30
+// launches that take them for it ran 1.53 times as long as slivers (geometric
+// mean; 0.82 to 4.9 times: fp16 2 x 540 x 723 x 5 x 28, 566 against 117 us).
+constexpr double kSliverTiles = 3000.0, kSliverSlots = 2.0, kSliverGain = 1.15;
+static double moved_bytes(const Geometry& g, int szA, int szB, bool beta) {
+  return (double)g.elements * (szA + szB * (beta ? 2.0 : 1.0));
+}
+static bool lane_sliver(const Geometry& g, const int* tile, int szA, int szB, int va, int vb, bool beta, double& cost) {
+  LaneFit f;
+  int div = 2;
+  while (div > 0 && !lane_fit(g, tile, szA, szB, va, vb, div, f)) --div;
+  if (div == 0 || std::min(f.R, f.C) > 5 || (double)f.ntiles < kSliverTiles) return false;
+  cost = slot_cost(szA, szB, va, vb, div, beta, (double)f.ntiles);
+  return cost >= kSliverSlots * moved_bytes(g, szA, szB, beta);
+}
+static bool sliver_loses(const Geometry& g, double sliver, const int* walk, int szA, int szB, int va, int vb,
+                         bool beta) {
+  double ntiles = 1.0;
+  for (int k = 0; k < g.rank; ++k) ntiles *= (double)tiles_of(g.size[k], walk[k]);
+  const double moved = moved_bytes(g, szA, szB, beta);
+  return moved + sliver >= kSliverGain * (moved + slot_cost(szA, szB, va, vb, 1, beta, ntiles));
 }
 
 // Tile of a launch of one work-group per tile: run-length targets on both
@@ -1333,6 +1363,8 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
   if (tile_in)
     for (int k = 0; k < g.rank; ++k) explicit_tile |= tile_in[k] != 0;
   int fam = family;
+  bool one_tile = pl->one_tile != 0;
+  pl->lane_div = pl->small = 0;  // (a variant starts as a copy of its plan)
   if (fam == kFamilyRow && g.perm[0] != 0) return TTC_ERROR_UNSUPPORTED;
   if (fam == kFamilyRow || (fam == 0 && !explicit_tile && g.perm[0] == 0)) {
     // A and B share the stride-1 dimension: rows move without LDS staging.
@@ -1366,32 +1398,43 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     for (int k = 0; k < kMaxDim; ++k) tile[k] = k < g.rank ? tile_in[k] : 1;
     if (fam == 0) fam = kFamilyBox;
   } else {
-    int rc_tile[kMaxDim];
+    int lane_tile[kMaxDim], rc_tile[kMaxDim];
     double rc_score = -1.0;
-    const bool lane = fam != kFamilyBox && pl->one_tile && run_a == 0 && run_b == 0 &&
-                      choose_lane_tile(g, pl->type_a, pl->type_b, va, vb, !pl->beta_is_zero, rc_tile, pl->min_div);
+    const int szA = dtype_bytes(pl->type_a), szB = dtype_bytes(pl->type_b);
+    bool lane = fam != kFamilyBox && one_tile && run_a == 0 && run_b == 0 &&
+                choose_lane_tile(g, pl->type_a, pl->type_b, va, vb, !pl->beta_is_zero, lane_tile, pl->min_div);
+    double sliver = 0.0;
+    const bool weigh = lane && !pl->in_group && lane_sliver(g, lane_tile, szA, szB, va, vb, !pl->beta_is_zero, sliver);
     // (a caller that names the family is refused the shapes choose_rc_tile refuses)
     if (lane && fam == kFamilyRC) {
       int t[kMaxDim];
       if (!choose_rc_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, t, nullptr)) return TTC_ERROR_UNSUPPORTED;
     }
-    if (lane) fam = kFamilyRC;
-    const bool rc_ok = fam != kFamilyBox && !lane &&
-                       choose_rc_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, rc_tile, &rc_score);
-    if (fam == kFamilyRC && !rc_ok && !lane) return TTC_ERROR_UNSUPPORTED;
-    if (fam != kFamilyRC) choose_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, tile);
-    if (fam == 0) {
-      // The row x column kernel issues all of a tile's slots: it wins when
-      // its tile fills at least half of them or is no smaller than the box.
-      long long vr = 1, vbox = 1;
-      for (int k = 0; k < g.rank; ++k) {
-        vr *= rc_ok ? rc_tile[k] : 1;
-        vbox *= tile[k];
+    if (!lane || weigh) {
+      const bool rc_ok = fam != kFamilyBox &&
+                         choose_rc_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, rc_tile, &rc_score);
+      if (fam == kFamilyRC && !rc_ok) return TTC_ERROR_UNSUPPORTED;
+      if (fam != kFamilyRC) choose_tile(g, pl->type_a, pl->type_b, va, vb, run_a, run_b, tile);
+      int walk = fam;
+      if (walk == 0) {
+        // The row x column kernel issues all of a tile's slots: it wins when
+        // its tile fills at least half of them or is no smaller than the box.
+        long long vr = 1, vbox = 1;
+        for (int k = 0; k < g.rank; ++k) {
+          vr *= rc_ok ? rc_tile[k] : 1;
+          vbox *= tile[k];
+        }
+        walk = rc_ok && (2 * vr >= max_rc_volume(pl->type_a, pl->type_b) || vr >= vbox) ? kFamilyRC : kFamilyBox;
       }
-      fam = rc_ok && (2 * vr >= max_rc_volume(pl->type_a, pl->type_b) || vr >= vbox) ? kFamilyRC : kFamilyBox;
+      if (walk == kFamilyRC)
+        for (int k = 0; k < kMaxDim; ++k) tile[k] = rc_tile[k];
+      if (weigh && sliver_loses(g, sliver, tile, szA, szB, va, vb, !pl->beta_is_zero)) lane = one_tile = false;
+      if (!lane) fam = walk;
     }
-    if (fam == kFamilyRC)
-      for (int k = 0; k < kMaxDim; ++k) tile[k] = rc_tile[k];
+    if (lane) {
+      fam = kFamilyRC;
+      for (int k = 0; k < kMaxDim; ++k) tile[k] = lane_tile[k];
+    }
   }
   pl->va = va;
   pl->vb = vb;
@@ -1408,9 +1451,7 @@ static ttc_status_t plan_fill(ttc_plan_s* pl, int va, int vb, const int* tile_in
     pl->p.grid_order = pl->rc.grid_order;
     // one tile per work-group unless the caller asks for resident
     // work-groups or LDS buffers, which only the pipelined kernel has
-    pl->lane_div = 0;
-    pl->small = 0;
-    if (pl->one_tile && st == TTC_SUCCESS)
+    if (one_tile && st == TTC_SUCCESS)
       for (int div = 2; div >= pl->min_div && pl->lane_div == 0; --div)
         if (build_lane_params(g, tile, pl->type_a, pl->type_b, va, vb, pl->grid_order, pl->tile_order, div, pl->lane,
                               pl->lane_lds))
