@@ -129,3 +129,25 @@ def test_slivers(gpu, code, perm, size):
         torch.cuda.synchronize()
         got, want = from_device(dB, B), oracle_run(tA, tB, A, B, 1.25, beta, perm, size)
         assert same_bits(got, want), (plan.launch(), first_diff(got, want))
+
+
+@pytest.mark.parametrize("code", ["s", "d", "b", "h", "c", "sb", "bs"])
+@pytest.mark.parametrize("perm,size", [([1, 5, 0, 2, 4, 3], [6, 6, 14, 14, 46, 6]), ([1, 0, 2], [512, 64, 40]),
+                                       ([1, 0], [1024, 6]), ([3, 1, 2, 4, 5, 0], [24, 3, 24, 2, 2, 40])])
+def test_misaligned_pointers_take_a_tile_of_their_own(gpu, code, perm, size):
+    import torch
+    from ttc_amd import runtime as rt
+    tA, tB = CODE[code]
+    for beta in (0.0, 0.75):
+        A, B = make_case(tA, tB, perm, size, seed=len(size))
+        dA = torch.zeros(A.nbytes + 16, dtype=torch.uint8, device=gpu)
+        dB = torch.zeros(B.nbytes + 16, dtype=torch.uint8, device=gpu)
+        a, b = dA[A.itemsize:A.itemsize + A.nbytes], dB[B.itemsize:B.itemsize + B.nbytes]
+        a.copy_(to_device(A, gpu))
+        b.copy_(to_device(B, gpu))
+        plan = rt.Plan(tA, tB, perm, size, beta_is_zero=beta == 0.0)
+        plan.execute(a, b, 1.25, beta)
+        torch.cuda.synchronize()
+        got, want = from_device(b, B), oracle_run(tA, tB, A, B, 1.25, beta, perm, size)
+        assert same_bits(got, want), (plan.launch(), first_diff(got, want))
+        assert not dB[:B.itemsize].any() and not dB[B.itemsize + B.nbytes:].any()
