@@ -1570,15 +1570,20 @@ ttc_status_t ttc::plan_create(ttc_plan_t* plan, ttc_dtype_t type_a, ttc_dtype_t 
     const int* t = pl->tile;
     long long v = 1;
     for (int k = 0; k < pl->g.rank; ++k) v *= t[k];
+    const bool reuse = pl->family == kFamilyRC || v <= max_tile_volume(type_a, type_b, 1, 1);
+    st = plan_fill(fb, 1, 1, reuse ? t : nullptr, c.run_a, c.run_b, pl->family);
     // A row x column tile of the planner's own is chosen again for scalar
-    // vectors: one picked for wide ones may have more lanes than a work-group,
-    // or runs too short for them (bf16 6 x 6 x 14 x 14 x 446 x 46 at an odd
-    // address: 681 us on the wide vectors' tile, 281 on its own).
-    const bool again = pl->family == kFamilyRC && !explicit_tile && c.run_a == 0 && c.run_b == 0 && !pl->in_group;
-    if (!again || plan_fill(fb, 1, 1, nullptr, 0, 0, c.family) != TTC_SUCCESS) {
-      const bool reuse = pl->family == kFamilyRC || v <= max_tile_volume(type_a, type_b, 1, 1);
-      st = plan_fill(fb, 1, 1, reuse ? t : nullptr, c.run_a, c.run_b, pl->family);
-    }
+    // vectors where at those it has more lanes than a work-group or is a sliver
+    // (bf16 6 x 6 x 14 x 14 x 446 x 46 at an odd address: 681 us on the wide
+    // vectors' tile, 281 on its own; of 898 shapes on 1 in 18, which then take
+    // 0.69 of the time from before one tile per work-group, not 1.17 times).
+    double sliver;
+    if (st == TTC_SUCCESS && pl->family == kFamilyRC && pl->lane_div && !explicit_tile && c.run_a == 0 && c.run_b == 0 &&
+        !pl->in_group &&
+        (fb->lane_div == 0 || lane_sliver(pl->g, t, dtype_bytes(type_a), dtype_bytes(type_b), 1, 1,
+                                          !pl->beta_is_zero, sliver)) &&
+        plan_fill(fb, 1, 1, nullptr, 0, 0, c.family) != TTC_SUCCESS)
+      st = plan_fill(fb, 1, 1, t, c.run_a, c.run_b, pl->family);
     if (st != TTC_SUCCESS) {
       delete fb;
       delete pl;
