@@ -87,6 +87,8 @@ def test_slivers_are_walked():
     assert launch(BF16, BF16, [1, 4, 3, 0, 2], [2, 540, 723, 5, 28], True)[0]["kernel"] in walks
     assert launch(BF16, BF16, [1, 0], [2, 1600001])[0]["kernel"] in walks
     assert launch(BF16, BF16, [1, 0], [2, 1600001], family=2)[0]["kernel"] == rt.KERNEL_TILE_WALK
+    # slots of over 6 times the bytes, in a group of 18
+    assert launch(BF16, BF16, [3, 0, 2, 1], [32, 16128, 18, 2], True, vec_a=1, vec_b=1)[0]["kernel"] in walks
     assert launch(BF16, BF16, [1, 0], [2, 400001])[0]["kernel"] == rt.KERNEL_TILE_SMALL  # few tiles
     assert launch(BF16, BF16, [1, 0], [16, 200001])[0]["kernel"] == rt.KERNEL_TILE
 

@@ -1171,11 +1171,13 @@ static double lane_cost(const Geometry& g, const int* tile, int szA, int szB, in
 
 // Whether the tile picked for one work-group per tile is a sliver: one group
 // of up to 5 positions, and the other cut to the work-group's lanes, so that
-// its slots cost more than twice the bytes moved.  The work-groups that walk
-// several tiles take longer tiles there (`walk`).  Over 1500 shapes, the 30
-// launches that take them for it ran 1.53 times as long as slivers (geometric
-// mean; 0.82 to 4.9 times: fp16 2 x 540 x 723 x 5 x 28, 566 against 117 us).
-constexpr double kSliverTiles = 3000.0, kSliverSlots = 2.0, kSliverGain = 1.15;
+// its slots cost more than twice the bytes moved; or, whatever its groups,
+// slots of over 6 times the bytes.  The work-groups that walk several tiles
+// take longer tiles there (`walk`).  Over 1500 shapes, the 30 launches that
+// take them for it ran 1.53 times as long as slivers (geometric mean; 0.82 to
+// 4.9 times: fp16 2 x 540 x 723 x 5 x 28, 566 against 117 us).  Wider groups
+// with cheaper slots are as often faster as slower.
+constexpr double kSliverTiles = 3000.0, kSliverSlots = 2.0, kThinSlots = 6.0, kSliverGain = 1.15;
 static double moved_bytes(const Geometry& g, int szA, int szB, bool beta) {
   return (double)g.elements * (szA + szB * (beta ? 2.0 : 1.0));
 }
@@ -1183,9 +1185,9 @@ static bool lane_sliver(const Geometry& g, const int* tile, int szA, int szB, in
   LaneFit f;
   int div = 2;
   while (div > 0 && !lane_fit(g, tile, szA, szB, va, vb, div, f)) --div;
-  if (div == 0 || std::min(f.R, f.C) > 5 || (double)f.ntiles < kSliverTiles) return false;
+  if (div == 0 || (double)f.ntiles < kSliverTiles) return false;
   cost = slot_cost(szA, szB, va, vb, div, beta, (double)f.ntiles);
-  return cost >= kSliverSlots * moved_bytes(g, szA, szB, beta);
+  return cost >= (std::min(f.R, f.C) <= 5 ? kSliverSlots : kThinSlots) * moved_bytes(g, szA, szB, beta);
 }
 static bool sliver_loses(const Geometry& g, double sliver, const int* walk, int szA, int szB, int va, int vb,
                          bool beta) {
