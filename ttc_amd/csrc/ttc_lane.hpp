@@ -6,7 +6,7 @@
 // (rc_tile_of) and the cache lines they share at their edges are fetched and
 // written back once; work-groups that stride over many tiles each (the
 // pipelined kernel of ttc_rc.hpp) drift apart and lose that.  Time per
-// launch, pipelined -> one tile per work-group (copy of 200 MiB: 5.5 TB/s):
+// launch, pipelined -> one tile per work-group (copy of 200 MiB: 5.9 TB/s):
 //   fp32 6507 x 8057, padded              110 -> 94 us  (4.5 TB/s)
 //   fp32 rank 6, odd extents, 200 MiB     131 -> 102    (4.1)
 //   fp64 rank 5, beta = 1, 200 MiB        133 -> 118    (5.3)

@@ -283,8 +283,8 @@ struct RCTile {
 };
 
 // Launches of few dimensions in few bytes of arguments: with at most 112
-// (kSmallArgs and A, B, alpha, beta) the host's part of a launch takes 2.7 us,
-// with more 3.7-4.3 (an empty kernel), and the kernel reads two lines of
+// (kSmallArgs and A, B, alpha, beta) the host's part of a launch takes 3.0 us,
+// with 160 to 992 3.1-3.4 (an empty kernel), and the kernel reads two lines of
 // arguments instead of up to ten.  Tiles, and vectors of rows, are counted
 // below 2^20, so that divisions go through floats (sdiv).  A tile's chain of
 // divisions is longer than with FastDiv's constants: tiles take this form up
@@ -412,7 +412,9 @@ constexpr int row_once_unroll(int bytes_a, int bytes_b, int v, bool fp8, bool un
 // others still work, leave few of those with anything to commit (bf16 1024 x
 // 4096, 1024 tiles: 17.9 us with one tile each, 10.1 so; 6.3 without amax).
 // Three and more cost locality (bf16 8192 x 14336: one 84, two 75, four 79 us;
-// fp32: 121, 120, 138). Up to 256 units each commits its own.
+// fp32: 121, 120, 138). Up to 256 units each commits its own.  (Work-group w
+// runs on XCD w % 8: with two units each the XCDs' shares of the walk
+// interleave, which these times include.)
 constexpr uint32_t kAmaxHead = 64;
 struct AmaxUnits {
   uint32_t n, per;

@@ -49,8 +49,8 @@ def row_widths(na, nb):
 
 
 def row_unaligned_widths(na, nb):
-    """Same rule as ttc::row_unaligned_widths (csrc/ttc_plan.h): vector widths
-    of the row copy in unaligned vectors."""
+    """The widths ttc::row_unaligned_width (csrc/ttc_plan.h) may return beside 1:
+    vectors of the row copy in unaligned vectors."""
     w = []
     v = 2
     while v * max(na, nb) <= 16:
