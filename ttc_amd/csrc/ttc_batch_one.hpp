@@ -40,11 +40,9 @@ struct alignas(64) OneLane {
   RCLaneParams p;
   unsigned char pad_[1024 - sizeof(OneHead) - sizeof(RCLaneParams)];
 };
-// (RowWalk alone, so that a work table of the fixed workspace's size holds as
-// many small row copies as it can.)
 struct OneRow {
   OneHead h;
-  RowWalk p;
+  RowParams p;
 };
 // Per op, in launch order: its first tile, and its record among those of its
 // kind, with kOneIsRow for row copies.
@@ -60,7 +58,6 @@ static_assert(alignof(OneLane) <= kTableAlign && alignof(OneRow) <= kTableAlign 
 // be left behind.
 static_assert(std::is_trivially_copyable<OneLane>::value && std::is_trivially_copyable<OneRow>::value,
               "records are copied as bytes");
-static_assert(std::is_base_of<RowWalk, RowParams>::value, "a row copy's record is a slice of its parameters");
 
 // Tiles per entry of the table that gives the op a block of tiles starts in.
 constexpr uint32_t kOneBlock = 64;

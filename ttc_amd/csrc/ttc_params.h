@@ -253,23 +253,20 @@ constexpr int kRowUnroll = 4;  // vectors in flight per lane in the row-copy ker
 TTC_HD inline uint32_t row_vectors(int32_t n0, int32_t v) { return ((uint32_t)n0 + (uint32_t)v - 1u) / (uint32_t)v; }
 TTC_HD inline int32_t row_shift(int32_t e, int32_t v, int32_t n0) { return e > n0 - v ? e - (n0 - v) : 0; }
 
-// What a work-group needs of its rows: the part of RowParams that a grouped
-// launch's work table holds, assigned whole.
-struct RowWalk {
+// A row copy: kernel argument, and record of a grouped launch's work table.
+struct RowParams {
   uint32_t total;         // rows * nv (< 2^31)
   uint32_t nv;            // vectors per row: extent of dimension 0 / V (rounded up on unaligned vectors)
   int32_t n0;             // extent of dimension 0
-  int32_t rank;           // row dimensions, in B order
+  int16_t rank;           // row dimensions, in B order
+  int16_t xcd_share;      // one chunk per work-group: XCDs take contiguous shares of the chunks (grouped launches:
+                          // not read)
   uint32_t nvm, nvs;      // division by nv
   DivBy dn[kMaxDim];      // their extents
   int64_t sa[kMaxDim];    // A byte strides
   int64_t sb[kMaxDim];    // B byte strides
 };
-struct RowParams : RowWalk {
-  int32_t xcd_share;      // one chunk per work-group: XCDs take contiguous shares of the chunks
-  int32_t pad_;
-};
-inline void row_set_vectors(RowWalk& p, uint32_t rows, uint32_t nv) {
+inline void row_set_vectors(RowParams& p, uint32_t rows, uint32_t nv) {
   const FastDiv f = make_fastdiv(nv);
   p.total = rows * nv, p.nv = nv, p.nvm = f.m, p.nvs = f.s;
 }

@@ -11,6 +11,15 @@
 
 namespace ttc {
 
+// touch_lines over a row kernel's arguments: RowParams, and behind it pointers,
+// scalars and scales.  One statement waits for all lines, so that none is left
+// for a second wait.
+__device__ __forceinline__ void touch_row_args() {
+  static_assert(sizeof(RowParams) > 192 && sizeof(RowParams) <= 256, "lines of the arguments");
+  KWord* const w = (KWord*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]), "s"(w[64]));
+}
+
 template <class OP, int V, int MODE>
 __global__ void __launch_bounds__(kThreads)
     row_kernel(const RowParams p, const typename OP::TA* __restrict__ A, typename OP::TB* __restrict__ B,
@@ -24,7 +33,7 @@ __global__ void __launch_bounds__(kThreads)
   constexpr bool NT = MODE == kModeBzNt;
   constexpr int U = kRowUnroll;  // vectors in flight per lane
   // (casts to fp8 of 8 to 32 MB 9-11% faster so, of 64 to 128 3-6%)
-  touch_lines<sizeof(RowParams)>(__builtin_amdgcn_kernarg_segment_ptr());
+  touch_row_args();
   float scale = 1.0f;
   if constexpr (FP8) {
     scale = scale_host;
@@ -127,8 +136,8 @@ template <class T, int V> struct __attribute__((packed, aligned(sizeof(T)))) Row
 // copy 4740 -> 6010; bf16 128 x 4096 x 32 x 8 perm (0,2,1,3) 4760 -> 5340;
 // fp32 rows of 127 3890 -> 4730, of 5 2210 -> 3040; bf16 rows of 127
 // 2180 -> 4070, of 5 1270 -> 2240.
-// P: RowParams as a kernel argument, RowWalk in a grouped launch's work table,
-// or RowSmall.
+// P: RowParams as a kernel argument or in a grouped launch's work table, or
+// RowSmall.
 // Returns max |alpha * a| of this lane's elements (fp8 casts).
 template <class OP, int V, int MODE, bool UNAL, class P>
 __device__ __forceinline__ float row_chunk(const P& p, uint32_t w, const typename OP::TA* __restrict__ A,
@@ -247,7 +256,7 @@ __global__ void __launch_bounds__(kThreads)
                     float fp8_max, float scale_host, float* __restrict__ amax_out,
                     float* __restrict__ scale_inv_out, AmaxUnits units) {
   constexpr bool FP8 = MODE == kModeFp8;
-  touch_lines<sizeof(RowParams)>(__builtin_amdgcn_kernarg_segment_ptr());
+  touch_row_args();
   float scale = 1.0f;
   if constexpr (FP8) {
     scale = scale_host;
